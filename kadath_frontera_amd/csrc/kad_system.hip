@@ -9,7 +9,8 @@
 //   xx_to_vars + old - var         -> CSR update kernel on the coefficient arrays
 #include "kad_common.hpp"
 #include "kad_ctx.hpp"
-#include "kad_spectral.hpp"
+#include "kad_apply3d.hpp"
+#include "kad_group.hpp"
 #include "host/xcts.hpp"
 #include "host/parsed_system.hpp"
 #include "../../include/kadath_amd.h"
@@ -33,11 +34,7 @@ using namespace kadhost;
 
 namespace {
 
-struct DevRow {
-  int pos, gpos;
-  double gw;
-};
-
+using kad::DevRow;
 using kad::ew_op;
 static_assert(EW_ADD == kad::EWOP_ADD && EW_SUB == kad::EWOP_SUB && EW_MUL == kad::EWOP_MUL &&
                   EW_DIV == kad::EWOP_DIV && EW_SCAL == kad::EWOP_SCAL && EW_ADDS == kad::EWOP_ADDS &&
@@ -415,6 +412,22 @@ struct DevProgram {
   int field = 0, dom = 0, off = 0, cnt = 0;
 };
 
+// A program's instructions by dependency level (kad_group.hip): ops [op0 + lev[l],
+// op0 + lev[l + 1]) of the device table run together.
+struct GroupProg {
+  bool ok = false;             // false: the program runs instruction by instruction
+  int op0 = 0, nphys = 0;      // nphys: tangent slots of one column
+  std::vector<int> lev;
+  std::vector<size_t> lds;     // per level: the most LDS of an instruction
+  std::vector<double> bytes;   // per level: algorithmic HBM bytes of one column (passes and element-wise)
+};
+// Columns [u0, u0 + nb) of a program, results in column col0 + (0 .. nb).
+struct GroupItem {
+  const GroupProg* p;
+  int u0, nb;
+  int64_t col0;
+};
+
 double now_s() {
   return std::chrono::duration<double>(std::chrono::steady_clock::now().time_since_epoch()).count();
 }
@@ -534,6 +547,25 @@ struct kad_system_impl {
   bool vsplit_ok = false;
   std::vector<std::vector<Instr>> vparts;
   std::vector<Instr> vexports;
+  // grouped execution: the instruction table, the value program, the tangent programs
+  // (one per layout entry) and the parameters' programs by dependency level
+  kad::GroupOp* gops = nullptr;
+  GroupProg gval;
+  std::vector<GroupProg> gtan, gpar;
+  bool gtan_ok = false;         // every tangent program can be grouped
+  double* grp_arena = nullptr;  // tangent slots of the columns of one round
+  size_t grp_cap = 0;           // doubles
+  int group_build(std::vector<Instr> code, int nvirt, bool value, int seed_tab, GroupProg& gp,
+                  std::vector<kad::GroupOp>& ops);
+  int group_round(const std::vector<GroupItem>& items, void* out, int64_t ldo, int dtype, const double* w);
+  int group_columns(std::vector<GroupItem> items, void* out, int64_t ldo, int dtype, const double* w);
+  // columns [c0, c1) of J (or, with w, entries of J^T w) into out, whose column 0 is
+  // column col_base of J: the double unknowns' programs, then the tangent programs'
+  int columns(int c0, int c1, int64_t col_base, void* out, int64_t ldo, int dtype = 0, const double* w = nullptr);
+  int ensure_tan_arena() {
+    if (tan_arena) return KAD_OK;
+    return dmalloc((void**)&tan_arena, (size_t)std::max(1, nphys_max) * B * stride * sizeof(double));
+  }
   bool vals_current = false;  // the value arena holds the value pass of the current fields
   int ensure_values() { return vals_current ? KAD_OK : value_pass(); }
   int value_pass();
@@ -815,7 +847,23 @@ int kad_system_impl::setup() {
     nphys_max = std::max(nphys_max, dp.nphys);
     glob_par_progs.push_back(std::move(dp));
   }
-  if ((rc = dmalloc((void**)&tan_arena, (size_t)std::max(1, nphys_max) * B * stride * sizeof(double)))) return rc;
+  // the same programs by dependency level
+  std::vector<kad::GroupOp> ops;
+  if ((rc = group_build(tr.val.code, 0, true, -1, gval, ops))) return rc;
+  gtan.resize(sys->tprog.size());
+  gtan_ok = !gtan.empty();
+  for (size_t p = 0; p < sys->tprog.size(); ++p) {
+    if ((rc = group_build(sys->tprog[p].code, sys->tprog[p].nslots, false, tprogs[p].seed_tab, gtan[p], ops))) return rc;
+    gtan_ok = gtan_ok && gtan[p].ok;
+  }
+  gpar.resize(sys->par_prog.size());
+  for (int k = 0; k < sys->ndouble; ++k) {
+    const int p = sys->dvar_par[k];
+    if ((rc = group_build(sys->par_prog[p].code, sys->par_prog[p].nslots, false, sys->par_tab[p], gpar[p], ops)))
+      return rc;
+    gtan_ok = gtan_ok && gpar[p].ok;
+  }
+  if ((rc = upload(ops, &gops))) return rc;
   if ((rc = dmalloc((void**)&F, (size_t)sys->n_rows * sizeof(double)))) return rc;
   if ((rc = dmalloc((void**)&scratch, 64 * sizeof(double)))) return rc;
   return KAD_OK;
@@ -824,7 +872,11 @@ int kad_system_impl::setup() {
 int kad_system_impl::run(const std::vector<Instr>& code, int nb, int u0, int seed_tab, void* out, int64_t col0,
                          int64_t ldo, int dtype, const double* w, hipStream_t st, double* tan) {
   hipStream_t s = st ? st : ctx->stream;
-  if (!tan) tan = tan_arena;
+  if (!tan) {
+    const int rc = ensure_tan_arena();
+    if (rc) return rc;
+    tan = tan_arena;
+  }
   auto slot_ptr = [&](const Opnd& o) { return this->slot_ptr(o, tan); };
   for (size_t t = 0; t < code.size(); ++t) {
     const Instr& in = code[t];
@@ -989,8 +1041,318 @@ bool kad_system_impl::split_values(int ns) {
   return vsplit_ok;
 }
 
+// The instructions of a program by dependency level: an instruction's level is one past
+// the last of its operands' (ASAP), so the instructions of a level are independent.
+// Tangent programs absorb element-wise chains first (mark_fusions) and their slots are
+// reused between levels: a slot is free again after the last level that reads it.
+// Exports add to rows that earlier exports may have written: in the value program an
+// export follows every earlier one that shares a row, in a tangent program every
+// earlier one (the transposed export adds all of them to one entry).  A program with
+// other instructions, or a slot written twice, stays on the per-instruction path (ok
+// false).
+int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value, int seed_tab, GroupProg& gp,
+                                 std::vector<kad::GroupOp>& ops) {
+  gp = GroupProg();
+  if (!value) mark_fusions(code, nvirt, plans);
+  const int space = value ? SP_VAL : SP_TAN;
+  const int nslots = std::max(1, value ? sys->tr.nval_slots : nvirt);
+  std::vector<int> wlev(nslots, -1), rlev(nslots, -1);  // level that writes / last reads a slot
+  struct Unit {
+    size_t t;
+    int m, level;
+    double cost;
+  };
+  std::vector<Unit> units;
+  struct Rows {
+    int lo, hi, level;
+  };
+  std::vector<Rows> written;
+  int depth = 0;
+  for (size_t t = 0; t < code.size(); ++t) {
+    const Instr& in = code[t];
+    const int m = (!value && (in.kind == I_LIN || in.kind == I_EW)) ? in.fuse : 0;
+    const bool exp = in.kind == I_EXPORT_IN || in.kind == I_EXPORT_BD || in.kind == I_EXPORT_GL;
+    if (!exp && in.kind != I_LIN && in.kind != I_EW && !(in.kind == I_SEED && !value)) return KAD_OK;
+    int level = 0;
+    std::vector<int> reads;
+    for (int k = 0; k <= m; ++k) {
+      const Instr& e = code[t + k];
+      for (const Opnd* o : {&e.a, &e.b}) {
+        if (o->slot < 0 || (in.kind == I_SEED)) continue;
+        if (o->space != space) {
+          if (value || exp) return KAD_OK;
+          continue;  // the values are there before any tangent
+        }
+        if (k > 0 && o->slot == code[t + k - 1].dst.slot) continue;  // the chain's own value
+        if (o->slot >= nslots) return KAD_OK;
+        level = std::max(level, wlev[o->slot] + 1);
+        reads.push_back(o->slot);
+      }
+    }
+    if (exp) {
+      const int n = in.kind == I_EXPORT_GL ? 1 : in.nrows;
+      for (const Rows& r : written)
+        if (!value || (in.row0 < r.hi && r.lo < in.row0 + n)) level = std::max(level, r.level + 1);
+      written.push_back({in.row0, in.row0 + n, level});
+    } else {
+      const Opnd& d = code[t + m].dst;
+      if (d.space != space || d.slot < 0 || d.slot >= nslots || wlev[d.slot] >= 0) return KAD_OK;
+      wlev[d.slot] = level;
+    }
+    for (int s : reads) rlev[s] = std::max(rlev[s], level);
+    units.push_back({t, m, level, 0.0});
+    depth = std::max(depth, level + 1);
+    t += m;
+  }
+  // slots: reused once no level reads them any more
+  std::vector<int> phys(nslots, -1), freelist;
+  std::vector<std::vector<int>> by_level(depth);
+  for (size_t u = 0; u < units.size(); ++u) by_level[units[u].level].push_back((int)u);
+  if (!value) {
+    std::vector<std::vector<int>> dies(depth);
+    for (int s = 0; s < nslots; ++s)
+      if (wlev[s] >= 0) dies[std::max(wlev[s], rlev[s])].push_back(s);
+    for (int l = 0; l < depth; ++l) {
+      for (int u : by_level[l]) {
+        const Instr& e = code[units[u].t + units[u].m];
+        if (e.dst.slot < 0 || e.dst.space != SP_TAN || e.kind == I_EXPORT_IN || e.kind == I_EXPORT_BD ||
+            e.kind == I_EXPORT_GL)
+          continue;
+        if (freelist.empty()) {
+          phys[e.dst.slot] = gp.nphys++;
+        } else {
+          phys[e.dst.slot] = freelist.back();
+          freelist.pop_back();
+        }
+      }
+      for (int s : dies[l]) freelist.push_back(phys[s]);
+    }
+  }
+  auto opnd = [&](const Opnd& o) {
+    kad::GroupOpnd g;
+    g.slot = o.slot;
+    g.tan = (o.slot >= 0 && o.space == SP_TAN) ? 1 : 0;
+    if (g.tan) g.slot = phys[o.slot];
+    return g;
+  };
+  gp.op0 = (int)ops.size();
+  gp.lev.assign(1, 0);
+  for (int l = 0; l < depth; ++l) {
+    size_t lds = 0;
+    double bytes = 0.0;
+    std::vector<std::pair<double, kad::GroupOp>> lv;  // cost, instruction: the longest start first
+    for (int u : by_level[l]) {
+      const size_t t = units[u].t;
+      const int m = units[u].m;
+      const Instr& in = code[t];
+      const Domain& dm = sys->doms[in.dom];
+      kad::GroupOp op;
+      double cost = 0.0;
+      op.a = opnd(in.a);
+      op.nstep = m;
+      for (int k = 0; k < m; ++k) {
+        const Instr& e = code[t + k + 1];
+        const int side = (e.a.space == SP_TAN && e.a.slot == code[t + k].dst.slot) ? 0 : 1;
+        op.st[k].kind = e.ew;
+        op.st[k].side = side;
+        op.st[k].o = opnd(side == 0 ? e.b : e.a);
+        op.st[k].s = e.s;
+      }
+      if (in.kind == I_LIN || in.kind == I_EW || in.kind == I_SEED) op.dst = opnd(code[t + m].dst);
+      int nout = in.size;
+      switch (in.kind) {
+        case I_LIN: {
+          op.kind = kad::GK_LIN;
+          op.d0 = in.din[0];
+          op.d1 = in.din[1];
+          op.d2 = in.din[2];
+          op.P = plans[in.plan].P;
+          op.pool = plans[in.plan].pool;
+          const kad::Apply3dShape sh = kad::apply3d_shape(op.d0, op.d1, op.d2, op.P);
+          op.stage_pool = sh.stage_pool;
+          op.inplace = sh.inplace;
+          if (sh.lds > 160 * 1024) return KAD_ERR_ARG;
+          lds = std::max(lds, sh.lds);
+          int od[3] = {op.d0, op.d1, op.d2};
+          for (int p = 0; p < op.P.npass; ++p) od[op.P.axis[p]] = op.P.nout[p];
+          nout = od[0] * od[1] * od[2];
+          bytes += 8.0 * ((double)op.d0 * op.d1 * op.d2 + nout);
+          cost = 1e6 * op.P.npass + nout;
+          break;
+        }
+        case I_EW:
+          op.kind = kad::GK_EW;
+          op.ew = in.ew;
+          op.size = in.size;
+          op.s = in.s;
+          op.b = opnd(in.b);
+          bytes += 8.0 * in.size * (2.0 + (in.b.slot >= 0 ? 1.0 : 0.0));
+          cost = in.size;
+          break;
+        case I_SEED: {
+          op.kind = kad::GK_SEED;
+          op.size = in.size;
+          op.spos = seed_pos[seed_tab];
+          op.sval = seed_val[seed_tab];
+          op.scnt = seed_cnt[seed_tab];
+          op.nu = (int)sys->seeds[seed_tab].cnt.size();
+          cost = in.size;
+          break;
+        }
+        case I_EXPORT_GL:
+          op.kind = kad::GK_EXPORT_GL;
+          op.row0 = in.row0;
+          op.nr = dm.nr;
+          op.nt = dm.nt;
+          op.aux = in.aux;
+          op.bsign = in.bsign;
+          op.s = in.s;
+          op.c0 = in.c0;
+          op.accumulate = in.accumulate;
+          op.pt = in.pt;
+          cost = 1e7;
+          break;
+        default:
+          op.kind = in.kind == I_EXPORT_BD ? kad::GK_EXPORT_BD : kad::GK_EXPORT_IN;
+          op.rows = row_tabs[in.rows];
+          op.nrows = in.nrows;
+          op.row0 = in.row0;
+          op.accumulate = in.accumulate;
+          op.bsign = in.bsign;
+          op.sign = in.sign;
+          op.nr = dm.nr;
+          lds = std::max(lds, (size_t)256 * sizeof(double));  // the transposed export's reduction
+          cost = in.nrows;
+          break;
+      }
+      for (int k = 0; k < m; ++k) bytes += op.st[k].o.tan ? 8.0 * nout : 0.0;
+      lv.push_back({cost, op});
+    }
+    std::stable_sort(lv.begin(), lv.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
+    for (auto& x : lv) ops.push_back(x.second);
+    gp.lev.push_back((int)ops.size() - gp.op0);
+    gp.lds.push_back(lds);
+    gp.bytes.push_back(bytes);
+  }
+  gp.ok = true;
+  return KAD_OK;
+}
+
+// One round: every level of the items' programs, all items of a level in one launch (at
+// most kGroupEntries items).
+int kad_system_impl::group_round(const std::vector<GroupItem>& items, void* out, int64_t ldo, int dtype,
+                                 const double* w) {
+  kad::GroupArgs g;
+  g.ops = gops;
+  g.val = val_arena;
+  g.tan = grp_arena;
+  g.stride = stride;
+  g.out = out;
+  g.ldo = ldo;
+  g.dtype = dtype;
+  g.w = w;
+  size_t depth = 0;
+  for (const GroupItem& it : items) depth = std::max(depth, it.p->lds.size());
+  for (size_t l = 0; l < depth; ++l) {
+    int blocks = 0, n = 0;
+    size_t lds = 0;
+    int64_t base = 0;
+    double bytes = 0.0;
+    for (const GroupItem& it : items) {
+      const GroupProg& p = *it.p;
+      const int64_t b0 = base;
+      base += (int64_t)p.nphys * it.nb * stride;
+      if (l >= p.lds.size()) continue;
+      const int nops = p.lev[l + 1] - p.lev[l];
+      // a column's workgroups keep their residue modulo 8, so the round-robin dispatch
+      // puts it on the same XCD (and its L2) at every level
+      const int nbp = it.nb == 1 ? 1 : (int)kad::cdiv(it.nb, 8) * 8;
+      if (nbp > 1) blocks = (int)kad::cdiv(blocks, 8) * 8;
+      g.e[n++] = {blocks, nops, p.op0 + p.lev[l], it.nb, nbp, it.u0, b0, it.col0};
+      blocks += nops * nbp;
+      lds = std::max(lds, p.lds[l]);
+      bytes += p.bytes[l] * it.nb;
+    }
+    g.nent = n;
+    kad::GemmTimer* tm = kad::g_apply_timer;
+    const int trc = tm && bytes > 0.0 ? tm->begin(ctx->stream, bytes) : 1;
+    if (trc < 0) return trc;
+    const int rc = kad::group_launch(g, blocks, lds, ctx->stream);
+    if (rc) return rc;
+    if (trc == 0 && tm->end(ctx->stream)) return KAD_ERR_HIP;
+  }
+  return KAD_OK;
+}
+
+// The items in rounds that fit the arena.
+int kad_system_impl::group_columns(std::vector<GroupItem> items, void* out, int64_t ldo, int dtype, const double* w) {
+  if (items.empty()) return KAD_OK;
+  if (!grp_arena) {
+    size_t all = 0, one = 0;
+    for (size_t p = 0; p < gtan.size(); ++p) {
+      all += (size_t)gtan[p].nphys * tprogs[p].cnt * stride;
+      one = std::max(one, (size_t)gtan[p].nphys * stride);
+    }
+    for (auto& p : gpar) {
+      all += (size_t)p.nphys * stride;
+      one = std::max(one, (size_t)p.nphys * stride);
+    }
+    // 3 GiB: every column of a 9x7x4 system at once (0.9 GB; 2.64 ms per Jacobian, 4.24
+    // when only 32 MiB of columns run together), several thousand columns of the larger
+    // ones (J^T w at 13x9x8: 42, 37, 34.4, 33.5 ms with 0.5, 1, 3, 12 GiB)
+    const size_t budget = (size_t)3 << 27;  // doubles
+    const size_t cap = std::max(std::min(all, budget), 64 * one);
+    const int rc = dmalloc((void**)&grp_arena, cap * sizeof(double));
+    if (rc) return rc;
+    grp_cap = cap;
+  }
+  std::vector<GroupItem> round;
+  size_t used = 0;
+  auto flush = [&]() -> int {
+    if (round.empty()) return KAD_OK;
+    const int rc = group_round(round, out, ldo, dtype, w);
+    round.clear();
+    used = 0;
+    return rc;
+  };
+  for (GroupItem it : items) {
+    const size_t per = std::max<size_t>(1, (size_t)it.p->nphys * stride);
+    while (it.nb > 0) {
+      const int64_t room = (int64_t)((grp_cap - used) / per);
+      if ((int)round.size() >= kad::kGroupEntries || room < std::min(it.nb, 64)) {
+        const int rc = flush();
+        if (rc) return rc;
+        continue;
+      }
+      GroupItem q = it;
+      q.nb = (int)std::min<int64_t>(it.nb, room);
+      round.push_back(q);
+      used += per * q.nb;
+      it.u0 += q.nb;
+      it.col0 += q.nb;
+      it.nb -= q.nb;
+    }
+  }
+  return flush();
+}
+
+int kad_system_impl::columns(int c0, int c1, int64_t col_base, void* out, int64_t ldo, int dtype, const double* w) {
+  std::vector<GroupItem> items;
+  for (int k = c0; k < c1 && k < sys->ndouble; ++k) items.push_back({&gpar[sys->dvar_par[k]], 0, 1, k - col_base});
+  for (size_t p = 0; p < tprogs.size(); ++p) {
+    const int lo = std::max(c0, tprogs[p].off), hi = std::min(c1, tprogs[p].off + tprogs[p].cnt);
+    if (lo < hi) items.push_back({&gtan[p], lo - tprogs[p].off, hi - lo, lo - col_base});
+  }
+  return group_columns(std::move(items), out, ldo, dtype, w);
+}
+
 int kad_system_impl::value_pass() {
   int rc;
+  if (gval.ok && fuse_ew) {
+    rc = group_round({{&gval, 0, 1, 0}}, F, 0, 0, nullptr);
+    vals_current = (rc == KAD_OK);
+    return rc;
+  }
   const int ns = std::max(1, std::min(nfill, kFillMax));
   if (ns > 1 && split_values(ns)) {
     hipStream_t s0 = ctx->stream;
@@ -998,7 +1360,7 @@ int kad_system_impl::value_pass() {
     KAD_HIP_CHECK(hipEventRecord(fev[0], s0));
     for (int i = 1; i < ns; ++i) KAD_HIP_CHECK(hipStreamWaitEvent(fstream[i], fev[0], 0));
     for (int i = 0; i < ns && rc == KAD_OK; ++i)
-      rc = run(vparts[i], 1, 0, -1, F, 0, 0, 0, nullptr, i ? fstream[i] : s0, tan_arena);
+      rc = run(vparts[i], 1, 0, -1, F, 0, 0, 0, nullptr, i ? fstream[i] : s0, val_arena);
     for (int i = 1; i < ns; ++i) {
       KAD_HIP_CHECK(hipEventRecord(fev[i], fstream[i]));
       KAD_HIP_CHECK(hipStreamWaitEvent(s0, fev[i], 0));
@@ -1015,11 +1377,21 @@ int kad_system_impl::jacobian(double* Jd, int64_t ldj) {
   int rc = value_pass();
   if (rc) return rc;
   KAD_HIP_CHECK(hipMemsetAsync(Jd, 0, (size_t)ldj * sys->n_unknowns * sizeof(double), ctx->stream));
-  if ((rc = double_columns(Jd, ldj, 0, sys->ndouble, 0))) return rc;
   return fill_columns(Jd, ldj);
 }
 
 int kad_system_impl::fill_columns(double* Jd, int64_t ldj) {
+  // Programs of 2048 columns and more fill the chip with each instruction (8 workgroups
+  // per CU); their launches on nfill streams overlap and keep an instruction's arrays
+  // closer together than a whole level's (17x13x12, 2397 columns per program: 0.139 s
+  // against 0.167 grouped; 13x9x8, 819 columns: 34 ms grouped against 62)
+  const bool wide = (int64_t)sys->n_unknowns >= (int64_t)2048 * (int64_t)tprogs.size();
+  if (gtan_ok && fuse_ew && !wide) return columns(0, sys->n_unknowns, 0, Jd, ldj);
+  {
+    int rc = double_columns(Jd, ldj, 0, sys->ndouble, 0);
+    if (!rc) rc = ensure_tan_arena();
+    if (rc) return rc;
+  }
   hipStream_t s0 = ctx->stream;
   const int ns = std::max(1, std::min(nfill, (int)tprogs.size()));
   {
@@ -1582,7 +1954,6 @@ static int newton_direction(kad_system_impl* S, int solver, double err, double* 
   if (!S->vals_current)
     if ((rc = S->value_pass())) return rc;
   KAD_HIP_CHECK(hipMemsetAsync(S->J, 0, (size_t)n * n * sizeof(double), st));
-  if ((rc = S->double_columns(S->J, n, 0, sy.ndouble, 0))) return rc;
   if ((rc = S->fill_columns(S->J, n))) return rc;
   KAD_HIP_CHECK(hipStreamSynchronize(st));
   double t2 = now_s();
@@ -2512,6 +2883,11 @@ int kad_jvp_fill(kad_system* s, int col_begin, int col_count, void* J_tile, int6
   const size_t es = dtype == 0 ? sizeof(double) : sizeof(float);
   KAD_HIP_CHECK(hipMemset2DAsync(J_tile, (size_t)ld * es, 0, (size_t)m * es, (size_t)col_count, st));
   const int c1 = col_begin + col_count;
+  if (S->gtan_ok && S->fuse_ew) {
+    if ((rc = S->columns(col_begin, c1, col_begin, J_tile, ld, dtype))) return rc;
+    KAD_HIP_CHECK(hipStreamSynchronize(st));
+    return KAD_OK;
+  }
   if ((rc = S->double_columns(J_tile, ld, col_begin, c1, col_begin, dtype))) return rc;
   for (auto& p : S->tprogs) {
     const int lo = std::max(col_begin, p.off), hi = std::min(c1, p.off + p.cnt);
@@ -2534,6 +2910,11 @@ int kad_vjp(kad_system* s, const double* w, double* out) {
   int rc = S->ensure_values();
   if (rc) return rc;
   KAD_HIP_CHECK(hipMemsetAsync(out, 0, (size_t)S->sys->n_unknowns * sizeof(double), st));
+  if (S->gtan_ok && S->fuse_ew) {
+    if ((rc = S->columns(0, S->sys->n_unknowns, 0, out, 0, 0, w))) return rc;
+    KAD_HIP_CHECK(hipStreamSynchronize(st));
+    return KAD_OK;
+  }
   for (int k = 0; k < S->sys->ndouble; ++k) {
     const DevProgram& pp = S->par_progs[S->sys->dvar_par[k]];
     if ((rc = S->run(pp.code, 1, 0, pp.seed_tab, out, k, 0, 0, w))) return rc;
