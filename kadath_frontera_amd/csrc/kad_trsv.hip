@@ -31,9 +31,21 @@ __device__ __forceinline__ double tri_at(const T* F, int64_t lda, int r, int c) 
   return TR ? (double)F[c + (int64_t)r * lda] : (double)F[r + (int64_t)c * lda];
 }
 
-// Inverse of diagonal block blockIdx.x of the factor's unit-lower (uplo 0) or
-// upper (uplo 1) triangle, by columns as LAPACK dtrti2; written transposed when
-// tr_out (the inverse of the transposed block).  Out: first TBS columns of W_k.
+// Inverse of diagonal block blockIdx.x of the factor's unit-lower (uplo 0) or upper
+// (uplo 1) triangle, written transposed when tr_out (the inverse of the transposed
+// block).  Out: first TBS columns of W_k.
+//
+// Bound by latency: one workgroup per block, and a column-by-column inversion is 128
+// dependent steps of up to 128 serial multiply-adds (400 us).  Here every row of the
+// inverse solves X T = I on its own, 32 columns at a time from the last: the product
+// with the columns already known (two threads per row, 16 columns each), then the
+// substitution with the 32 x 32 diagonal block, one row per thread in registers: 64 us.
+// Each row's residual X T - I is at rounding level, as the column-by-column inversion's
+// was (joining inverted quarters by products would square the conditioning of
+// ill-conditioned blocks into it).  The block is held as a lower triangle (an upper one
+// with both index orders reversed).
+constexpr int DIB = 32;  // columns per step
+
 template <typename T>
 __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__ F, int64_t lda, int n, int uplo,
                                                            int tr_out, double* __restrict__ W, int64_t sF = 0,
@@ -41,91 +53,142 @@ __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__
   F += (int64_t)blockIdx.y * sF;  // factors blockIdx.y of a batch
   W += (int64_t)blockIdx.y * sW;
   __shared__ double M[TBS][TBS + 1];
-  __shared__ double col[TBS];
+  __shared__ double pbuf[TBS][DIB / 2 + 1];
   const int blk = blockIdx.x;
   const int r0 = blk * TBS;
   const int nb = min(TBS, n - r0);
   const int t = threadIdx.x;
-  for (int e = t; e < TBS * TBS; e += 256) {
-    const int i = e % TBS, c = e / TBS;
-    double v = 0.0;
-    if (i < nb && c < nb) {
-      const bool in_tri = uplo == 0 ? (i > c) : (i <= c);
-      if (in_tri) v = (double)F[(r0 + i) + (int64_t)(r0 + c) * lda];
-      if (uplo == 0 && i == c) v = 1.0;
+  // M(i, c), i >= c: the triangle (reversed for uplo 1), the identity past nb
+  for (int e0 = 0; e0 < TBS * TBS; e0 += 256 * 8) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = e0 + u * 256 + t;
+      const int i = e % TBS, c = e / TBS;
+      const bool tri = i < nb && c < nb && (uplo == 0 ? i > c : i <= c);
+      v[u] = tri ? (double)F[(r0 + i) + (int64_t)(r0 + c) * lda] : 0.0;
+      if (i == c && (uplo == 0 || i >= nb)) v[u] = 1.0;
     }
-    M[i][c] = v;
+#pragma unroll
+    for (int u = 0; u < 8; ++u) {
+      const int e = e0 + u * 256 + t;
+      const int i = e % TBS, c = e / TBS;
+      if (uplo == 0) M[i][c] = v[u];
+      else M[TBS - 1 - i][TBS - 1 - c] = v[u];
+    }
   }
   __syncthreads();
-  if (uplo == 1) {
-    // column j: M[j][j] <- 1/M[j][j]; M[0:j, j] <- -M[j][j] * (inv(M[0:j, 0:j]) M[0:j, j])
-    for (int j = 0; j < nb; ++j) {
-      if (t < j) col[t] = M[t][j];
-      __syncthreads();
-      const double ajj = 1.0 / M[j][j];
-      if (t < j) {
-        double s = 0.0;
-        for (int k = t; k < j; ++k) s += M[t][k] * col[k];
-        M[t][j] = -ajj * s;
-      }
-      __syncthreads();
-      if (t == 0) M[j][j] = ajj;
-      __syncthreads();
+  const int r = t & (TBS - 1), half = t >> 7, rb = r / DIB;
+#pragma unroll 1
+  for (int J = TBS / DIB - 1; J >= 0; --J) {
+    const int j0 = J * DIB, jh = j0 + half * (DIB / 2);
+    // p(j) = I(r, j) - sum over the later column blocks of X(r, k) T(k, j)
+    double p[DIB / 2];
+#pragma unroll
+    for (int j = 0; j < DIB / 2; ++j) p[j] = jh + j == r ? 1.0 : 0.0;
+    for (int k = j0 + DIB; k < (rb + 1) * DIB; ++k) {
+      const double xk = M[r][k];
+#pragma unroll
+      for (int j = 0; j < DIB / 2; ++j) p[j] -= xk * M[k][jh + j];
     }
-  } else {
-    // column j (descending): M[j+1:, j] <- -(inv(M[j+1:, j+1:]) M[j+1:, j])
-    for (int j = nb - 2; j >= 0; --j) {
-      if (t > j && t < nb) col[t] = M[t][j];
-      __syncthreads();
-      if (t > j && t < nb) {
-        double s = 0.0;
-        for (int k = j + 1; k <= t; ++k) s += M[t][k] * col[k];
-        M[t][j] = -s;
+    if (half)
+#pragma unroll
+      for (int j = 0; j < DIB / 2; ++j) pbuf[r][j] = p[j];
+    __syncthreads();
+    const bool mine = !half && rb >= J;
+    double x[DIB];
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < DIB / 2; ++j) {
+        x[j] = p[j];
+        x[DIB / 2 + j] = pbuf[r][j];
       }
-      __syncthreads();
+#pragma unroll
+      for (int j = DIB - 1; j >= 0; --j) {
+#pragma unroll
+        for (int k = j + 1; k < DIB; ++k) x[j] -= x[k] * M[j0 + k][j0 + j];
+        if (uplo == 1) x[j] /= M[j0 + j][j0 + j];
+      }
     }
+    __syncthreads();  // the column block of T has been read by every row
+    if (mine) {
+#pragma unroll
+      for (int j = 0; j < DIB; ++j)
+        if (j0 + j <= r) M[r][j0 + j] = x[j];
+    }
+    __syncthreads();
   }
   double* out = W + (int64_t)blk * TBS * WCOLS;
   for (int e = t; e < TBS * TBS; e += 256) {
-    const int i = e % TBS, c = e / TBS;
-    out[e] = tr_out ? M[c][i] : M[i][c];
+    const int i = tr_out ? e / TBS : e % TBS, c = tr_out ? e % TBS : e / TBS;
+    const bool tri = i < nb && c < nb && (uplo == 0 ? i >= c : i <= c);
+    out[e] = !tri ? 0.0 : uplo == 0 ? M[i][c] : M[TBS - 1 - i][TBS - 1 - c];
   }
 }
 
 // Coupling half of W_k: -inv(T_kk) T_kp, with T accessed through tri_at and
-// p = k - 1 (forward) or k + 1 (backward).  One workgroup per k with a p.
+// p = k - 1 (forward) or k + 1 (backward).  Workgroup (k, y) makes 32 of the 128
+// columns with the fp64 matrix cores: a wave owns 32 rows (2 x 2 tiles of 16), the
+// inverse is read straight into the A operand (16 consecutive rows per column), T_kp
+// goes through LDS.  160 us -> 12 us (a whole 128^3 product by one workgroup's VALU
+// before, its loads of the inverse each waited for).
+constexpr int CPC = 32;  // columns per workgroup
 template <typename T, bool TR, bool FWD>
 __global__ __launch_bounds__(256) void couple_kernel(const T* __restrict__ F, int64_t lda, int n, int nblk,
                                                      double* __restrict__ W, int64_t sF = 0, int64_t sW = 0) {
-  F += (int64_t)blockIdx.y * sF;  // factors blockIdx.y of a batch
-  W += (int64_t)blockIdx.y * sW;
-  __shared__ double B[TBS][TBS + 1];
+  F += (int64_t)blockIdx.z * sF;  // factors blockIdx.z of a batch
+  W += (int64_t)blockIdx.z * sW;
+  __shared__ double B[CPC][TBS + 2];  // B[j][k] = T_kp(k, column j)
   const int k = FWD ? blockIdx.x + 1 : blockIdx.x;
   const int p = FWD ? k - 1 : k + 1;
   if (k >= nblk || p < 0 || p >= nblk) return;
-  const int r0 = k * TBS, c0 = p * TBS;
-  const int nr = min(TBS, n - r0), nc = min(TBS, n - c0);
+  const int r0 = k * TBS, c0 = p * TBS + blockIdx.y * CPC;
+  const int nr = min(TBS, n - r0), nc = min(CPC, n - c0);
   const int t = threadIdx.x;
-  for (int e = t; e < TBS * TBS; e += 256) {
-    const int i = e % TBS, c = e / TBS;
-    B[i][c] = (i < nr && c < nc) ? tri_at<T, TR>(F, lda, r0 + i, c0 + c) : 0.0;
+  {
+    double v[TBS * CPC / 256];
+#pragma unroll
+    for (int u = 0; u < TBS * CPC / 256; ++u) {
+      const int e = u * 256 + t;
+      const int i = TR ? e / CPC : e % TBS, c = TR ? e % CPC : e / TBS;  // coalesced in the stored order
+      v[u] = (i < nr && c < nc) ? tri_at<T, TR>(F, lda, r0 + i, c0 + c) : 0.0;
+    }
+#pragma unroll
+    for (int u = 0; u < TBS * CPC / 256; ++u) {
+      const int e = u * 256 + t;
+      const int i = TR ? e / CPC : e % TBS, c = TR ? e % CPC : e / TBS;
+      B[c][i] = v[u];
+    }
   }
   __syncthreads();
   double* Wk = W + (int64_t)k * TBS * WCOLS;
-  const int j = t % TBS;            // output column
-  const int i0 = (t / TBS) * 64;    // 64 output rows per thread
-  double acc[64];
+  const int lane = t & 63, l16 = lane & 15, lk = lane >> 4, m0 = (t >> 6) * 32;
+  d4v acc[2][2] = {};
+  constexpr int KS = 8;  // k steps (of 4) whose operands are loaded together
+  for (int q0 = 0; q0 < TBS; q0 += 4 * KS) {
+    double a[2][KS];
 #pragma unroll
-  for (int i = 0; i < 64; ++i) acc[i] = 0.0;
-  for (int q = 0; q < TBS; ++q) {
-    const double b = B[q][j];
-    const double* dq = Wk + (int64_t)q * TBS + i0;  // column q of inv(T_kk), same for all lanes
+    for (int q = 0; q < KS; ++q)
 #pragma unroll
-    for (int i = 0; i < 64; ++i) acc[i] += dq[i] * b;
+      for (int i = 0; i < 2; ++i) a[i][q] = Wk[(int64_t)(q0 + 4 * q + lk) * TBS + m0 + 16 * i + l16];
+#pragma unroll
+    for (int q = 0; q < KS; ++q) {
+      double b[2];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) b[j] = B[16 * j + l16][q0 + 4 * q + lk];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][q], b[j], acc[i][j], 0, 0, 0);
+    }
   }
-  double* G = Wk + (int64_t)(TBS + j) * TBS + i0;
+  double* G = Wk + (int64_t)(TBS + blockIdx.y * CPC) * TBS;
 #pragma unroll
-  for (int i = 0; i < 64; ++i) G[i] = -acc[i];
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) G[(int64_t)(16 * j + l16) * TBS + m0 + 16 * i + 4 * r + lk] = -acc[i][j][r];
 }
 
 // One block step.  cur: the block whose solution is final (outside [0, nblk) at
@@ -308,11 +371,11 @@ int trsv_prepare(const T* LU, int64_t lda, int n, int trans, double* W, int* fla
   diag_inverse_kernel<T><<<nblk, 256, 0, s>>>(LU, lda, n, trans ? 0 : 1, trans, Wb);
   if (nblk > 1) {
     if (!trans) {
-      couple_kernel<T, false, true><<<nblk - 1, 256, 0, s>>>(LU, lda, n, nblk, Wf);
-      couple_kernel<T, false, false><<<nblk - 1, 256, 0, s>>>(LU, lda, n, nblk, Wb);
+      couple_kernel<T, false, true><<<dim3(nblk - 1, TBS / CPC), 256, 0, s>>>(LU, lda, n, nblk, Wf);
+      couple_kernel<T, false, false><<<dim3(nblk - 1, TBS / CPC), 256, 0, s>>>(LU, lda, n, nblk, Wb);
     } else {
-      couple_kernel<T, true, true><<<nblk - 1, 256, 0, s>>>(LU, lda, n, nblk, Wf);
-      couple_kernel<T, true, false><<<nblk - 1, 256, 0, s>>>(LU, lda, n, nblk, Wb);
+      couple_kernel<T, true, true><<<dim3(nblk - 1, TBS / CPC), 256, 0, s>>>(LU, lda, n, nblk, Wf);
+      couple_kernel<T, true, false><<<dim3(nblk - 1, TBS / CPC), 256, 0, s>>>(LU, lda, n, nblk, Wb);
     }
   }
   KAD_HIP_CHECK(hipGetLastError());
@@ -381,8 +444,8 @@ int trsv_prepare_batched(const double* LU, int64_t lda, int n, int nbat, int64_t
   diag_inverse_kernel<double><<<dim3(nblk, nbat), 256, 0, s>>>(LU, lda, n, 0, 0, Wf, sA, sW);
   diag_inverse_kernel<double><<<dim3(nblk, nbat), 256, 0, s>>>(LU, lda, n, 1, 0, Wb, sA, sW);
   if (nblk > 1) {
-    couple_kernel<double, false, true><<<dim3(nblk - 1, nbat), 256, 0, s>>>(LU, lda, n, nblk, Wf, sA, sW);
-    couple_kernel<double, false, false><<<dim3(nblk - 1, nbat), 256, 0, s>>>(LU, lda, n, nblk, Wb, sA, sW);
+    couple_kernel<double, false, true><<<dim3(nblk - 1, TBS / CPC, nbat), 256, 0, s>>>(LU, lda, n, nblk, Wf, sA, sW);
+    couple_kernel<double, false, false><<<dim3(nblk - 1, TBS / CPC, nbat), 256, 0, s>>>(LU, lda, n, nblk, Wb, sA, sW);
   }
   KAD_HIP_CHECK(hipGetLastError());
   return KAD_OK;
