@@ -173,9 +173,11 @@ int trtri_rec(const T* L, int64_t lda, int nb, T* Linv, int64_t ldo, LuWork& w) 
 // Structural-zero masks of the trailing update: per 128-row tile of the L panel
 // (rows x ncols) and per 128-column tile of the U row panel (nrows x cols): 1 if the
 // tile holds any entry != 0 (NaN counts as nonzero), else 0.
+// 1024 threads and 8 loads in flight each: a tile's 256 columns are 4 round trips to
+// memory (128 dependent ones took 36 us).
 template <typename T>
-__global__ __launch_bounds__(256) void row_tile_mask_kernel(const T* __restrict__ A, int64_t lda, int nrows,
-                                                            int ncols, int* __restrict__ mask, int nzrows = -1) {
+__global__ __launch_bounds__(1024) void row_tile_mask_kernel(const T* __restrict__ A, int64_t lda, int nrows,
+                                                             int ncols, int* __restrict__ mask, int nzrows = -1) {
   // rows at or past nzrows (when given) are known to be zero: those tiles are not read
   if (nzrows >= 0 && (int)blockIdx.x * 128 >= nzrows) {
     if (threadIdx.x == 0) mask[blockIdx.x] = 0;
@@ -184,29 +186,39 @@ __global__ __launch_bounds__(256) void row_tile_mask_kernel(const T* __restrict_
   const int r = blockIdx.x * 128 + (threadIdx.x & 127);
   int any = 0;
   if (r < nrows)
-    for (int c = threadIdx.x >> 7; c < ncols; c += 2) any |= (A[r + (int64_t)c * lda] != T(0));
+    for (int c0 = threadIdx.x >> 7; c0 < ncols; c0 += 64) {
+      T v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = c0 + 8 * u < ncols ? A[r + (int64_t)(c0 + 8 * u) * lda] : T(0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) any |= v[u] != T(0);
+    }
   any = __syncthreads_or(any);
   if (threadIdx.x == 0) mask[blockIdx.x] = any;
 }
-// Last nonzero row (or -1) of each 128-column tile within each 2048-row chunk:
-// out[chunk * ntc + tile].  One workgroup per (tile, chunk); rows coalesced.
+// Last nonzero row of each 128-column tile: out[tile] = max over the 2048-row chunks
+// (workgroup (tile, chunk); out starts at -1).  A chunk is read from its end, 32 rows at
+// a time, until a nonzero is met, so a dense matrix costs one step of it (a full scan
+// took 180 us at n = 1215, 470 at 8191).
 template <typename T>
 __global__ __launch_bounds__(256) void col_extent_kernel(const T* __restrict__ A, int64_t lda, int n,
                                                          int* __restrict__ out) {
-  __shared__ int red[256];
   const int c0 = blockIdx.x * 128, r0 = blockIdx.y * 2048;
   const int ce = min(c0 + 128, n), re = min(r0 + 2048, n);
-  int last = -1;
-  for (int c = c0; c < ce; ++c)
-    for (int r = r0 + threadIdx.x; r < re; r += 256)
-      if (A[r + (int64_t)c * lda] != T(0)) last = max(last, r);
-  red[threadIdx.x] = last;
-  __syncthreads();
-  for (int st = 128; st > 0; st >>= 1) {
-    if (threadIdx.x < st) red[threadIdx.x] = max(red[threadIdx.x], red[threadIdx.x + st]);
-    __syncthreads();
+  const int tr = threadIdx.x & 31, tc = threadIdx.x >> 5;  // row within a step, one of 8 column groups
+  for (int rb = r0 + (re - r0 - 1) / 32 * 32; rb >= r0; rb -= 32) {
+    const int r = rb + tr;
+    int any = 0;
+    if (r < re) {
+      T v[16];
+#pragma unroll
+      for (int u = 0; u < 16; ++u) v[u] = c0 + tc + 8 * u < ce ? A[r + (int64_t)(c0 + tc + 8 * u) * lda] : T(0);
+#pragma unroll
+      for (int u = 0; u < 16; ++u) any |= v[u] != T(0);
+    }
+    if (any) atomicMax(&out[blockIdx.x], r);
+    if (__syncthreads_or(any)) return;
   }
-  if (threadIdx.x == 0) out[blockIdx.y * gridDim.x + blockIdx.x] = red[0];
 }
 
 // Compacted lists of the active row / column tiles: list[0..) rows, list[stride..)
@@ -225,13 +237,19 @@ __global__ void tile_lists_kernel(const int* __restrict__ rmask, int nr, const i
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void col_tile_mask_kernel(const T* __restrict__ A, int64_t lda, int nrows,
-                                                            int ncols, int* __restrict__ mask) {
-  const int c0 = blockIdx.x * 128;
-  const int ce = min(c0 + 128, ncols);
+__global__ __launch_bounds__(1024) void col_tile_mask_kernel(const T* __restrict__ A, int64_t lda, int nrows,
+                                                             int ncols, int* __restrict__ mask) {
+  const int c0 = blockIdx.x * 128 + (threadIdx.x >> 8);
+  const int ce = min((int)blockIdx.x * 128 + 128, ncols);
   int any = 0;
-  for (int c = c0; c < ce; ++c)
-    for (int r = threadIdx.x; r < nrows; r += 256) any |= (A[r + (int64_t)c * lda] != T(0));
+  for (int r = threadIdx.x & 255; r < nrows; r += 256)
+    for (int c = c0; c < ce; c += 32) {
+      T v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) v[u] = c + 4 * u < ce ? A[r + (int64_t)(c + 4 * u) * lda] : T(0);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) any |= v[u] != T(0);
+    }
   any = __syncthreads_or(any);
   if (threadIdx.x == 0) mask[blockIdx.x] = any;
 }
@@ -461,75 +479,52 @@ int lu_solve_permuted_batched(const double* LU, int64_t lda, int n, int nbat, in
   return trsm_left_upper<double>(LU, lda, n, B, ldb, nrhs, w, F64, nbat, sA, sB, zcols);
 }
 
-// Row interchanges of pivots [k1, k2) (at most 512) applied to COLS columns per
-// workgroup through LDS.  Slots 0 .. nsw-1 hold rows k1 .. k2-1; slot nsw + j holds the
-// pivot row of step j when that row lies below k2 and step j is its first occurrence.
-// All slots are loaded in parallel, the interchange sequence is replayed in LDS (one
-// thread per column, LAPACK order), and every touched row is written back: the
-// result equals the sequential interchanges.
+// Row interchanges of pivots [k1, k2) (at most NSW) applied to COLS columns per
+// workgroup.  The affected rows are k1 .. k2-1 and the pivot rows below them (2 nsw
+// entries; a row that occurs twice carries the same value both times); entry e's content
+// comes from the row found by undoing the interchanges in reverse order, every entry at
+// once from the pivots in LDS.  Then one gather (COLS loads per entry in flight) and one
+// scatter.  Bound by latency: replaying the interchanges in LDS, one thread per column,
+// cost most of the kernel's 52 us (256 interchanges, n = 1215; 60 us at 8191); this one
+// takes 14 (24).
 template <typename T, int NSW, int COLS>
-__global__ __launch_bounds__(256) void laswp_lds_kernel(T* __restrict__ A, int64_t lda, int c0, int c1,
-                                                        const int* __restrict__ ipiv, int k1, int k2, int64_t sA,
-                                                        int sP) {
+__global__ __launch_bounds__(256) void laswp_gather_kernel(T* __restrict__ A, int64_t lda, int c0, int c1,
+                                                           const int* __restrict__ ipiv, int k1, int k2, int64_t sA,
+                                                           int sP) {
   A += (int64_t)blockIdx.y * sA;  // matrix blockIdx.y of a batch
   ipiv += (int64_t)blockIdx.y * sP;
-  __shared__ double vals[2 * NSW * COLS];  // [slot][column]
-  __shared__ int slot_of[NSW];
-  __shared__ int prow[NSW];                // row of slot nsw + j, or -1
-  __shared__ int piv[NSW];                 // ipiv[k1 .. k2), staged once (the searches below read it)
-  const int nsw = k2 - k1;                 // <= NSW (checked by the launcher)
+  constexpr int NE = 2 * NSW / 256;  // entries per thread
+  __shared__ int piv[NSW];
+  const int nsw = k2 - k1;           // <= NSW (checked by the launcher)
   const int t = threadIdx.x;
   const int cb = c0 + blockIdx.x * COLS;
   const int nc = min(COLS, c1 - cb);
   for (int j = t; j < nsw; j += 256) piv[j] = ipiv[k1 + j];
   __syncthreads();
-  for (int j = t; j < nsw; j += 256) {
-    const int p = piv[j];
-    if (p < k2) {
-      slot_of[j] = p - k1;
-      prow[j] = -1;
-    } else {
-      int first = j;
-      for (int q = 0; q < j; ++q)
-        if (piv[q] == p) {
-          first = q;
-          break;
-        }
-      slot_of[j] = nsw + first;
-      prow[j] = (first == j) ? p : -1;
-    }
+  int row[NE], src[NE];
+#pragma unroll
+  for (int u = 0; u < NE; ++u) {
+    const int e = u * 256 + t;
+    row[u] = e < nsw ? k1 + e : (e < 2 * nsw && piv[e - nsw] >= k2 ? piv[e - nsw] : -1);
+    src[u] = row[u];
   }
-  __syncthreads();
-  // load: rows k1 .. k2-1 (coalesced along rows) and the first-occurrence pivot rows
-  for (int e = t; e < nsw * COLS; e += 256) {
-    const int r = e % nsw, c = e / nsw;
-    if (c < nc) vals[r * COLS + c] = (double)A[(k1 + r) + (int64_t)(cb + c) * lda];
+  for (int j = nsw - 1; j >= 0; --j) {
+    const int r = k1 + j, p = piv[j];
+#pragma unroll
+    for (int u = 0; u < NE; ++u) src[u] = src[u] == r ? p : (src[u] == p ? r : src[u]);
   }
-  for (int e = t; e < nsw * COLS; e += 256) {
-    const int j = e % nsw, c = e / nsw;
-    const int p = prow[j];
-    if (c < nc && p >= 0) vals[(nsw + j) * COLS + c] = (double)A[p + (int64_t)(cb + c) * lda];
-  }
-  __syncthreads();
-  if (t < nc)
-    for (int j = 0; j < nsw; ++j) {
-      const int b = slot_of[j];
-      if (b != j) {
-        const double x = vals[j * COLS + t];
-        vals[j * COLS + t] = vals[b * COLS + t];
-        vals[b * COLS + t] = x;
-      }
-    }
-  __syncthreads();
-  for (int e = t; e < nsw * COLS; e += 256) {
-    const int r = e % nsw, c = e / nsw;
-    if (c < nc) A[(k1 + r) + (int64_t)(cb + c) * lda] = (T)vals[r * COLS + c];
-  }
-  for (int e = t; e < nsw * COLS; e += 256) {
-    const int j = e % nsw, c = e / nsw;
-    const int p = prow[j];
-    if (c < nc && p >= 0) A[p + (int64_t)(cb + c) * lda] = (T)vals[(nsw + j) * COLS + c];
-  }
+  T val[NE][COLS];
+#pragma unroll
+  for (int u = 0; u < NE; ++u)
+#pragma unroll
+    for (int c = 0; c < COLS; ++c)
+      if (row[u] >= 0 && c < nc) val[u][c] = A[src[u] + (int64_t)(cb + c) * lda];
+  __syncthreads();  // every read of these columns precedes every write
+#pragma unroll
+  for (int u = 0; u < NE; ++u)
+#pragma unroll
+    for (int c = 0; c < COLS; ++c)
+      if (row[u] >= 0 && c < nc) A[row[u] + (int64_t)(cb + c) * lda] = val[u][c];
 }
 
 template <typename T>
@@ -538,13 +533,11 @@ int laswp(T* A, int64_t lda, int c0, int c1, const int* ipiv, int k1, int k2, Lu
   if (c1 <= c0 || k2 <= k1) return KAD_OK;
   const int nsw = k2 - k1;
   const unsigned nz = (unsigned)bt.nbat;
-  // 8 (4) columns per workgroup: ~33 KB of LDS, so the workgroups fit beside the
-  // concurrent update's GEMM workgroups instead of waiting for a whole CU
   if (nsw <= 256) {
-    laswp_lds_kernel<T, 256, 8><<<dim3((unsigned)cdiv(c1 - c0, 8), nz), 256, 0, w.stream>>>(A, lda, c0, c1, ipiv, k1,
+    laswp_gather_kernel<T, 256, 8><<<dim3((unsigned)cdiv(c1 - c0, 8), nz), 256, 0, w.stream>>>(A, lda, c0, c1, ipiv, k1,
                                                                                            k2, bt.sA, bt.sP);
   } else if (nsw <= 512) {
-    laswp_lds_kernel<T, 512, 4><<<dim3((unsigned)cdiv(c1 - c0, 4), nz), 256, 0, w.stream>>>(A, lda, c0, c1, ipiv, k1,
+    laswp_gather_kernel<T, 512, 4><<<dim3((unsigned)cdiv(c1 - c0, 4), nz), 256, 0, w.stream>>>(A, lda, c0, c1, ipiv, k1,
                                                                                            k2, bt.sA, bt.sP);
   } else {
     laswp_kernel<T><<<dim3((unsigned)cdiv(c1 - c0, 256), nz), 256, 0, w.stream>>>(A, lda, c0, c1, ipiv, k1, k2, bt.sA,
@@ -1448,13 +1441,11 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
   const int ntc = (int)cdiv(n, 128), nrc = (int)cdiv(n, 2048);
   std::vector<int> ext(ntc, bat ? n - 1 : -1);
   if (!bat) {
+    KAD_HIP_CHECK(hipMemsetAsync(w.ext, 0xff, ntc * sizeof(int), w.stream));  // -1
     col_extent_kernel<T><<<dim3(ntc, nrc), 256, 0, w.stream>>>(A, lda, n, w.ext);
     KAD_HIP_CHECK(hipGetLastError());
-    std::vector<int> hext((size_t)ntc * nrc);
-    KAD_HIP_CHECK(hipMemcpyAsync(hext.data(), w.ext, hext.size() * sizeof(int), hipMemcpyDeviceToHost, w.stream));
+    KAD_HIP_CHECK(hipMemcpyAsync(ext.data(), w.ext, ntc * sizeof(int), hipMemcpyDeviceToHost, w.stream));
     KAD_HIP_CHECK(hipStreamSynchronize(w.stream));
-    for (int r = 0; r < nrc; ++r)
-      for (int t = 0; t < ntc; ++t) ext[t] = std::max(ext[t], hext[(size_t)r * ntc + t]);
   }
   int r_prev = 0;
   // factor panel [k0, k1) on the panel stream (rows [k0, R)), then its L21 mask
@@ -1469,7 +1460,7 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
     if (rc) return rc;
     if (k1 < n && mask) {
       // the panel's rows at or below R are zero in its columns
-      row_tile_mask_kernel<T><<<(unsigned)cdiv(n - k1, 128), 256, 0, wp.stream>>>(A + k1 + (int64_t)k0 * lda, lda,
+      row_tile_mask_kernel<T><<<(unsigned)cdiv(n - k1, 128), 1024, 0, wp.stream>>>(A + k1 + (int64_t)k0 * lda, lda,
                                                                                  n - k1, k1 - k0, mask, R - k1);
       KAD_HIP_CHECK(hipGetLastError());
     }
@@ -1505,7 +1496,7 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
       rc = laswp<T>(A, lda, k2, k3, ipiv, k0, k1, wm);
       if (rc) return rc;
       // structural zeros of A12 (column tiles; U12 = L11^{-1} A12 keeps them)
-      col_tile_mask_kernel<T><<<(unsigned)cdiv(k3 - k2, 128), 256, 0, w.stream>>>(A + k0 + (int64_t)k2 * lda, lda,
+      col_tile_mask_kernel<T><<<(unsigned)cdiv(k3 - k2, 128), 1024, 0, w.stream>>>(A + k0 + (int64_t)k2 * lda, lda,
                                                                                  k1 - k0, k3 - k2, w.mask_c);
       KAD_HIP_CHECK(hipGetLastError());
       rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k2 * lda, lda, k3 - k2, wm, gemm_prec,
@@ -1529,7 +1520,7 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
     } else if (k3 < n) {
       rc = laswp<T>(A, lda, k3, n, ipiv, k0, k1, wm);
       if (rc) return rc;
-      col_tile_mask_kernel<T><<<(unsigned)cdiv(n - k3, 128), 256, 0, w.stream>>>(A + k0 + (int64_t)k3 * lda, lda,
+      col_tile_mask_kernel<T><<<(unsigned)cdiv(n - k3, 128), 1024, 0, w.stream>>>(A + k0 + (int64_t)k3 * lda, lda,
                                                                                 k1 - k0, n - k3, w.mask_c2);
       KAD_HIP_CHECK(hipGetLastError());
       rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k3 * lda, lda, n - k3, wm, gemm_prec,
