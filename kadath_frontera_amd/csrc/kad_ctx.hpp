@@ -65,10 +65,9 @@ struct LuWork {
   unsigned* bcnt = nullptr;     // arrival counters of the static-pivot base panel (LU_MAX_BATCH, kept at 0)
   unsigned long long* bgrowth = nullptr;  // largest |multiplier| per matrix of a static-pivot factorisation
   int red_cap = 0;
-  void* tinv = nullptr;         // unit-lower inverse, nb x nb
-  void* tmp = nullptr;          // GEMM scratch for L11^{-1} A12
+  void* tmp = nullptr;          // row gathers of the deferred left interchanges
   size_t tmp_bytes = 0;
-  void* tmp2 = nullptr;         // scratch of the recursive triangular inverse / panel row gather
+  void* tmp2 = nullptr;         // panel row gather of the per-column kernels
   size_t tmp2_bytes = 0;
   int* map = nullptr;           // 2 x n logical -> physical row maps of the base panel
   int* mask_r = nullptr;        // per 128-row tile of the L panel: any nonzero
@@ -84,10 +83,6 @@ struct LuWork {
   // look-ahead: the next panel is updated and factored on a second stream
   hipStream_t stream2 = nullptr;
   hipEvent_t ev_panel[2] = {nullptr, nullptr}, ev_next[2] = {nullptr, nullptr}, ev_start = nullptr;
-  // triangular-inverse and GEMM scratch of the main stream (the panel stream uses tinv / tmp)
-  void* tinv_m = nullptr;
-  void* tmp_m = nullptr;
-  size_t tmp_m_bytes = 0;
   // persistent base panel: the flagged exchange slots, the abort word (ffp_sync[2])
   // and the CU count that bounds its grid
   void* ffp = nullptr;
@@ -159,7 +154,7 @@ struct Ctx {
   hipStream_t stream = nullptr;
   bool own_stream = false;
   LuWork lu;
-  size_t cap_redv = 0, cap_redi = 0, cap_tinv = 0, cap_map = 0, cap_mask = 0, cap_tinv_m = 0;
+  size_t cap_redv = 0, cap_redi = 0, cap_map = 0, cap_mask = 0;
   double* gemv_part = nullptr;
   size_t cap_part = 0;
   double* vwork = nullptr;

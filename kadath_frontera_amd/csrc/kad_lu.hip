@@ -14,8 +14,8 @@
 // performs exact partial pivoting (first index of max |a|, as idamax) and whose
 // internal updates are MFMA GEMMs.  The trailing update A22 -= L21 U12 is the
 // MFMA GEMM of kad_gemm.hip in the factor precision (f64, f32, or bf16 operands
-// with f32 accumulation).  U12 = L11^{-1} A12 is a blocked substitution whose
-// updates are GEMMs and whose 64-row leaves use explicit inverses.  Trailing-update
+// with f32 accumulation).  U12 = L11^{-1} A12 is a blocked substitution,
+// one launch per 256 rows.  Trailing-update
 // tile pairs whose L21 row tile or U12 column tile is exactly zero are skipped
 // (structural zeros of a block-sparse Jacobian); the result is unchanged.
 #include "kad_common.hpp"
@@ -87,36 +87,6 @@ __global__ void laswp_kernel(T* A, int64_t lda, int c0, int c1, const int* __res
   }
 }
 
-// Inverse of a unit-lower nb x nb block (nb <= 64), written as a full square
-// (zeros above, ones on the diagonal) into Linv (ld ldo).  One workgroup of 256:
-// X = I, then for j = 0..nb-1 every (i > j, c <= j) entry does
-// X[i][c] -= L[i][j] X[j][c]  (row-oriented forward substitution, one barrier per j).
-template <typename T>
-__global__ __launch_bounds__(256) void trtri_small_kernel(const T* L, int64_t lda, int nb, T* Linv, int64_t ldo) {
-  __shared__ double Ls[64][65];
-  __shared__ double X[64][65];
-  const int t = threadIdx.x;
-  for (int e = t; e < nb * nb; e += 256) {
-    const int i = e % nb, c = e / nb;
-    Ls[i][c] = (double)L[i + (int64_t)c * lda];
-    X[i][c] = (i == c) ? 1.0 : 0.0;
-  }
-  __syncthreads();
-  for (int j = 0; j < nb - 1; ++j) {
-    // rows i in (j, nb), columns c in [0, j]
-    const int nrow = nb - 1 - j, ncol = j + 1;
-    for (int e = t; e < nrow * ncol; e += 256) {
-      const int i = j + 1 + e % nrow, c = e / nrow;
-      X[i][c] -= Ls[i][j] * X[j][c];
-    }
-    __syncthreads();
-  }
-  for (int e = t; e < nb * nb; e += 256) {
-    const int i = e % nb, c = e / nb;
-    Linv[i + (int64_t)c * ldo] = (T)X[i][c];
-  }
-}
-
 template <typename T>
 __global__ void copy2d_kernel(const T* src, int64_t lds, T* dst, int64_t ldd, int m, int n) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -124,51 +94,7 @@ __global__ void copy2d_kernel(const T* src, int64_t lds, T* dst, int64_t ldd, in
   if (i < m && c < n) dst[i + (int64_t)c * ldd] = src[i + (int64_t)c * lds];
 }
 
-template <typename T>
-__global__ void negate_copy_kernel(const T* src, int64_t lds, T* dst, int64_t ldd, int m, int n, T scale) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int c = blockIdx.y;
-  if (i < m && c < n) dst[i + (int64_t)c * ldd] = scale * src[i + (int64_t)c * lds];
-}
-
-template <typename T>
-__global__ void zero_upper_kernel(T* Lv, int64_t ld, int nb) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int c = blockIdx.y;
-  if (i < nb && c < nb && i < c) Lv[i + (int64_t)c * ld] = T(0);
-}
-
 template <typename T> constexpr int prec_of() { return sizeof(T) == 8 ? F64 : F32; }
-
-// Recursive inverse of unit-lower L (nb x nb) into Linv (ld ldo), full square.
-template <typename T>
-int trtri_rec(const T* L, int64_t lda, int nb, T* Linv, int64_t ldo, LuWork& w) {
-  if (nb <= 64) {
-    trtri_small_kernel<T><<<1, 256, 0, w.stream>>>(L, lda, nb, Linv, ldo);
-    KAD_HIP_CHECK(hipGetLastError());
-    return KAD_OK;
-  }
-  const int h = nb / 2;
-  int rc = trtri_rec<T>(L, lda, h, Linv, ldo, w);
-  if (rc) return rc;
-  rc = trtri_rec<T>(L + h + (int64_t)h * lda, lda, nb - h, Linv + h + (int64_t)h * ldo, ldo, w);
-  if (rc) return rc;
-  // T1 = L21 * Linv11  ((nb-h) x h) into tmp2
-  T* t1 = (T*)w.tmp2;
-  rc = gemm_launch(prec_of<T>(), GOP_SET, nb - h, h, h, L + h, lda, Linv, ldo, t1, nb - h, w.stream);
-  if (rc) return rc;
-  // Linv21 = -Linv22 * T1
-  T* out21 = Linv + h;
-  rc = gemm_launch(prec_of<T>(), GOP_SET, nb - h, h, nb - h, Linv + h + (int64_t)h * ldo, ldo, t1, nb - h, out21, ldo,
-                   w.stream);
-  if (rc) return rc;
-  dim3 g((unsigned)cdiv(nb - h, 256), h);
-  negate_copy_kernel<T><<<g, 256, 0, w.stream>>>(out21, ldo, out21, ldo, nb - h, h, T(-1));
-  dim3 gz((unsigned)cdiv(nb, 256), nb);
-  zero_upper_kernel<T><<<gz, 256, 0, w.stream>>>(Linv, ldo, nb);
-  KAD_HIP_CHECK(hipGetLastError());
-  return KAD_OK;
-}
 
 // Structural-zero masks of the trailing update: per 128-row tile of the L panel
 // (rows x ncols) and per 128-column tile of the U row panel (nrows x cols): 1 if the
@@ -254,25 +180,6 @@ __global__ __launch_bounds__(1024) void col_tile_mask_kernel(const T* __restrict
   if (threadIdx.x == 0) mask[blockIdx.x] = any;
 }
 
-// A12 <- L^{-1} A12 with L unit lower (r x r).  Blocked substitution as LAPACK's
-// dtrsm: X1 = L11^{-1} B1, B2 -= L21 X1, X2 = L22^{-1} B2, recursively; only the
-// leaves (at most 64 rows) use an explicit inverse, whose error grows with the
-// leaf's condition number.
-constexpr int TRSM_LEAF = 64;
-
-// L X = B in place for a unit-lower L of order 32 and B of 32 rows: one lane per
-// column of B, 64 columns per wave.  The lane keeps the rows not yet final in a
-// window y[0..31] of registers: at step k, y[0] = B(k) is final (stored), and every
-// other entry is updated and shifted down, y[i-1] = y[i] - L(k+i, k) y[0] -- the
-// indices into y are constants, so the step loop needs no unrolling and no dynamic
-// register indexing; entries past the rows still open compute values that are
-// never used.  L is staged in LDS once and read with broadcast loads.  The order of
-// operations on every B(i) is the column-oriented substitution of LAPACK's xTRSM
-// ('L', 'L', 'N', 'U').  cmask (optional): 128-column tiles of B that are
-// structurally zero stay untouched; a batch's ZeroRhs skips the 64-column groups whose
-// rows here are all zero.
-constexpr int TRSM_FUSED = 32;
-
 // Where a batch's right-hand sides are known to be zero (a batch of sparse right-hand
 // sides such as unit vectors); the solves skip that work, whose results would be zero.
 struct ZeroRhs {
@@ -283,36 +190,161 @@ struct ZeroRhs {
   int row0 = 0;  // the sub-system's first row in the full system (rows of start)
 };
 
+// Triangular solves of up to 256 rows in one launch: L X = B (unit lower) or, UP, U X = B
+// (non-unit upper), in place, 16 columns of B per workgroup, held in LDS.
+// The rows are taken 32 at a time (from the last for UP):
+// - substitution with the 32 x 32 diagonal block, in LAPACK xTRSM's order of operations:
+//   a column of B is spread over the 16 lanes of a DPP row, two rows per lane (reversed
+//   for UP), and the solved entry of each step reaches the other lanes by a row
+//   broadcast, so a step is one broadcast and two multiply-adds (and a division for UP);
+// - the rows not yet solved subtract the block's product with the matrix cores (16 x 16
+//   tiles, k = 32), whose operands were loaded before the substitution.
+// Bound by latency, not by arithmetic: it replaces 8 launches of a 32-row leaf (a lane
+// per column, 15-20 us each) and 7 products between them (10-13 us) per 256 rows, which
+// were on the panel's critical path.  TRSM_FIGURES
+constexpr int TRB = 32;          // rows per step
+constexpr int TRSM_ROWS = 256;   // most rows of one launch
+constexpr int TRSM_COLS = 16;    // columns per workgroup
+
 template <typename T>
-__global__ __launch_bounds__(64, 4) void trsm_leaf_kernel(const T* __restrict__ L, int64_t lda, T* __restrict__ B,
-                                                       int64_t ldb, int ncols, const int* __restrict__ cmask,
-                                                       int64_t sL, int64_t sB, ZeroRhs zr) {
-  constexpr int R = TRSM_FUSED;
-  L += (int64_t)blockIdx.y * sL;  // system blockIdx.y of a batch
-  B += (int64_t)blockIdx.y * sB;
-  __builtin_amdgcn_s_setprio(2);  // a serial chain on the critical path, beside the bulk GEMM
-  __shared__ T Ls[R * R + R];  // column-major, Ls[i + R k] = L(i, k); R entries of padding read past the end
-  const int c0 = blockIdx.x * 64;
-  if (cmask && !cmask[c0 / 128]) return;  // uniform: the block lies in one 128-column tile
-  if (zr.cols && c0 >= zr.cols[blockIdx.y]) return;
-  if (zr.start && zr.start[(int)blockIdx.y * zr.ng + (int)blockIdx.x] >= zr.row0 + R) return;
-  for (int e = threadIdx.x; e < R * R; e += 64) Ls[e] = L[(int64_t)(e % R) + (int64_t)(e / R) * lda];
-  if (threadIdx.x < R) Ls[R * R + threadIdx.x] = T(0);
-  const int c = c0 + threadIdx.x;
-  const bool act = c < ncols;
-  T* b = B + (int64_t)(act ? c : c0) * ldb;
-  T y[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) y[i] = act ? b[i] : T(0);
-  __syncthreads();
-#pragma unroll 1
-  for (int k = 0; k < R; ++k) {
-    const T xk = y[0];
-    if (act) b[k] = xk;
-    const T* lk = Ls + k + R * k;  // lk[i] = L(k + i, k); i + k < 2 R stays inside Ls
-#pragma unroll
-    for (int i = 1; i < R; ++i) y[i - 1] = y[i] - lk[i] * xk;
+struct Mfma16;  // 16 x 16 x 4 tile: register r of lane l holds row(l, r), column l % 16
+template <>
+struct Mfma16<double> {
+  typedef d4v V;
+  static __device__ __forceinline__ V mul(double a, double b, V c) {
+    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
   }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * r + (lane >> 4); }
+};
+template <>
+struct Mfma16<float> {
+  typedef f4v V;
+  static __device__ __forceinline__ V mul(float a, float b, V c) {
+    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+  }
+  static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
+};
+
+// The value of lane N of every 16-lane row, to all its lanes (DPP row_newbcast).
+template <int N>
+__device__ __forceinline__ float row_bcast(float v) {
+  const int w = __builtin_bit_cast(int, v);
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(w, w, 0x150 + N, 0xF, 0xF, false));
+}
+template <int N>
+__device__ __forceinline__ double row_bcast(double v) {
+  const long long b = __double_as_longlong(v);
+  const int hi = (int)(b >> 32), lo = (int)b;
+  const int ohi = __builtin_amdgcn_update_dpp(hi, hi, 0x150 + N, 0xF, 0xF, false);
+  const int olo = __builtin_amdgcn_update_dpp(lo, lo, 0x150 + N, 0xF, 0xF, false);
+  return __longlong_as_double(((long long)ohi << 32) | (unsigned)olo);
+}
+
+// Steps K .. 31 of the substitution: lane g of a row holds rows 2g and 2g + 1 (y0, y1).
+template <typename T, bool UP, int K>
+__device__ __forceinline__ void trsm_steps(T& y0, T& y1, const T* __restrict__ Ls, const T* __restrict__ ds, int g) {
+  const T l0 = Ls[K * TRB + 2 * g], l1 = Ls[K * TRB + 2 * g + 1];
+  T q = (K & 1) ? y1 : y0;
+  if constexpr (UP) {
+    q = q / ds[K];
+    if (g == K / 2) ((K & 1) ? y1 : y0) = q;
+  }
+  const T x = row_bcast<K / 2>(q);
+  y0 = 2 * g > K ? y0 - l0 * x : y0;
+  y1 = 2 * g + 1 > K ? y1 - l1 * x : y1;
+  if constexpr (K + 1 < TRB) trsm_steps<T, UP, K + 1>(y0, y1, Ls, ds, g);
+}
+
+// r <= 256 rows (UP: a multiple of 32); system blockIdx.y of a batch.  cmask (optional):
+// 128-column tiles of B that are structurally zero stay untouched; zr: as ZeroRhs.
+template <typename T, bool UP>
+__global__ __launch_bounds__(256) void trsm_block_kernel(const T* __restrict__ L, int64_t lda, T* __restrict__ B,
+                                                         int64_t ldb, int r, int ncols, const int* __restrict__ cmask,
+                                                         int64_t sL, int64_t sB, ZeroRhs zr) {
+  constexpr int LD = TRSM_ROWS + 2;  // 16 columns x 4 words apart: conflict-free tile reads
+  __shared__ __align__(16) T X[TRSM_COLS * LD];
+  __shared__ __align__(16) T Ls[TRB * TRB];
+  __shared__ T ds[TRB];
+  const int c0 = blockIdx.x * TRSM_COLS;
+  if (cmask && !cmask[c0 / 128]) return;
+  if (zr.cols && c0 >= zr.cols[blockIdx.y]) return;
+  if (zr.start && zr.start[(int)blockIdx.y * zr.ng + c0 / 64] >= zr.row0 + r) return;
+  __builtin_amdgcn_s_setprio(2);  // on the critical path, beside the bulk GEMM
+  L += (int64_t)blockIdx.y * sL;
+  B += (int64_t)blockIdx.y * sB;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, l16 = lane & 15, lk = lane >> 4;
+  const int nbk = (r + TRB - 1) / TRB;
+  // 32 x 32 diagonal block of step `it`: column-major, rows and columns reversed for UP;
+  // only the part below the diagonal is used, and the diagonal (UP)
+  auto diag = [&](int it, T (&v)[4]) {
+    const int o = (UP ? nbk - 1 - it : it) * TRB;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = u * 256 + tid;
+      const int i = UP ? TRB - 1 - e % TRB : e % TRB, k = UP ? TRB - 1 - e / TRB : e / TRB;
+      v[u] = (o + i < r && o + k < r) ? L[(o + i) + (int64_t)(o + k) * lda] : T(0);
+    }
+  };
+  T lv[4];
+  diag(0, lv);
+  {
+    T v[TRSM_COLS];
+#pragma unroll
+    for (int c = 0; c < TRSM_COLS; ++c)
+      v[c] = (tid < r && c0 + c < ncols) ? B[tid + (int64_t)(c0 + c) * ldb] : T(0);
+#pragma unroll
+    for (int c = 0; c < TRSM_COLS; ++c) X[c * LD + tid] = v[c];
+  }
+  for (int it = 0; it < nbk; ++it) {
+    const int kb = UP ? nbk - 1 - it : it;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int e = u * 256 + tid;
+      Ls[e] = lv[u];
+      if (e % TRB == e / TRB) ds[e % TRB] = lv[u];
+    }
+    // this wave's 16-row tiles of the update and their operands
+    const int t0 = (UP ? 0 : 2 * (kb + 1)) + wave, t1 = UP ? 2 * kb : 2 * nbk;
+    T a[4][8];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int row = 16 * (t0 + 4 * q) + l16;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) {
+        const int k = kb * TRB + 4 * s + lk;
+        a[q][s] = (t0 + 4 * q < t1 && row < r && k < r) ? L[row + (int64_t)k * lda] : T(0);
+      }
+    }
+    if (it + 1 < nbk) diag(it + 1, lv);
+    __syncthreads();
+    {
+      T* const xc = X + (wave * 4 + lk) * LD + kb * TRB;
+      const int i0 = UP ? TRB - 1 - 2 * l16 : 2 * l16, i1 = UP ? i0 - 1 : i0 + 1;
+      T y0 = xc[i0], y1 = xc[i1];
+      trsm_steps<T, UP, 0>(y0, y1, Ls, ds, l16);
+      xc[i0] = y0;
+      xc[i1] = y1;
+    }
+    __syncthreads();
+    T b[8];
+#pragma unroll
+    for (int s = 0; s < 8; ++s) b[s] = X[l16 * LD + kb * TRB + 4 * s + lk];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      if (t0 + 4 * q < t1) {
+        typename Mfma16<T>::V acc = {};
+#pragma unroll
+        for (int s = 0; s < 8; ++s) acc = Mfma16<T>::mul(a[q][s], b[s], acc);
+        T* const xr = X + l16 * LD + 16 * (t0 + 4 * q);
+#pragma unroll
+        for (int rr = 0; rr < 4; ++rr) xr[Mfma16<T>::row(lane, rr)] -= acc[rr];
+      }
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int c = 0; c < TRSM_COLS; ++c)
+    if (tid < r && c0 + c < ncols) B[tid + (int64_t)(c0 + c) * ldb] = X[c * LD + tid];
 }
 
 // C_z -= A_z B_z over a batch at strides (sa, sb, sc).  zr (may be NULL): B_z is zero
@@ -335,9 +367,10 @@ static int batched_sub(int prec, int m, int n, int k, const void* A, int64_t lda
   return gemm_launch_sel(prec, GOP_SUB, m, n, k, A, lda, B, ldb, C, ldc, sel, s);
 }
 
-// nbat > 1: nbat systems at L + z sL, A12 + z sB (no masks; r a multiple of 32, so
-// every leaf is a 32-row kernel).  zr (may be NULL): where the batch's right-hand sides
-// are zero; the work on those parts, which stay zero, is skipped.
+// A12 <- L^{-1} A12 with L unit lower (r x r): X1 = L11^{-1} B1, B2 -= L21 X1,
+// X2 = L22^{-1} B2, recursively, as LAPACK's dtrsm, down to blocks of one launch.
+// nbat > 1: nbat systems at L + z sL, A12 + z sB (no masks).  zr (may be NULL): where the
+// batch's right-hand sides are zero; the work on those parts, which stay zero, is skipped.
 template <typename T>
 int trsm_left_unit_lower(const T* L, int64_t lda, int r, T* A12, int64_t ld12, int ncols, LuWork& w, int gemm_prec,
                          const int* cmask = nullptr, int nbat = 1, int64_t sL = 0, int64_t sB = 0,
@@ -346,113 +379,51 @@ int trsm_left_unit_lower(const T* L, int64_t lda, int r, T* A12, int64_t ld12, i
   if (nbat > 1 && cmask) return arg_error("trsm_left_unit_lower: masks with a batch");
   if (zr && (nbat < 2 || (zr->start && zr->ng < cdiv(ncols, 64))))
     return arg_error("trsm_left_unit_lower: zero right-hand-side parts need a batch and a group per 64 columns");
-  if (r > TRSM_LEAF || r == 2 * TRSM_FUSED) {
-    const int h = std::max(32, (r / 2) / 32 * 32);
-    int rc = trsm_left_unit_lower<T>(L, lda, h, A12, ld12, ncols, w, gemm_prec, cmask, nbat, sL, sB, zr);
-    if (rc) return rc;
-    const int gp = gemm_prec == BF16 ? F32 : gemm_prec;
-    rc = nbat > 1 ? batched_sub(gp, r - h, ncols, h, L + h, lda, sL, A12, ld12, sB, A12 + h, ld12, sB, nbat, zr,
-                                w.stream)
-                  : gemm_launch_masked(gp, GOP_SUB, r - h, ncols, h, L + h, lda, A12, ld12, A12 + h, ld12, nullptr,
-                                       cmask, w.stream);
-    if (rc) return rc;
-    ZeroRhs z2;
-    if (zr) {
-      z2 = *zr;
-      z2.row0 += h;
-    }
-    return trsm_left_unit_lower<T>(L + h + (int64_t)h * lda, lda, r - h, A12 + h, ld12, ncols, w, gemm_prec, cmask,
-                                   nbat, sL, sB, zr ? &z2 : nullptr);
-  }
-  if (r == TRSM_FUSED) {
-    trsm_leaf_kernel<T><<<dim3((unsigned)cdiv(ncols, 64), nbat), 64, 0, w.stream>>>(L, lda, A12, ld12, ncols, cmask,
-                                                                                  sL, sB, zr ? *zr : ZeroRhs());
+  if (r <= TRSM_ROWS) {
+    trsm_block_kernel<T, false><<<dim3((unsigned)cdiv(ncols, TRSM_COLS), nbat), 256, 0, w.stream>>>(
+        L, lda, A12, ld12, r, ncols, cmask, sL, sB, zr ? *zr : ZeroRhs());
     KAD_HIP_CHECK(hipGetLastError());
     return KAD_OK;
   }
-  // leaves of other orders use an explicit inverse (one system)
-  if (nbat > 1) return arg_error("trsm_left_unit_lower: a batch needs orders that are multiples of 32");
-  T* linv = (T*)w.tinv;
-  // Column chunks so that the scratch holds r x chunk; with more than one chunk they
-  // are multiples of 128 (the mask granularity), else the masks are not used.
-  const int64_t cap = w.tmp ? (int64_t)(w.tmp_bytes / sizeof(T)) / r : 0;
-  if (!linv || cap < 1) return KAD_ERR_ALLOC;
-  int chunk = (int)std::min<int64_t>(cap, ncols);
-  if (chunk < ncols && chunk >= 128) chunk = chunk / 128 * 128;
-  if (chunk < ncols && chunk % 128 != 0) cmask = nullptr;
-  int rc = trtri_rec<T>(L, lda, r, linv, r, w);
+  const int h = std::max(TRSM_ROWS, (r / 2) / TRSM_ROWS * TRSM_ROWS);
+  int rc = trsm_left_unit_lower<T>(L, lda, h, A12, ld12, ncols, w, gemm_prec, cmask, nbat, sL, sB, zr);
   if (rc) return rc;
-  for (int c = 0; c < ncols; c += chunk) {
-    const int nc = std::min(chunk, ncols - c);
-    T* tmp = (T*)w.tmp;
-    rc = gemm_launch_masked(gemm_prec == BF16 ? F32 : gemm_prec, GOP_SET, r, nc, r, linv, r, A12 + (int64_t)c * ld12,
-                            ld12, tmp, r, nullptr, cmask ? cmask + c / 128 : nullptr, w.stream);
-    if (rc) return rc;
-    dim3 g((unsigned)cdiv(r, 256), nc);
-    copy2d_kernel<T><<<g, 256, 0, w.stream>>>(tmp, r, A12 + (int64_t)c * ld12, ld12, r, nc);
-    KAD_HIP_CHECK(hipGetLastError());
+  const int gp = gemm_prec == BF16 ? F32 : gemm_prec;
+  rc = nbat > 1
+           ? batched_sub(gp, r - h, ncols, h, L + h, lda, sL, A12, ld12, sB, A12 + h, ld12, sB, nbat, zr, w.stream)
+           : gemm_launch_masked(gp, GOP_SUB, r - h, ncols, h, L + h, lda, A12, ld12, A12 + h, ld12, nullptr, cmask,
+                                w.stream);
+  if (rc) return rc;
+  ZeroRhs z2;
+  if (zr) {
+    z2 = *zr;
+    z2.row0 += h;
   }
-  return KAD_OK;
-}
-
-// U X = B in place for a non-unit upper U of order 32 and B of 32 rows: the leaf of
-// trsm_left_upper.  The rows are taken in reverse (U'(i, k) = U(31 - i, 31 - k) is
-// lower), so the lane's register window works as in trsm_leaf_kernel; each step
-// divides by the diagonal, then updates, as LAPACK's xTRSM ('L', 'U', 'N', 'N').
-template <typename T>
-__global__ __launch_bounds__(64, 4) void trsm_leaf_upper_kernel(const T* __restrict__ U, int64_t ldu,
-                                                             T* __restrict__ B, int64_t ldb, int ncols, int64_t sU,
-                                                             int64_t sB, const int* __restrict__ zcols) {
-  constexpr int R = TRSM_FUSED;
-  __builtin_amdgcn_s_setprio(2);
-  if (zcols && (int)blockIdx.x * 64 >= zcols[blockIdx.y]) return;  // only zero columns
-  U += (int64_t)blockIdx.y * sU;  // system blockIdx.y of a batch
-  B += (int64_t)blockIdx.y * sB;
-  __shared__ T Us[R * R + R];  // Us[i + R k] = U(R-1-i, R-1-k); R entries of padding read past the end
-  for (int e = threadIdx.x; e < R * R; e += 64) {
-    const int i = e % R, k = e / R;
-    Us[e] = U[(int64_t)(R - 1 - i) + (int64_t)(R - 1 - k) * ldu];
-  }
-  if (threadIdx.x < R) Us[R * R + threadIdx.x] = T(0);
-  const int c0 = blockIdx.x * 64;
-  const int c = c0 + threadIdx.x;
-  const bool act = c < ncols;
-  T* b = B + (int64_t)(act ? c : c0) * ldb;
-  T y[R];
-#pragma unroll
-  for (int i = 0; i < R; ++i) y[i] = act ? b[R - 1 - i] : T(0);
-  __syncthreads();
-#pragma unroll 1
-  for (int k = 0; k < R; ++k) {
-    const T* uk = Us + k + R * k;  // uk[i] = U'(k + i, k)
-    const T xk = y[0] / uk[0];
-    if (act) b[R - 1 - k] = xk;
-#pragma unroll
-    for (int i = 1; i < R; ++i) y[i - 1] = y[i] - uk[i] * xk;
-  }
+  return trsm_left_unit_lower<T>(L + h + (int64_t)h * lda, lda, r - h, A12 + h, ld12, ncols, w, gemm_prec, cmask, nbat,
+                                 sL, sB, zr ? &z2 : nullptr);
 }
 
 // B <- U^{-1} B with U non-unit upper (r x r, r a multiple of 32): X2 = U22^{-1} B2,
-// B1 -= U12 X2, X1 = U11^{-1} B1, recursively down to 32-row leaves.  nbat systems at
-// U + z sU, B + z sB; zcols (device, nbat entries, may be NULL): B_z is zero past
+// B1 -= U12 X2, X1 = U11^{-1} B1, recursively down to blocks of one launch.  nbat systems
+// at U + z sU, B + z sB; zcols (device, nbat entries, may be NULL): B_z is zero past
 // column zcols[z], and those columns are skipped.
 template <typename T>
 int trsm_left_upper(const T* U, int64_t ldu, int r, T* B, int64_t ldb, int ncols, LuWork& w, int gemm_prec, int nbat,
                     int64_t sU, int64_t sB, const int* zcols = nullptr) {
   if (ncols <= 0 || r <= 0) return KAD_OK;
-  if (r % TRSM_FUSED != 0) return arg_error("trsm_left_upper: order not a multiple of 32");
-  if (r == TRSM_FUSED) {
-    trsm_leaf_upper_kernel<T><<<dim3((unsigned)cdiv(ncols, 64), nbat), 64, 0, w.stream>>>(U, ldu, B, ldb, ncols, sU,
-                                                                                        sB, zcols);
+  if (r % TRB != 0) return arg_error("trsm_left_upper: order not a multiple of 32");
+  ZeroRhs zc;
+  zc.cols = zcols;
+  if (r <= TRSM_ROWS) {
+    trsm_block_kernel<T, true><<<dim3((unsigned)cdiv(ncols, TRSM_COLS), nbat), 256, 0, w.stream>>>(
+        U, ldu, B, ldb, r, ncols, nullptr, sU, sB, zc);
     KAD_HIP_CHECK(hipGetLastError());
     return KAD_OK;
   }
-  const int h = std::max(32, (r / 2) / 32 * 32);
+  const int h = std::max(TRSM_ROWS, (r / 2) / TRSM_ROWS * TRSM_ROWS);
   int rc =
       trsm_left_upper<T>(U + h + (int64_t)h * ldu, ldu, r - h, B + h, ldb, ncols, w, gemm_prec, nbat, sU, sB, zcols);
   if (rc) return rc;
-  ZeroRhs zc;
-  zc.cols = zcols;
   rc = batched_sub(gemm_prec, h, ncols, r - h, U + (int64_t)h * ldu, ldu, sU, B + h, ldb, sB, B, ldb, sB, nbat,
                    zcols ? &zc : nullptr, w.stream);
   if (rc) return rc;
@@ -467,7 +438,7 @@ int trsm_left_upper(const T* U, int64_t ldu, int r, T* B, int64_t ldb, int ncols
 // zero above row zstart[z zng + g], which the unit-lower solve skips.
 int lu_solve_permuted_batched(const double* LU, int64_t lda, int n, int nbat, int64_t sA, double* B, int64_t ldb,
                               int64_t sB, int nrhs, LuWork& w, const int* zcols, const int* zstart, int zng) {
-  if (n % TRSM_FUSED != 0 || nbat < 1) return arg_error("lu_solve_permuted_batched: order or batch");
+  if (n % TRB != 0 || nbat < 1) return arg_error("lu_solve_permuted_batched: order or batch");
   if (zstart && !zcols) return arg_error("lu_solve_permuted_batched: row starts without column counts");
   ZeroRhs zr;
   zr.cols = zcols;
@@ -1300,7 +1271,7 @@ int panel_rec(T* A, int64_t lda, int n, int c0, int c1, int* ipiv, LuWork& w, in
     return fused ? ffp_launch<T>(A, lda, n, c0, c1, pk0, pk1, ipiv, w, bt) : panel_base<T>(A, lda, n, c0, c1, ipiv, w);
   }
   int h = wdt / 2;
-  h = (h + 15) / 16 * 16;
+  h = (h + PANEL_BASE - 1) / PANEL_BASE * PANEL_BASE;
   const int cm = c0 + h;
   int rc = panel_rec<T>(A, lda, n, c0, cm, ipiv, w, pk0, pk1, fused, bt);
   if (rc) return rc;
@@ -1396,10 +1367,9 @@ int apply_left_swaps(T* A, int64_t lda, int n, const int* ipiv, int nb, LuWork& 
 //     step, which runs beside the next panel instead of ahead of it.
 // Events (ping-pong by step parity so a new record never overtakes a pending
 // wait): ev_panel "panel p and its mask are done", ev_next "columns of the panel
-// after next are up to date".  The two streams work on disjoint columns, each with
-// its own triangular-inverse / GEMM scratch.  The L21 row-tile masks rotate over
-// three buffers: part B of step p still reads panel p's mask while the panel stream
-// writes panel p+2's.
+// after next are up to date".  The two streams work on disjoint columns, and the L21
+// row-tile masks rotate over three buffers: part B of step p still reads panel p's mask
+// while the panel stream writes panel p+2's.
 //
 // A batch (bt.nbat > 1) factors bt.nbat matrices of order n together: every launch
 // covers all of them, so the panel chain is that of one matrix.  The matrices are
@@ -1407,10 +1377,10 @@ int apply_left_swaps(T* A, int64_t lda, int n, const int* ipiv, int nb, LuWork& 
 template <typename T>
 int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w, const LuBatch& bt) {
   // both streams' scratch must exist before anything is launched
-  if (!w.stream2 || !w.tinv || !w.tinv_m || !w.tmp || !w.tmp_m || w.tmp_m_bytes < w.tmp_bytes || !w.tmp2 ||
+  if (!w.stream2 || !w.tmp || !w.tmp2 ||
       !w.mask_r || !w.mask_r2 || !w.mask_r3 || !w.ext)
     return KAD_ERR_ALLOC;
-  LuWork wp = w;  // panel stream: tinv, tmp, tmp2 and the panel reductions
+  LuWork wp = w;  // panel stream: tmp, tmp2 and the panel reductions
   wp.stream = w.stream2;
   // the persistent panel's launch sequence advances in wp; it outlives this call on
   // every return path (reused flags would let stale exchange slots look current)
@@ -1419,10 +1389,6 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
     const LuWork& from;
     ~SeqBack() { to.ffp_seq = from.ffp_seq; }
   } seq_back{w, wp};
-  LuWork wm = w;  // main stream: its own triangular inverse and GEMM scratch
-  wm.tinv = w.tinv_m;
-  wm.tmp = w.tmp_m;
-  wm.tmp_bytes = w.tmp_m_bytes;
   int* mask_rows[3] = {w.mask_r, w.mask_r2, w.mask_r3};
   const int stride = (int)cdiv(n, 128) + 1;
   // Row extent of every 128-column tile of the input (one pass, one readback).
@@ -1484,8 +1450,8 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
     KAD_HIP_CHECK(hipStreamWaitEvent(w.stream, w.ev_panel[par], 0));
     if (k1 >= n) break;
     if (k2 < n && bat) {
-      if (piv && (rc = laswp<T>(A, lda, k2, k3, ipiv, k0, k1, wm, bt))) return rc;
-      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k2 * lda, lda, k3 - k2, wm, gemm_prec,
+      if (piv && (rc = laswp<T>(A, lda, k2, k3, ipiv, k0, k1, w, bt))) return rc;
+      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k2 * lda, lda, k3 - k2, w, gemm_prec,
                                    nullptr, bt.nbat, bt.sA, bt.sA);
       if (rc) return rc;
       rc = gemm_launch_batched(gemm_prec, GOP_SUB, n - k1, k3 - k2, k1 - k0, L21, lda, bt.sA,
@@ -1493,13 +1459,13 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
                                bt.nbat, w.stream);
       if (rc) return rc;
     } else if (k2 < n) {
-      rc = laswp<T>(A, lda, k2, k3, ipiv, k0, k1, wm);
+      rc = laswp<T>(A, lda, k2, k3, ipiv, k0, k1, w);
       if (rc) return rc;
       // structural zeros of A12 (column tiles; U12 = L11^{-1} A12 keeps them)
       col_tile_mask_kernel<T><<<(unsigned)cdiv(k3 - k2, 128), 1024, 0, w.stream>>>(A + k0 + (int64_t)k2 * lda, lda,
                                                                                  k1 - k0, k3 - k2, w.mask_c);
       KAD_HIP_CHECK(hipGetLastError());
-      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k2 * lda, lda, k3 - k2, wm, gemm_prec,
+      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k2 * lda, lda, k3 - k2, w, gemm_prec,
                                    w.mask_c);
       if (rc) return rc;
       rc = gemm_launch_masked(gemm_prec, GOP_SUB, n - k1, k3 - k2, k1 - k0, L21, lda, A + k0 + (int64_t)k2 * lda, lda,
@@ -1509,8 +1475,8 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
     KAD_HIP_CHECK(hipEventRecord(w.ev_next[par], w.stream));
     // ---- main stream, part B: columns [k3, n), beside the next panel
     if (k3 < n && bat) {
-      if (piv && (rc = laswp<T>(A, lda, k3, n, ipiv, k0, k1, wm, bt))) return rc;
-      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k3 * lda, lda, n - k3, wm, gemm_prec,
+      if (piv && (rc = laswp<T>(A, lda, k3, n, ipiv, k0, k1, w, bt))) return rc;
+      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k3 * lda, lda, n - k3, w, gemm_prec,
                                    nullptr, bt.nbat, bt.sA, bt.sA);
       if (rc) return rc;
       rc = gemm_launch_batched(gemm_prec, GOP_SUB, n - k1, n - k3, k1 - k0, L21, lda, bt.sA,
@@ -1518,12 +1484,12 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
                                bt.nbat, w.stream);
       if (rc) return rc;
     } else if (k3 < n) {
-      rc = laswp<T>(A, lda, k3, n, ipiv, k0, k1, wm);
+      rc = laswp<T>(A, lda, k3, n, ipiv, k0, k1, w);
       if (rc) return rc;
       col_tile_mask_kernel<T><<<(unsigned)cdiv(n - k3, 128), 1024, 0, w.stream>>>(A + k0 + (int64_t)k3 * lda, lda,
                                                                                 k1 - k0, n - k3, w.mask_c2);
       KAD_HIP_CHECK(hipGetLastError());
-      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k3 * lda, lda, n - k3, wm, gemm_prec,
+      rc = trsm_left_unit_lower<T>(L11, lda, k1 - k0, A + k0 + (int64_t)k3 * lda, lda, n - k3, w, gemm_prec,
                                    w.mask_c2);
       if (rc) return rc;
       // active tile pairs of the update, compacted on the grid (all XCDs busy)

@@ -136,13 +136,9 @@ int Ctx::lu_work(int n, int nb) {
     const char* sp = std::getenv("KAD_LU_SPIN");
     if (sp) lu.ffp_spin = std::max(0, std::atoi(sp));
   }
-  if ((rc = ensure(&lu.tinv, &cap_tinv, (size_t)nb * nb * 8))) return rc;
-  // GEMM scratch for L11^{-1} A12: nb x chunk (bounded at 64 MiB).
+  // row-gather scratch of the deferred left interchanges: nb x chunk (bounded at 64 MiB)
   const size_t want = std::min<size_t>((size_t)nb * (size_t)n * 8, (size_t)64 << 20);
   if ((rc = ensure(&lu.tmp, &lu.tmp_bytes, std::max<size_t>(want, (size_t)nb * nb * 8)))) return rc;
-  // the main stream's own copies (sized after tmp: the look-ahead runs both at once)
-  if ((rc = ensure(&lu.tinv_m, &cap_tinv_m, (size_t)nb * nb * 8))) return rc;
-  if ((rc = ensure(&lu.tmp_m, &lu.tmp_m_bytes, lu.tmp_bytes))) return rc;
   if ((rc = ensure(&lu.tmp2, &lu.tmp2_bytes, std::max<size_t>((size_t)nb * nb * 8, (size_t)n * 32 * 8)))) return rc;
   lu.stream = stream;
   return KAD_OK;
@@ -204,7 +200,7 @@ int Ctx::upload(const void* host, size_t bytes, void** dev) {
 Ctx::~Ctx() {
   for (auto& kv : plans) delete kv.second;
   for (void* p : owned) (void)hipFree(p);
-  void* bufs[] = {lu.red_val, lu.red_idx, lu.counter, lu.tinv,    lu.tmp,    lu.tmp2,  lu.map,  lu.mask_r,
+  void* bufs[] = {lu.red_val, lu.red_idx, lu.counter, lu.tmp,    lu.tmp2,  lu.map,  lu.mask_r,
                   lu.swap_map, lu.ext,     lu.ffp,     gemv_part, vwork,     krylov,   trs_tab, trs_flag, bsolve};
   for (void* b : bufs)
     if (b) (void)hipFree(b);
@@ -213,8 +209,6 @@ Ctx::~Ctx() {
     if (lu.ev_next[q]) (void)hipEventDestroy(lu.ev_next[q]);
   }
   if (lu.ev_start) (void)hipEventDestroy(lu.ev_start);
-  if (lu.tinv_m) (void)hipFree(lu.tinv_m);
-  if (lu.tmp_m) (void)hipFree(lu.tmp_m);
   if (lu.stream2) (void)hipStreamDestroy(lu.stream2);
   if (own_stream && stream) (void)hipStreamDestroy(stream);
 }
