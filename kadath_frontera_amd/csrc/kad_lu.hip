@@ -20,6 +20,7 @@
 // (structural zeros of a block-sparse Jacobian); the result is unchanged.
 #include "kad_common.hpp"
 #include "kad_ctx.hpp"
+#include <utility>
 #include <vector>
 #include <cmath>
 #include <algorithm>
@@ -655,27 +656,30 @@ __global__ void ff_scatter_kernel(T* __restrict__ A, int64_t lda, int n, int c0,
 
 // ---------------------------------------------------------------------------
 // Persistent base panel: one launch factors columns [c0, c1) (c1 - c0 <= W) of rows
-// [c0, n).  Workgroup g owns logical rows [c0 + g rpw, c0 + (g + 1) rpw) of the block,
-// one per thread, and keeps them in registers for the whole launch; interchanges move
-// row contents between owners.  Per column j:
-//   1. every workgroup publishes its pivot candidate (logical row and the candidate's
-//      row of the block); the owner of row j publishes row j;
-//   2. every workgroup reads all candidates with their rows in one round trip, each
-//      word flagged with its column (no grid barrier: a word is current when its flag
-//      is), reduces them itself -- LAPACK's choice, the first index of max |a| -- and
-//      swaps, scales and updates its rows with the per-column kernel's operations.
+// [c0, n).  Every thread keeps one row of the block in registers for the whole launch,
+// with its logical position: an interchange swaps the positions of two rows, no row
+// moves, and every row is written to its final position at the end.  Per column j:
+//   1. every wave takes its candidate (the largest |a| of its rows, the first position
+//      among ties); after one barrier every wave knows the workgroup's best, and the
+//      wave that owns it stages that row in LDS;
+//   2. with several workgroups, each publishes its candidate's position and the columns
+//      >= j of its row, reads all candidates in one round trip, each word flagged with
+//      its column (no grid barrier: a word is current when its flag is), and reduces them
+//      itself -- LAPACK's choice, the first index of max |a|;
+//   3. positions, multipliers and the rank-1 update, with the per-column kernel's
+//      operations; the next column's candidates come out of the update.
 // At the end the interchanges are applied to the panel's other columns [k0, c0) and
 // [c1, k1) (exact: those columns are not read in between).
-// The exchange's cost grows with the number of workgroups, so each one holds 256 rows,
-// and it fits beside a GEMM workgroup on one CU (the trailing update runs
-// concurrently): 144 VGPRs (FP64) and 19 KB of LDS, 4 waves.
+// Bound by latency: the chain of its columns is the factorisation's critical path.
+// 3.6 us per column with several workgroups, 1.8 with one (5.1 before, when every row moved
+// with its interchange, row j was published beside the candidates and every wave read the
+// pivot row by LDS broadcasts).
 // The grid must be resident at once: the host launches at most one workgroup per
 // CU, and nothing else on the device waits on this kernel.  Every wait is bounded: a
 // workgroup that reaches the spin limit raises the abort flag (sync[2]), every waiter
 // leaves on it, and the host reports the failure.
 // ---------------------------------------------------------------------------
 constexpr int FFP_MAX_GRID = 64;
-constexpr int FFP_THREADS = 256;
 
 // Exchange slots.  Every 64-bit slot holds one 32-bit data word and, in its high half,
 // the flag of the column that wrote it (launch sequence x 32 + column).  Slots are
@@ -684,27 +688,14 @@ constexpr int FFP_THREADS = 256;
 // that column's word: each slot validates itself, no slot is ordered against another,
 // and no device-scope fence (a write-back and invalidate of the XCD's whole L2, the
 // concurrent GEMM's working set) or arrival counter is needed.  A column's slots are
-// one record per workgroup (its candidate's logical row, for FP64 a pad word that
-// keeps the values 8-byte aligned, then the W values of that row, one word each for
-// FP32 and two for FP64) and, after the G records, the W values of row j.  Every
-// record and row j carry all W values (those of columns past the panel's end are
-// never read).  A column's stride covers whole 256-slot strips, so every thread reads
-// NU slots unconditionally and keeps those below G records + row j.
+// one record per workgroup, packed: its candidate's position (and for FP64 a pad word
+// that keeps the values 8-byte aligned), then the row's values from the column on, one
+// word each for FP32 and two for FP64.
 template <typename T, int W>
 struct FfpSlots {
-  static constexpr int VW = (int)(sizeof(T) / 4);        // words per value
-  static constexpr int VOFF = VW;                        // first value word of a record
-  static constexpr int REC = VOFF + VW * W;              // one workgroup's record
-  static constexpr int USED = FFP_MAX_GRID * REC + VW * W;  // G <= FFP_MAX_GRID records, row j
-  static constexpr int NU = (USED + 255) / 256;          // slots per thread (256 threads)
-  static constexpr int COL = NU * 256;                   // one column's stride
-  // where logical slot e (strip e / 256, thread e % 256) lies: wave-major, so one
-  // thread's NU slots are 512 bytes apart (immediate offsets from one or two bases)
-  // while each wave's load of a strip stays 64 consecutive slots
-  static __device__ __forceinline__ int pos(int e) {
-    const int t = e & 255;
-    return (t >> 6) * (NU * 64) + (e >> 8) * 64 + (t & 63);
-  }
+  static constexpr int VW = (int)(sizeof(T) / 4);  // words per value (and of a record's head)
+  static constexpr int REC = VW * (1 + W);         // the first column's record, the longest
+  static constexpr int COL = FFP_MAX_GRID * REC;   // one column's stride
 };
 
 __device__ __forceinline__ void slot_store(unsigned long long* p, unsigned long long v) {
@@ -713,295 +704,276 @@ __device__ __forceinline__ void slot_store(unsigned long long* p, unsigned long 
 __device__ __forceinline__ unsigned long long slot_load(const unsigned long long* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
-template <typename T>
-__device__ __forceinline__ unsigned word_of(T v, int k) {
-  if constexpr (sizeof(T) == 8) {
-    const unsigned long long b = __builtin_bit_cast(unsigned long long, v);
-    return k ? (unsigned)(b >> 32) : (unsigned)b;
-  } else {
-    return __builtin_bit_cast(unsigned, v);
+
+// |v| as an unsigned key that orders as the value does (high and low words; FP32: one).
+__device__ __forceinline__ void abs_key(double v, unsigned& hi, unsigned& lo) {
+  const unsigned long long b = (unsigned long long)__double_as_longlong(v);
+  hi = (unsigned)(b >> 32) & 0x7fffffffu;
+  lo = (unsigned)b;
+}
+__device__ __forceinline__ void abs_key(float v, unsigned& hi, unsigned& lo) {
+  hi = __builtin_bit_cast(unsigned, v) & 0x7fffffffu;
+  lo = 0;
+}
+
+// Largest value over a wave (DPP row shifts, then the two row broadcasts; lane 63 holds it).
+__device__ __forceinline__ unsigned wave_umax(unsigned v) {
+  auto step = [&v](int o) { v = (unsigned)o > v ? (unsigned)o : v; };
+  step(__builtin_amdgcn_update_dpp(0, (int)v, 0x111, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, (int)v, 0x112, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, (int)v, 0x114, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, (int)v, 0x118, 0xF, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, (int)v, 0x142, 0xA, 0xF, false));
+  step(__builtin_amdgcn_update_dpp(0, (int)v, 0x143, 0xC, 0xF, false));
+  return (unsigned)__builtin_amdgcn_readlane((int)v, 63);
+}
+
+// The lane of the largest (hi, lo) among a wave's lanes with pos >= 0, the smallest pos
+// among equal ones; -1 when there is none.  Uniform.  One 32-bit reduction decides it
+// unless the high words tie.
+__device__ __forceinline__ int wave_best(unsigned hi, unsigned lo, int pos) {
+  const bool in = pos >= 0;
+  const unsigned m = wave_umax(in ? hi : 0u);
+  unsigned long long c = __ballot(in && hi == m);
+  if (__popcll(c) > 1) {
+    const bool tie = in && hi == m;
+    const unsigned ml = wave_umax(tie ? lo : 0u);
+    c = __ballot(tie && lo == ml);
+    if (__popcll(c) > 1) {
+      int best = -1, bp = 0;
+      for (unsigned long long q = c; q; q &= q - 1) {
+        const int l = __ffsll((long long)q) - 1;
+        const int pl = __builtin_amdgcn_readlane(pos, l);
+        if (best < 0 || pl < bp) {
+          best = l;
+          bp = pl;
+        }
+      }
+      return best;
+    }
   }
+  return c ? __ffsll((long long)c) - 1 : -1;
 }
 
-__device__ __forceinline__ void argmax_take(double& v, int& i, double ov, int oi) {
-  if (oi >= 0 && (i < 0 || ov > v || (ov == v && oi < i))) {
-    v = ov;
-    i = oi;
-  }
+// The value of lane N of every 16-lane row to all its lanes.  Every lane must be active.
+template <int N>
+__device__ __forceinline__ double lane16(double v) {
+  return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + N, 0xF, 0xF, true));
+}
+template <int N>
+__device__ __forceinline__ float lane16(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + N, 0xF, 0xF, true));
 }
 
-// One step of a wave-level argmax: combine with the lane that DPP control CTRL reads
-// (a permutation inside each 16-lane row, so every source lane is valid).
-template <int CTRL>
-__device__ __forceinline__ void argmax_dpp(double& v, int& i) {
-  const long long b = __double_as_longlong(v);
-  const int hi = (int)(b >> 32), lo = (int)b;
-  const int ohi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, 0xF, 0xF, false);
-  const int olo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, 0xF, 0xF, false);
-  const int oi = __builtin_amdgcn_update_dpp(i, i, CTRL, 0xF, 0xF, false);
-  argmax_take(v, i, __longlong_as_double(((long long)ohi << 32) | (unsigned)olo), oi);
+// f(integral_constant 0), f(1), ..., f(N - 1): a loop whose index is a constant expression.
+template <typename F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>()), ...);
+}
+template <int N, typename F>
+__device__ __forceinline__ void static_for(F&& f) {
+  static_for_impl(f, std::make_integer_sequence<int, N>());
 }
 
-// Max |a| with the smallest index among ties (invalid entries carry index -1) over
-// one wave; the result reaches every lane.  Quad swaps, then half-row and row mirrors
-// (every lane of a 16-lane row ends with the row's best), then the four rows' results
-// are read from lanes 0, 16, 32, 48.  The selection is a total order, so the result
-// does not depend on the reduction order.
-__device__ __forceinline__ void argmax_wave(double& v, int& i) {
-  argmax_dpp<0xB1>(v, i);   // quad_perm [1,0,3,2]
-  argmax_dpp<0x4E>(v, i);   // quad_perm [2,3,0,1]
-  argmax_dpp<0x141>(v, i);  // row_half_mirror
-  argmax_dpp<0x140>(v, i);  // row_mirror
-  const long long b = __double_as_longlong(v);
-  const int hi = (int)(b >> 32), lo = (int)b;
-  double wv = -1.0;
-  int wi = -1;
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int rhi = __builtin_amdgcn_readlane(hi, 16 * r), rlo = __builtin_amdgcn_readlane(lo, 16 * r);
-    argmax_take(wv, wi, __longlong_as_double(((long long)rhi << 32) | (unsigned)rlo),
-                __builtin_amdgcn_readlane(i, 16 * r));
-  }
-  v = wv;
-  i = wi;
-}
-
-// The same over the 256-thread block, through 4 entries of LDS (sv / si) and one
-// barrier.  Every thread of the block must call it, and the caller must pass another
-// barrier before the next call writes sv / si.
-__device__ __forceinline__ void argmax_256(double& v, int& i, double* sv, int* si) {
-  argmax_wave(v, i);
-  if ((threadIdx.x & 63) == 0) {
-    sv[threadIdx.x >> 6] = v;
-    si[threadIdx.x >> 6] = i;
-  }
-  __syncthreads();
-  v = -1.0;
-  i = -1;
-#pragma unroll
-  for (int q = 0; q < FFP_THREADS / 64; ++q) argmax_take(v, i, sv[q], si[q]);
-}
-
-template <typename T, int W>
-__global__ __launch_bounds__(FFP_THREADS) void ffp_kernel(T* __restrict__ A, int64_t lda, int n, int c0, int c1,
-                                                          int k0, int k1, int rpw,
-                                                          unsigned long long* __restrict__ xbuf, unsigned flag0,
-                                                          int* __restrict__ ipiv, int* __restrict__ info,
-                                                          int* __restrict__ sync, int spin_limit, int64_t sA, int sP,
-                                                          int64_t sX) {
+// TH threads, one row each.
+template <typename T, int W, int TH>
+__global__ __launch_bounds__(TH) void ffp_kernel(T* __restrict__ A, int64_t lda, int n, int c0, int c1, int k0, int k1,
+                                                 int rpw, unsigned long long* __restrict__ xbuf, unsigned flag0,
+                                                 int* __restrict__ ipiv, int* __restrict__ info,
+                                                 int* __restrict__ sync, int spin_limit, int64_t sA, int sP,
+                                                 int64_t sX) {
   static_assert(FFP_MAX_GRID <= 64, "one candidate per lane of a wave");
-  static_assert(FFP_THREADS == 256, "256-slot strips");
-  static_assert((W & (W - 1)) == 0, "rotation mask");
+  constexpr int R4 = 4;  // columns between two rotations of the row registers
+  static_assert(W % R4 == 0, "rotation");
   using S = FfpSlots<T, W>;
-  constexpr int NU = S::NU;
+  constexpr int VW = S::VW, NW = TH / 64;
   // issue priority over the GEMM waves that share the SIMDs: every column waits for
   // the slowest workgroup, and the GEMM's MFMA chains leave issue slots to spare
   __builtin_amdgcn_s_setprio(3);
-  // this column's slots, data words only: G records, then row j
-  __shared__ __align__(16) unsigned xim[S::COL];
-  __shared__ double sv[FFP_THREADS / 64];
-  __shared__ int si[FFP_THREADS / 64];
+  __shared__ __align__(16) unsigned xim[TH == 1024 ? 4 : S::COL];  // this column's records, data words only
+  __shared__ __align__(16) T stage[W];         // the workgroup's candidate row
+  __shared__ unsigned wk[2][NW][4];            // the waves' candidates: key and position, by column parity
   __shared__ int s_piv[W];
   __shared__ int s_rows[2 * W];
   __shared__ int s_src[2 * W];
-  __shared__ int s_nrows;
-  __shared__ __align__(16) T stage[2][W];  // the candidate row and row j, for their waves
   // matrix blockIdx.y of a batch: its own rows, interchanges, exchange slots and info
   // word; the workgroups of one matrix (blockIdx.x) exchange only among themselves
   A += (int64_t)blockIdx.y * sA;
   ipiv += (int64_t)blockIdx.y * sP;
   xbuf += (int64_t)blockIdx.y * sX;
   info += blockIdx.y;
-  const int G = gridDim.x, g = blockIdx.x, tid = threadIdx.x;
-  const T* const jrow = reinterpret_cast<const T*>(xim + G * S::REC);
+  const int G = TH == 1024 ? 1 : (int)gridDim.x, g = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid & 63, wave = tid >> 6;
   const int r0 = c0 + g * rpw;
   const int nr = max(0, min(rpw, n - r0));
   const int w = c1 - c0;
-  // this thread's row of the block, in registers for the whole launch (one row per
-  // thread: the host launches at most FFP_THREADS rows per workgroup); columns past
-  // the panel's end hold zeros
-  // (rotated by one position per column: at column jj, row[q] holds column
-  // (q + jj) mod W, so the active column is row[0] and every index into the array is
-  // a compile-time constant)
-  const int r = tid;
-  const bool own = r < nr;
+  const bool own = tid < nr;
+  int pos = own ? r0 + tid : -1;  // this row's logical position; rows above the current column are done
+  // the row's columns; columns past the panel's end hold zeros (rotated by R4 positions
+  // every R4 columns: after jj columns, row[q] holds column (q + jj / R4 R4) mod W, so
+  // every index into the array is a compile-time constant)
   T row[W];
 #pragma unroll
-  for (int c = 0; c < W; ++c) row[c] = own && c < w ? A[(int64_t)(r0 + r) + (int64_t)(c0 + c) * lda] : T(0);
-  // local candidate of the first column; later columns' come out of the update
-  double v = own ? fabs((double)row[0]) : -1.0;
-  int id = own ? r0 + r : -1;
+  for (int c = 0; c < W; ++c) row[c] = own && c < w ? A[(int64_t)(r0 + tid) + (int64_t)(c0 + c) * lda] : T(0);
   bool live = true;  // uniform: false once a wait was abandoned
   int jfail = w;     // first column not factored (after an abandoned wait)
-  for (int jj = 0; jj < w; ++jj) {
-    const int j = c0 + jj;
-    // 1. the workgroup's candidate among its logical rows >= j, then publish its
-    //    record (logical row -1: none) and, from row j's owner, row j
-    argmax_256(v, id, sv, si);
-    const unsigned flag = flag0 + (unsigned)jj;
-    const unsigned long long tag = (unsigned long long)flag << 32;
-    unsigned long long* const col = xbuf + (size_t)jj * S::COL;
-    // the owning lane stages the row in LDS, then its wave stores the row's words
-    // (one slot per lane) without a workgroup barrier
-    const int lane = tid & 63;
-    const bool cand_wave = id >= 0 && (tid >> 6) == ((id - r0) >> 6);
-    const bool rowj_wave = j >= r0 && j < r0 + nr && (tid >> 6) == ((j - r0) >> 6);
-    if (cand_wave && tid == id - r0) {
-#pragma unroll
-      for (int q = 0; q < W; ++q) stage[0][(q + jj) & (W - 1)] = row[q];
-    }
-    if (rowj_wave && tid == j - r0) {
-#pragma unroll
-      for (int q = 0; q < W; ++q) stage[1][(q + jj) & (W - 1)] = row[q];
-    }
-    if (cand_wave || rowj_wave) {
-      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-      __builtin_amdgcn_wave_barrier();
-      __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    }
-    static_assert(S::VW * W <= 64, "one word per lane");
-    if (cand_wave) {
-      if (lane < S::VOFF) slot_store(col + S::pos(g * S::REC + lane), tag | (lane == 0 ? (unsigned)id : 0u));
-      if (lane < S::VW * W)
-        slot_store(col + S::pos(g * S::REC + S::VOFF + lane),
-                   tag | reinterpret_cast<const unsigned*>(stage[0])[lane]);
-    } else if (id < 0 && tid < S::REC) {
-      slot_store(col + S::pos(g * S::REC + tid), tag | (tid == 0 ? (unsigned)id : 0u));
-    }
-    if (rowj_wave && lane < S::VW * W)
-      slot_store(col + S::pos(G * S::REC + lane), tag | reinterpret_cast<const unsigned*>(stage[1])[lane]);
-    // 2. every record and row j, in one round trip: a thread loads its NU slots
-    //    (strip u, logical slot u * 256 + tid) at once, then reads again those below the used
-    //    slots until they carry this column's flag.  Bounded: at the spin limit the
-    //    workgroup raises the abort flag, and every waiter leaves on it; the host then
-    //    reports the failure.
-    const int nused = G * S::REC + S::VW * W;
-    const int nv = min(NU, max(0, (nused - tid + 255) >> 8));  // strips below nused
-    const unsigned valid = nv >= 32 ? ~0u : (1u << nv) - 1u;
-    const unsigned long long* const colt = col + (tid >> 6) * (NU * 64) + lane;  // strip u: + 64 u
-    // every word goes to the LDS image as it arrives; only the pending mask is carried
-    unsigned pend = 0;
-    {
-      unsigned long long xs[NU];
-#pragma unroll
-      for (int u = 0; u < NU; ++u) xs[u] = slot_load(colt + u * 64);
-#pragma unroll
-      for (int u = 0; u < NU; ++u) {
-        xim[u * 256 + tid] = (unsigned)xs[u];
-        pend |= (unsigned)((unsigned)(xs[u] >> 32) != flag) << u;
+  for (int j0 = 0; j0 < w && live; j0 += R4) {
+    static_for<R4>([&](auto sc) {
+      constexpr int s = decltype(sc)::value;
+      const int jj = j0 + s;
+      if (jj >= w || !live) return;
+      const int j = c0 + jj, par = s & 1;
+      // 1. the wave's candidate among its rows at positions >= j, then the workgroup's
+      unsigned hi, lo;
+      abs_key(row[s], hi, lo);
+      const int best = wave_best(hi, lo, pos >= j ? pos : -1);
+      if (lane == (best < 0 ? 0 : best)) {
+        wk[par][wave][0] = hi;
+        wk[par][wave][1] = lo;
+        wk[par][wave][2] = best < 0 ? ~0u : (unsigned)pos;
       }
-    }
-    pend &= valid;
-    int bad = 0;
-    for (int it = 0; pend; ++it) {
-      if (it >= spin_limit) {
-        __hip_atomic_store(&sync[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        bad = 1;
-        break;
+      __syncthreads();
+      unsigned khi = 0, klo = 0;
+      int kpos = -1;
+      if (lane < NW) {
+        khi = wk[par][lane][0];
+        klo = wk[par][lane][1];
+        kpos = (int)wk[par][lane][2];
       }
-      if ((it & 255) == 255 && __hip_atomic_load(&sync[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-        bad = 1;
-        break;
+      const int bw = wave_best(khi, klo, kpos);
+      int p = bw < 0 ? -1 : __builtin_amdgcn_readlane(kpos, bw);
+      if (wave == bw && lane == best) {
+#pragma unroll
+        for (int q = s; q < W; ++q) stage[q - s] = row[q];  // values from column jj on
       }
-      __builtin_amdgcn_s_sleep(1);
-      // again the groups of 4 strips that hold a pending slot
-#pragma unroll
-      for (int u0 = 0; u0 < NU; u0 += 4) {
-        if ((pend >> u0) & 15u) {
-          constexpr int GU = 4;
-          unsigned long long y[GU];
-#pragma unroll
-          for (int q = 0; q < GU; ++q)
-            if (u0 + q < NU) y[q] = slot_load(colt + (u0 + q) * 64);
-          unsigned nb = 0;
-#pragma unroll
-          for (int q = 0; q < GU; ++q)
-            if (u0 + q < NU) {
-              xim[(u0 + q) * 256 + tid] = (unsigned)y[q];
-              nb |= (unsigned)((unsigned)(y[q] >> 32) != flag) << q;
-            }
-          pend = (pend & ~(15u << u0)) | ((nb << u0) & valid);
+      const T* urow = stage;
+      if (G == 1) {
+        __syncthreads();
+      } else {
+        // 2. publish (position -1: no candidate), then read every record
+        const unsigned flag = flag0 + (unsigned)jj;
+        const unsigned long long tag = (unsigned long long)flag << 32;
+        unsigned long long* const col = xbuf + (size_t)jj * S::COL;
+        const int rec = VW * (1 + W - jj);
+        if (wave == (bw < 0 ? 0 : bw)) {  // the wave that staged the row
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          for (int e = lane; e < rec; e += 64) {
+            const unsigned word = e < VW ? (unsigned)p : reinterpret_cast<const unsigned*>(stage)[e - VW];
+            slot_store(col + g * rec + e, tag | word);
+          }
         }
+        const int nused = G * rec;
+        int bad = 0;
+        // groups of 4 strips of TH slots, loaded together and read again until every slot
+        // carries this column's flag.  Bounded: at the spin limit the workgroup raises
+        // the abort flag, and every waiter leaves on it; the host reports the failure.
+        for (int e0 = 0; e0 < nused && !bad; e0 += 4 * TH) {
+          for (int it = 0;; ++it) {
+            unsigned long long x[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) x[u] = e0 + u * TH + tid < nused ? slot_load(col + e0 + u * TH + tid) : tag;
+            bool pend = false;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              if (e0 + u * TH + tid < nused) xim[e0 + u * TH + tid] = (unsigned)x[u];
+              pend |= (unsigned)(x[u] >> 32) != flag;
+            }
+            if (!pend) break;
+            if (it >= spin_limit) {
+              __hip_atomic_store(&sync[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+              bad = 1;
+              break;
+            }
+            if ((it & 255) == 255 && __hip_atomic_load(&sync[2], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
+              bad = 1;
+              break;
+            }
+          }
+        }
+        if (__syncthreads_or(bad)) {  // uniform; the host sees sync[2] and reports the failure
+          live = false;
+          jfail = jj;
+          return;
+        }
+        // the pivot: every wave reduces the G <= 64 candidates itself
+        unsigned chi = 0, clo = 0;
+        int cpos = -1;
+        if (lane < G) {
+          cpos = (int)xim[lane * rec];
+          abs_key(reinterpret_cast<const T*>(xim + lane * rec + VW)[0], chi, clo);
+        }
+        const int bg = wave_best(chi, clo, cpos);
+        p = bg < 0 ? -1 : __builtin_amdgcn_readlane(cpos, bg);
+        urow = reinterpret_cast<const T*>(xim + (bg < 0 ? 0 : bg) * rec + VW);
       }
-    }
-    if (__syncthreads_or(bad)) {  // uniform; the host sees sync[2] and reports the failure
-      live = false;
-      jfail = jj;
-      break;
-    }
-    // 3. the pivot: LAPACK's choice, the first logical row of max |a| (a candidate's
-    //    |a| is its row's entry in this column); every wave reduces the G <= 64
-    //    candidates itself
-    v = -1.0;
-    id = -1;
-    if (lane < G && (int)xim[lane * S::REC] >= 0) {
-      v = fabs((double)reinterpret_cast<const T*>(xim + lane * S::REC + S::VOFF)[jj]);
-      id = (int)xim[lane * S::REC];
-    }
-    argmax_wave(v, id);
-    int p = id;
-    if (p < j || p >= n) {
-      // only reachable with corrupt candidates: keep every index in range and fail
-      p = j;
-      if (tid == 0) __hip_atomic_store(&sync[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    }
-    const T* urow = reinterpret_cast<const T*>(xim + ((p - c0) / rpw) * S::REC + S::VOFF);  // p's owner's
-    if (tid == 0) s_piv[jj] = p;
-    if (g == 0 && tid == 0) {
-      ipiv[j] = p;
-      if (v == 0.0 && *info == 0) *info = j + 1;
-    }
-    // 4. the interchange: row j's owner takes the pivot row, row p's owner row j
-    //    (registers of one thread each: no barrier)
-    if (p != j) {
-      if (j >= r0 && j < r0 + nr && tid == j - r0) {
-#pragma unroll
-        for (int q = 0; q < W; ++q) row[q] = urow[(q + jj) & (W - 1)];
-      } else if (p >= r0 && p < r0 + nr && tid == p - r0) {
-#pragma unroll
-        for (int q = 0; q < W; ++q) row[q] = jrow[(q + jj) & (W - 1)];
+      if (p < j || p >= n) {
+        // only reachable with corrupt candidates: keep every index in range and fail
+        p = j;
+        if (tid == 0) __hip_atomic_store(&sync[2], 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       }
-    }
-    // 5. rows below j: the multiplier (column jj: row[0]), the rank-1 update of
-    //    columns jj < c < W (row[q], q = c - jj: no wrap; columns past the panel's end
-    //    are never written back) with the pivot row, and the candidate of the next
-    //    column (row[1]); then every row rotates by one position
-    const bool below = own && r0 + r > j;
-    const T* const uj = urow + jj;  // uj[q]: the pivot row's column jj + q
-    const T piv = uj[0];
-    v = -1.0;
-    id = -1;
-    if (below) {
-      T l = row[0];
-      if (piv != T(0)) l = l / piv;
-      row[0] = l;
-#pragma unroll
-      for (int q = 1; q < W; ++q)
-        if (q < W - jj) row[q] = row[q] - l * uj[q];
-      if (jj + 1 < w) {
-        v = fabs((double)row[1]);
-        id = r0 + r;
+      // 3. the interchange: row p moves to position j, the row there to p; the pivot row
+      //    is then final
+      const T piv = urow[0];
+      if (tid == 0) s_piv[jj] = p;
+      if (g == 0 && tid == 0) {
+        ipiv[j] = p;
+        if (piv == T(0) && *info == 0) *info = j + 1;
       }
-    }
-    {
-      const T t = row[0];
+      if (pos == p) pos = j;
+      else if (pos == j) pos = p;
+      // rows below j: the multiplier (row[s]) and the rank-1 update of the columns after
+      // it (row[q]: column jj + q - s, no wrap below W - j0; columns past the panel's end
+      // are never written back).  The pivot row's values sit in the lanes of each 16-lane
+      // row, 16 in each of u0 and u1, and reach the multiply-adds by row broadcasts (as
+      // broadcast LDS reads by every wave they filled the LDS pipe).
+      const T u0 = urow[lane & 15], u1 = urow[16 + (lane & 15)];
+      const bool below = pos > j;
+      T l = row[s];
+      if (below) {
+        if (piv != T(0)) l = l / piv;
+        row[s] = l;
+      }
+      static_for<W / R4>([&](auto bc) {
+        constexpr int q0 = decltype(bc)::value * R4;
+        if (q0 >= W - j0) return;  // uniform
+        T ub[R4];
+        static_for<R4>([&](auto qc) {
+          constexpr int v = q0 + decltype(qc)::value - s;  // the value's place in the record
+          if constexpr (v > 0 && v < 16) ub[decltype(qc)::value] = lane16<v>(u0);
+          if constexpr (v >= 16) ub[decltype(qc)::value] = lane16<v - 16>(u1);
+        });
+        if (below) {
 #pragma unroll
-      for (int q = 0; q < W - 1; ++q) row[q] = row[q + 1];
-      row[W - 1] = t;
-    }
+          for (int q = 0; q < R4; ++q)
+            if (q0 + q > s) row[q0 + q] = row[q0 + q] - l * ub[q];
+        }
+      });
+    });
+    T t[R4];
+#pragma unroll
+    for (int q = 0; q < R4; ++q) t[q] = row[q];
+#pragma unroll
+    for (int q = 0; q < W - R4; ++q) row[q] = row[q + R4];
+#pragma unroll
+    for (int q = 0; q < R4; ++q) row[W - R4 + q] = t[q];
   }
   if (!live) {
     // the columns not factored get identity interchanges: later kernels index rows
     // with ipiv, which must stay within the matrix (the factors are reported invalid)
     if (g == 0)
-      for (int jj = jfail + tid; jj < w; jj += FFP_THREADS) ipiv[c0 + jj] = c0 + jj;
+      for (int jj = jfail + tid; jj < w; jj += TH) ipiv[c0 + jj] = c0 + jj;
     return;
   }
-  if (own) {  // after w columns, row[q] holds column (q + w) mod W
+  // rows to their final positions: every row of the block was read before the first
+  // column's exchange (one workgroup: its barrier) ended, so none is overwritten unread
+  const int turn = (w + R4 - 1) / R4 * R4;  // row[q] holds column (q + turn) mod W
+  if (own) {
 #pragma unroll
     for (int q = 0; q < W; ++q) {
-      const int c = (q + w) & (W - 1);
-      if (c < w) A[(int64_t)(r0 + r) + (int64_t)(c0 + c) * lda] = row[q];
+      const int c = (q + turn) & (W - 1);
+      if (c < w) A[(int64_t)pos + (int64_t)(c0 + c) * lda] = row[q];
     }
   }
   __syncthreads();  // s_piv of the last column
@@ -1019,24 +991,23 @@ __global__ __launch_bounds__(FFP_THREADS) void ffp_kernel(T* __restrict__ A, int
     s_rows[tid] = r;
     s_src[tid] = x;
   }
-  if (tid == 0) s_nrows = 2 * w;
   __syncthreads();
   // (column, affected row) pairs, columns split over the workgroups: every thread
   // gathers up to FFP_TAIL of them into registers, the workgroup synchronises, then
   // every thread scatters them -- one round trip per batch, and no row of a column is
   // written before all of that column's reads (a column stays in one workgroup)
   constexpr int FFP_TAIL = 16;
-  const int nrw = s_nrows, nleft = c0 - k0, nother = (c0 - k0) + (k1 - c1);
+  const int nrw = 2 * w, nleft = c0 - k0, nother = (c0 - k0) + (k1 - c1);
   const int cpg = (int)cdiv(nother, G);  // columns of this workgroup: [g cpg, (g + 1) cpg)
   const int qa = min(nother, g * cpg), qe = min(nother, qa + cpg);
   const int npairs = (qe - qa) * nrw;
-  const int step = ((FFP_TAIL * FFP_THREADS) / nrw) * nrw;  // whole columns per batch (nrw <= 2 W)
+  const int step = ((FFP_TAIL * TH) / nrw) * nrw;  // whole columns per batch (nrw <= 2 W)
   for (int b0 = 0; b0 < npairs; b0 += step) {
     const int bend = min(npairs, b0 + step);
     T val[FFP_TAIL];
 #pragma unroll
     for (int u = 0; u < FFP_TAIL; ++u) {
-      const int e = b0 + u * FFP_THREADS + tid;
+      const int e = b0 + u * TH + tid;
       if (e < bend) {
         const int q = qa + e / nrw, k = e - (e / nrw) * nrw;
         const int col = q < nleft ? k0 + q : c1 + (q - nleft);
@@ -1046,7 +1017,7 @@ __global__ __launch_bounds__(FFP_THREADS) void ffp_kernel(T* __restrict__ A, int
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < FFP_TAIL; ++u) {
-      const int e = b0 + u * FFP_THREADS + tid;
+      const int e = b0 + u * TH + tid;
       if (e < bend) {
         const int q = qa + e / nrw, k = e - (e / nrw) * nrw;
         const int col = q < nleft ? k0 + q : c1 + (q - nleft);
@@ -1063,30 +1034,39 @@ __global__ __launch_bounds__(FFP_THREADS) void ffp_kernel(T* __restrict__ A, int
 constexpr int64_t ffp_matrix_words() { return (int64_t)PANEL_BASE * FfpSlots<double, PANEL_BASE>::COL; }
 size_t ffp_bytes() { return (size_t)LU_MAX_BATCH * ffp_matrix_words() * sizeof(unsigned long long); }
 
-// Launch shape of the persistent base panel for m rows of element type T: grid and
-// rows per workgroup, or false when it does not fit (the per-column kernels run).
-template <typename T>
-bool ffp_shape(int m, int ncu, int& grid, int& rpw) {
-  // one row per thread, held in registers: a second row for a few threads would
-  // double the latency of every column step for the whole workgroup
-  grid = (int)cdiv(m, FFP_THREADS);
-  if (m < 1 || grid > std::min(ncu, FFP_MAX_GRID)) return false;
-  rpw = (int)cdiv(m, grid);
-  grid = (int)cdiv(m, rpw);
+// Launch shape of the persistent base panel for m rows of each of nbat matrices: threads
+// (= most rows) per workgroup, grid and rows per workgroup, or false when it does not
+// fit (the per-column kernels run).  Up to 1024 rows one workgroup needs no exchange.
+// A batch launches the workgroups of every matrix together; all of them must be
+// resident at once, so it holds at most one workgroup per CU in total.
+struct FfpShape {
+  int th = 0, grid = 0, rpw = 0;
+};
+inline bool ffp_shape(int m, int nbat, int ncu, FfpShape& s) {
+  if (m < 1) return false;
+  // one workgroup of 1024 rows against several of 256: n = 600 2.05 ms against 2.39, 1215
+  // 4.07 against 4.74; beyond that 256 rows per workgroup (n = 5000 20.4 ms, 20.9 with
+  // 512), 512 where 256 would need too many workgroups
+  for (int th : {1024, 256, 512}) {
+    s.th = th;
+    s.grid = (int)cdiv(m, th);
+    if (s.grid <= (th == 1024 ? 1 : FFP_MAX_GRID) && s.grid * nbat <= ncu) break;
+    s.grid = 0;
+  }
+  if (!s.grid) return false;
+  s.rpw = (int)cdiv(m, s.grid);
+  s.grid = (int)cdiv(m, s.rpw);
   return true;
 }
 
 // One persistent base panel: columns [c0, c1) of rows [c0, n), interchanges applied
 // across the panel's columns [k0, k1).
-// A batch launches the workgroups of every matrix together (grid y); all of them must
-// be resident at once, so a batch holds at most one workgroup per CU in total.
 template <typename T>
 int ffp_launch(T* A, int64_t lda, int n, int c0, int c1, int k0, int k1, int* ipiv, LuWork& w,
                const LuBatch& bt = LuBatch()) {
-  int grid, rpw;
-  if (!ffp_shape<T>(n - c0, w.ncu, grid, rpw) || rpw > FFP_THREADS || c1 - c0 > PANEL_BASE || c1 > n)
-    return arg_error("ffp_launch: panel shape");
-  if (bt.nbat < 1 || bt.nbat > LU_MAX_BATCH || grid * bt.nbat > w.ncu || (bt.nbat > 1 && !bt.info))
+  FfpShape s;
+  if (c1 - c0 > PANEL_BASE || c1 > n) return arg_error("ffp_launch: panel shape");
+  if (bt.nbat < 1 || bt.nbat > LU_MAX_BATCH || (bt.nbat > 1 && !bt.info) || !ffp_shape(n - c0, bt.nbat, w.ncu, s))
     return arg_error("ffp_launch: batch does not fit the CUs");
   // flags: PANEL_BASE per launch, never one the slots still hold (the buffer starts
   // zeroed and the sequence at 1; before the 32-bit flags wrap it is cleared again)
@@ -1095,9 +1075,14 @@ int ffp_launch(T* A, int64_t lda, int n, int c0, int c1, int k0, int k1, int* ip
     w.ffp_seq = 1;
   }
   const unsigned flag0 = w.ffp_seq * (unsigned)PANEL_BASE;
-  ffp_kernel<T, PANEL_BASE><<<dim3(grid, bt.nbat), FFP_THREADS, 0, w.stream>>>(
-      A, lda, n, c0, c1, k0, k1, rpw, (unsigned long long*)w.ffp, flag0, ipiv, bt.info ? bt.info : w.info, w.ffp_sync,
-      w.ffp_spin, bt.sA, bt.sP, ffp_matrix_words());
+  auto run = [&](auto kernel) {
+    kernel<<<dim3(s.grid, bt.nbat), s.th, 0, w.stream>>>(A, lda, n, c0, c1, k0, k1, s.rpw, (unsigned long long*)w.ffp,
+                                                         flag0, ipiv, bt.info ? bt.info : w.info, w.ffp_sync,
+                                                         w.ffp_spin, bt.sA, bt.sP, ffp_matrix_words());
+  };
+  if (s.th == 1024) run(ffp_kernel<T, PANEL_BASE, 1024>);
+  else if (s.th == 256) run(ffp_kernel<T, PANEL_BASE, 256>);
+  else run(ffp_kernel<T, PANEL_BASE, 512>);
   KAD_HIP_CHECK(hipGetLastError());
   return KAD_OK;
 }
@@ -1420,8 +1405,8 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
     for (int t = k0 / 128; t <= (k1 - 1) / 128; ++t) R = std::max(R, ext[t] + 1);
     R = std::min(R, n);
     r_prev = R;
-    int fg, frpw;
-    const bool fused = bt.nopiv || (wp.ffp && !wp.ffp_off && ffp_shape<T>(R - k0, wp.ncu, fg, frpw));
+    FfpShape fs;
+    const bool fused = bt.nopiv || (wp.ffp && !wp.ffp_off && ffp_shape(R - k0, bt.nbat, wp.ncu, fs));
     int rc = panel_rec<T>(A, lda, R, k0, k1, ipiv, wp, k0, k1, fused, bt);
     if (rc) return rc;
     if (k1 < n && mask) {
