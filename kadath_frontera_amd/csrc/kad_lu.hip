@@ -20,7 +20,7 @@
 // (structural zeros of a block-sparse Jacobian); the result is unchanged.
 #include "kad_common.hpp"
 #include "kad_ctx.hpp"
-#include <utility>
+#include "kad_lanes.hpp"
 #include <vector>
 #include <cmath>
 #include <algorithm>
@@ -123,15 +123,15 @@ __global__ __launch_bounds__(1024) void row_tile_mask_kernel(const T* __restrict
   any = __syncthreads_or(any);
   if (threadIdx.x == 0) mask[blockIdx.x] = any;
 }
-// Last nonzero row of each 128-column tile: out[tile] = max over the 2048-row chunks
+// Last nonzero row of each 128-column tile: out[tile] = max over the 256-row chunks
 // (workgroup (tile, chunk); out starts at -1).  A chunk is read from its end, 32 rows at
 // a time, until a nonzero is met, so a dense matrix costs one step of it (a full scan
 // took 180 us at n = 1215, 470 at 8191).
 template <typename T>
 __global__ __launch_bounds__(256) void col_extent_kernel(const T* __restrict__ A, int64_t lda, int n,
                                                          int* __restrict__ out) {
-  const int c0 = blockIdx.x * 128, r0 = blockIdx.y * 2048;
-  const int ce = min(c0 + 128, n), re = min(r0 + 2048, n);
+  const int c0 = blockIdx.x * 128, r0 = blockIdx.y * 256;
+  const int ce = min(c0 + 128, n), re = min(r0 + 256, n);
   const int tr = threadIdx.x & 31, tc = threadIdx.x >> 5;  // row within a step, one of 8 column groups
   for (int rb = r0 + (re - r0 - 1) / 32 * 32; rb >= r0; rb -= 32) {
     const int r = rb + tr;
@@ -730,49 +730,19 @@ __device__ __forceinline__ unsigned wave_umax(unsigned v) {
 
 // The lane of the largest (hi, lo) among a wave's lanes with pos >= 0, the smallest pos
 // among equal ones; -1 when there is none.  Uniform.  One 32-bit reduction decides it
-// unless the high words tie.
+// unless the high words tie (a column of zeros, the structural zeros of a Jacobian).
 __device__ __forceinline__ int wave_best(unsigned hi, unsigned lo, int pos) {
   const bool in = pos >= 0;
   const unsigned m = wave_umax(in ? hi : 0u);
   unsigned long long c = __ballot(in && hi == m);
   if (__popcll(c) > 1) {
-    const bool tie = in && hi == m;
+    bool tie = in && hi == m;
     const unsigned ml = wave_umax(tie ? lo : 0u);
-    c = __ballot(tie && lo == ml);
-    if (__popcll(c) > 1) {
-      int best = -1, bp = 0;
-      for (unsigned long long q = c; q; q &= q - 1) {
-        const int l = __ffsll((long long)q) - 1;
-        const int pl = __builtin_amdgcn_readlane(pos, l);
-        if (best < 0 || pl < bp) {
-          best = l;
-          bp = pl;
-        }
-      }
-      return best;
-    }
+    tie = tie && lo == ml;
+    const unsigned mp = wave_umax(tie ? ~(unsigned)pos : 0u);
+    c = __ballot(tie && ~(unsigned)pos == mp);
   }
   return c ? __ffsll((long long)c) - 1 : -1;
-}
-
-// The value of lane N of every 16-lane row to all its lanes.  Every lane must be active.
-template <int N>
-__device__ __forceinline__ double lane16(double v) {
-  return __longlong_as_double(__builtin_amdgcn_update_dpp(0LL, __double_as_longlong(v), 0x150 + N, 0xF, 0xF, true));
-}
-template <int N>
-__device__ __forceinline__ float lane16(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x150 + N, 0xF, 0xF, true));
-}
-
-// f(integral_constant 0), f(1), ..., f(N - 1): a loop whose index is a constant expression.
-template <typename F, int... I>
-__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>) {
-  (f(std::integral_constant<int, I>()), ...);
-}
-template <int N, typename F>
-__device__ __forceinline__ void static_for(F&& f) {
-  static_for_impl(f, std::make_integer_sequence<int, N>());
 }
 
 // TH threads, one row each.
@@ -1389,7 +1359,7 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
     if (!bt.growth) return arg_error("getrf: static pivoting needs growth words");
     KAD_HIP_CHECK(hipMemsetAsync(bt.growth, 0, bt.nbat * sizeof(unsigned long long), w.stream));
   }
-  const int ntc = (int)cdiv(n, 128), nrc = (int)cdiv(n, 2048);
+  const int ntc = (int)cdiv(n, 128), nrc = (int)cdiv(n, 256);
   std::vector<int> ext(ntc, bat ? n - 1 : -1);
   if (!bat) {
     KAD_HIP_CHECK(hipMemsetAsync(w.ext, 0xff, ntc * sizeof(int), w.stream));  // -1
