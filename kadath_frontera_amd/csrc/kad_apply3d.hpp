@@ -1,262 +1,254 @@
 // Device body of a chain of 1-D passes over one 3-D domain array staged in LDS: used by
 // the batched transform kernel (kad_spectral.hip) and by the grouped execution of the
 // device programs (kad_group.hip), so both give the same bits.
+//
+// One thread per line and part of its outputs: the line goes to registers once, the
+// outputs are a small dense matrix times the line.  Bound by the vector unit once warm
+// (about 8 cycles per matrix entry and wave).  The matrix row of an output sits in the
+// lanes of each 16-lane row of the wave (one LDS read per output) and its entries reach the
+// multiply-adds by DPP row broadcasts; entries past 16 are broadcast LDS reads.  With the
+// entries read by scalar loads every output waited for the scalar cache: 4096 transforms
+// there and back took 247 us at 17x13x12 and 390 at 18x13x12, now 217 and 226.  Chains of
+// small arrays take a thread per output.
 #pragma once
+#include "kad_lanes.hpp"
 #include "kad_spectral.hpp"
 
 namespace kad {
 
-// One pass along any axis with NIN (12..17) input points per line, one line per
-// thread: the thread reads its line into registers once and produces all of the
-// line's outputs; the line's matrix is read with wave-uniform (scalar) loads from
-// the read-only matrix pool in global memory, so each FMA takes one operand from
-// SGPRs and one from VGPRs and LDS carries only the line in and the outputs out.
-// Waves whose lines use different matrices (e.g. theta lines of even and odd phi
-// index) are served one matrix at a time (a waterfall over the distinct offsets).
-// x and y may be the same buffer when the pass keeps the line length: the thread
-// reads its whole line before writing the line's outputs, and lines are disjoint.
+// The outputs [o0, o1) of one line per lane (ni <= NIN points from x + q sin to y + o sout;
+// the entries past ni count as zeros).  Waves whose lines use different matrices are served
+// one matrix at a time.  one (the output may lie over the input): every thread passes the
+// barrier between its reads and its writes.
 template <int NIN>
-__device__ __forceinline__ void pass_lines(const double* x, double* y,
-                                           const double* __restrict__ pool, const int* __restrict__ lm, int ax,
-                                           const int dims[3], const int od[3], int nout_ax) {
-  const int nl0 = ax == 0 ? od[1] : od[0];
-  const int nlines = ax == 0 ? od[1] * od[2] : (ax == 1 ? od[0] * od[2] : od[0] * od[1]);
-  const int sin_ = ax == 0 ? 1 : (ax == 1 ? dims[0] : dims[0] * dims[1]);
-  const int sout = ax == 0 ? 1 : (ax == 1 ? od[0] : od[0] * od[1]);
-  for (int li = threadIdx.x; li - (int)(threadIdx.x & 63) < nlines; li += blockDim.x) {
-    // every lane of a wave runs the same iterations (the vote below needs them all)
-    const bool act = li < nlines;
-    const int a = act ? li % nl0 : 0, bq = act ? li / nl0 : 0;
-    int xb, yb, lmi;
-    if (ax == 0) {         // line (j, k) = (a, bq)
-      xb = dims[0] * (a + dims[1] * bq);
-      yb = od[0] * (a + od[1] * bq);
-      lmi = a + od[1] * bq;
-    } else if (ax == 1) {  // line (i, k) = (a, bq)
-      xb = a + dims[0] * dims[1] * bq;
-      yb = a + od[0] * od[1] * bq;
-      lmi = bq;
-    } else {               // line (i, j) = (a, bq)
-      xb = a + dims[0] * bq;
-      yb = a + od[0] * bq;
-      lmi = 0;
+__device__ __forceinline__ void pass_lines(const double* x, double* y, const double* mats, const LineEnt en, bool act,
+                                           int ni, int sin, int sout, int o0, int o1, bool one) {
+  double xv[NIN];
+#pragma unroll
+  for (int q = 0; q < NIN; ++q) xv[q] = q < ni ? x[en.xb + q * sin] : 0.0;  // (lanes without a line read line 0)
+  if (one) __syncthreads();
+  const int l16 = threadIdx.x & 15;
+  bool todo = act;
+  while (true) {
+    const unsigned long long pend = __ballot(todo);
+    if (pend == 0) break;
+    const int off = __builtin_amdgcn_readlane(en.off, __ffsll((long long)pend) - 1);
+    const bool mine = todo && en.off == off;
+    todo = todo && !mine;
+    double* yl = y + en.yb + o0 * sout;
+    if (off < 0) {  // a line without a matrix is zero
+      if (mine)
+        for (int o = o0; o < o1; ++o, yl += sout) *yl = 0.0;
+      continue;
     }
-    const int off = act ? lm[lmi] : -1;
-    double xv[NIN];
+    const double* M = mats + off + o0 * ni;
+    double m = l16 < ni ? M[l16] : 0.0;
+#pragma unroll 1
+    for (int o = o0; o < o1; ++o, yl += sout) {
+      const double mc = m;
+      double tail[NIN > 16 ? NIN - 16 : 1];
 #pragma unroll
-    for (int q = 0; q < NIN; ++q) xv[q] = act ? x[xb + q * sin_] : 0.0;
-    // waterfall over the distinct matrices of the wave, in uniform control flow (so
-    // the matrix address is uniform and its loads are scalar): every lane computes
-    // with the chosen matrix, the lanes whose line uses it store
-    bool todo = act;
-    while (true) {
-      const unsigned long long pend = __ballot(todo);
-      if (pend == 0) break;
-      const int off0 = __builtin_amdgcn_readlane(off, __ffsll((long long)pend) - 1);
-      const bool mine = todo && off == off0;
-      todo = todo && !mine;
-      if (off0 < 0) {
-        for (int o = 0; o < nout_ax; ++o)
-          if (mine) y[yb + o * sout] = 0.0;
-        continue;
-      }
-      // the pool is read-only for the whole kernel: read it through the constant
-      // address space, so the uniform address gives scalar loads
-      typedef const double __attribute__((address_space(4)))* cdptr;
-      const cdptr M = (cdptr)(pool + off0);
-#pragma unroll 2
-      for (int o = 0; o < nout_ax; ++o) {
-        double s0 = 0.0, s1 = 0.0;
-#pragma unroll
-        for (int q = 0; q + 1 < NIN; q += 2) {
-          s0 += M[o * NIN + q] * xv[q];
-          s1 += M[o * NIN + q + 1] * xv[q + 1];
-        }
-        if (NIN % 2) s0 += M[o * NIN + NIN - 1] * xv[NIN - 1];
-        if (mine) y[yb + o * sout] = s0 + s1;
-      }
+      for (int q = 16; q < NIN; ++q) tail[q - 16] = q < ni ? M[q] : 0.0;
+      M += ni;
+      if (o + 1 < o1) m = l16 < ni ? M[l16] : 0.0;  // the next output's row, ahead of its use
+      double s0 = 0.0, s1 = 0.0;
+      static_for<NIN>([&](auto qc) {
+        constexpr int q = decltype(qc)::value;
+        double c;
+        if constexpr (q < 16) c = lane16<q>(mc);
+        else c = tail[q - 16];
+        if constexpr (q % 2 == 0) s0 += c * xv[q];
+        else s1 += c * xv[q];
+        if constexpr (q % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // four broadcasts in registers, not all
+      });
+      double r = s0 + s1;
+      asm volatile("" : "+v"(r));  // computed by every lane: kept out of the store's branch, with its broadcasts
+      if (mine) *yl = r;
     }
   }
 }
 
+// One output: a matrix row times a line, both in LDS.
+__device__ __forceinline__ double line_dot(const double* M, const double* x, int ni, int sin) {
+  double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
+  int q = 0;
+  for (; q + 4 <= ni; q += 4) {
+    s0 += M[q] * x[q * sin];
+    s1 += M[q + 1] * x[(q + 1) * sin];
+    s2 += M[q + 2] * x[(q + 2) * sin];
+    s3 += M[q + 3] * x[(q + 3) * sin];
+  }
+  for (; q < ni; ++q) s0 += M[q] * x[q * sin];
+  return (s0 + s1) + (s2 + s3);
+}
+
 // One workgroup (256 threads) takes the array src (batch element b of the chain post) to
-// dst.  lds: two ping-pong buffers (one when inplace), then the plan's matrix pool (when
-// stage_pool) and per-line matrix tables (a few KB, staged once), so the contraction of
-// every output element reads only LDS.  PP: Passes, as a kernel argument or in the
-// constant address space (read with scalar loads either way).
+// dst.  lds: one buffer (two when a pass has more lines than threads), then the matrix
+// pool.  PP: LinePlan, as a kernel argument or in the constant address space (read with
+// scalar loads either way).
 template <typename PP>
-__device__ __forceinline__ void apply3d_body(const double* __restrict__ src, double* __restrict__ dst, int d0, int d1,
-                                             int d2, const PP& P, const double* __restrict__ pool, int accumulate,
-                                             double scale, int stage_pool, int inplace, const PostOp& post, int64_t b,
-                                             double* lds) {
-  // the two ping-pong buffers are selected by value (not through an array of
-  // pointers), so every access stays an LDS access and the matrix-pool loads can be
-  // proven unclobbered (scalar loads); inplace: every pass keeps its line length and
-  // runs line by line, so one buffer serves as input and output (half the LDS)
+__device__ __forceinline__ void apply3d_body(const double* __restrict__ src, double* __restrict__ dst, const PP& P,
+                                             const PostOp& post, int64_t b, double* lds) {
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int nin = P.size_in, npass = P.npass, npool = P.pool_size, maxsize = P.maxsize;
+  const bool single = P.single != 0;
+  const double* const pool = P.pool;
   double* const buf0 = lds;
-  double* const buf1 = inplace ? lds : lds + P.maxsize;
-  double* mats = lds + (inplace ? 1 : 2) * P.maxsize;
-  int* ltab = reinterpret_cast<int*>(mats + (stage_pool ? P.pool_size : 0));
-  const int nin = d0 * d1 * d2;
-  // 8 loads in flight per thread (one load per iteration would wait out the HBM
-  // latency ~10 times per array)
+  double* const buf1 = single ? lds : lds + maxsize;
+  double* const mats = lds + (single ? 1 : 2) * maxsize;
+  // A wave takes 64 lines and a part of their outputs at a time (a unit).  One or two groups
+  // of 64 lines share the four waves evenly; other remainders do so by halves or quarters
+  // where lines may be read twice, with two buffers (17x13x16, 5 groups: 216 us for 3072
+  // transforms there and back, 276 in whole lines).
+  auto split = [&](int nlines, int& groups, int& sh) {  // 1 << sh parts
+    groups = (nlines + 63) >> 6;
+    sh = groups == 1 ? 2 : (groups == 2 ? 1 : (single || (groups & 3) == 0 ? 0 : (groups == 3 ? 2 : 1)));
+  };
+  auto entry = [&](int p, int slot) -> LineEnt {
+    LineEnt e{0, 0, -1, 0};
+    if (slot < P.p[p].nlines) e = P.p[p].tab[slot];
+    return e;
+  };
+  int groups, sh;
+  split(P.p[0].nlines, groups, sh);
+  LineEnt en = entry(0, (wave >> sh) * 64 + lane);
+  // the array and the matrices, 8 loads in flight per thread (one load per iteration
+  // would wait out the memory latency ~10 times per array)
   constexpr int UL = 8;
   for (int e0 = 0; e0 < nin; e0 += UL * 256) {
     double v[UL];
 #pragma unroll
     for (int u = 0; u < UL; ++u) {
-      const int e = e0 + u * 256 + (int)threadIdx.x;
+      const int e = e0 + u * 256 + tid;
       v[u] = e < nin ? src[e] : 0.0;
+    }
+    double mv[2] = {0.0, 0.0};
+    if (e0 == 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u) mv[u] = u * 256 + tid < npool ? pool[u * 256 + tid] : 0.0;
     }
 #pragma unroll
     for (int u = 0; u < UL; ++u) {
-      const int e = e0 + u * 256 + (int)threadIdx.x;
+      const int e = e0 + u * 256 + tid;
       if (e < nin) buf0[e] = v[u];
     }
-  }
-  if (stage_pool)  // only passes outside 12..17 points per line read the matrices from LDS
-    for (int e = threadIdx.x; e < P.pool_size; e += blockDim.x) mats[e] = pool[e];
-  {
-    int o = 0;
-    for (int p = 0; p < P.npass; ++p) {
-      for (int e = threadIdx.x; e < P.nlines[p]; e += blockDim.x) ltab[o + e] = P.line_mat[p][e];
-      o += P.nlines[p];
+    if (e0 == 0) {
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+        if (u * 256 + tid < npool) mats[u * 256 + tid] = mv[u];
     }
   }
+  for (int e = 512 + tid; e < npool; e += 256) mats[e] = pool[e];
   __syncthreads();
   int cur = 0;
-  int dims[3] = {d0, d1, d2};
-  int loff = 0;
-  for (int p = 0; p < P.npass; ++p) {
-    const int ax = P.axis[p];
-    const int nout_ax = P.nout[p];
-    const int nin_ax = dims[ax];
-    int od[3] = {dims[0], dims[1], dims[2]};
-    od[ax] = nout_ax;
-    const int nout = od[0] * od[1] * od[2];
-    const double* x = cur ? buf1 : buf0;
-    double* y = cur ? buf0 : buf1;
-    const int* lm = ltab + loff;
-    const int stride = ax == 0 ? 1 : (ax == 1 ? dims[0] : dims[0] * dims[1]);
-    if (nin_ax >= 12 && nin_ax <= 17) {
-      switch (nin_ax) {
-        case 12: pass_lines<12>(x, y, pool, lm, ax, dims, od, nout_ax); break;
-        case 13: pass_lines<13>(x, y, pool, lm, ax, dims, od, nout_ax); break;
-        case 14: pass_lines<14>(x, y, pool, lm, ax, dims, od, nout_ax); break;
-        case 15: pass_lines<15>(x, y, pool, lm, ax, dims, od, nout_ax); break;
-        case 16: pass_lines<16>(x, y, pool, lm, ax, dims, od, nout_ax); break;
-        default: pass_lines<17>(x, y, pool, lm, ax, dims, od, nout_ax); break;
-      }
-      loff += P.nlines[p];
-      dims[0] = od[0];
-      dims[1] = od[1];
-      dims[2] = od[2];
-      cur ^= 1;
-      __syncthreads();
-      continue;
-    }
-    for (int e = threadIdx.x; e < nout; e += blockDim.x) {
-      const int i = e % od[0];
-      const int t = e / od[0];
-      const int j = t % od[1];
-      const int k = t / od[1];
-      int line, o, base_idx;
-      if (ax == 0) {
-        line = j + od[1] * k;
-        o = i;
-        base_idx = dims[0] * (j + dims[1] * k);
-      } else if (ax == 1) {
-        line = k;
-        o = j;
-        base_idx = i + dims[0] * dims[1] * k;
-      } else {
-        line = 0;
-        o = k;
-        base_idx = i + dims[0] * j;
-      }
-      const int off = lm[line];
-      double s0 = 0.0, s1 = 0.0, s2 = 0.0, s3 = 0.0;
-      if (off >= 0) {
-        const double* M = mats + off + o * nin_ax;
-        const double* xv = x + base_idx;
-        int q = 0;
-        for (; q + 4 <= nin_ax; q += 4) {
-          s0 += M[q] * xv[q * stride];
-          s1 += M[q + 1] * xv[(q + 1) * stride];
-          s2 += M[q + 2] * xv[(q + 2) * stride];
-          s3 += M[q + 3] * xv[(q + 3) * stride];
+  if (P.small) {
+    // up to 768 outputs per pass: three per thread, straight from LDS (a Jacobian at 9x7x4
+    // takes 2.45 ms, 2.96 with a thread per line); the next pass's places are loaded ahead
+    constexpr int US = kSmallArray / 256;
+    LineEnt a[US];
+    int oo[US];
+    auto places = [&](int p) {
+      const int no = P.p[p].nout, n = P.p[p].nlines * no;
+#pragma unroll
+      for (int u = 0; u < US; ++u) {
+        const int e = u * 256 + tid;
+        a[u].xb = -1;
+        oo[u] = 0;
+        if (e < n) {
+          const int l = e / no;
+          a[u] = P.p[p].tab[l];
+          oo[u] = e - l * no;
         }
-        for (; q < nin_ax; ++q) s0 += M[q] * xv[q * stride];
       }
-      y[e] = (s0 + s1) + (s2 + s3);
+    };
+    places(0);
+    for (int p = 0; p < npass; ++p) {
+      const int ni = P.p[p].nin, sin = P.p[p].sin, sout = P.p[p].sout;
+      const double* const x = cur ? buf1 : buf0;
+      double* const y = cur ? buf0 : buf1;
+      LineEnt c[US];
+      int o[US];
+#pragma unroll
+      for (int u = 0; u < US; ++u) {
+        c[u] = a[u];
+        o[u] = oo[u];
+      }
+      if (p + 1 < npass) places(p + 1);
+#pragma unroll
+      for (int u = 0; u < US; ++u) {
+        if (c[u].xb < 0) continue;
+        y[c[u].yb + o[u] * sout] = c[u].off < 0 ? 0.0 : line_dot(mats + c[u].off + o[u] * ni, x + c[u].xb, ni, sin);
+      }
+      __syncthreads();
+      cur ^= 1;
     }
-    loff += P.nlines[p];
-    dims[0] = od[0];
-    dims[1] = od[1];
-    dims[2] = od[2];
-    cur ^= 1;
+  } else
+  for (int p = 0; p < npass; ++p) {
+    const int nlines = P.p[p].nlines, no = P.p[p].nout, sin = P.p[p].sin, sout = P.p[p].sout;
+    const int ni = __builtin_amdgcn_readfirstlane(P.p[p].nin);
+    const double* const x = cur ? buf1 : buf0;
+    double* const y = single ? buf0 : (cur ? buf0 : buf1);
+    const int per = (no + (1 << sh) - 1) >> sh;
+    // the thread's line is all that is overwritten by it, or every line is read first
+    const bool barrier = single && groups <= 4;
+    LineEnt next{0, 0, -1, 0};
+    int ngroups = 0, nsh = 0;
+    if (p + 1 < npass) {
+      split(P.p[p + 1].nlines, ngroups, nsh);
+      next = entry(p + 1, (wave >> nsh) * 64 + lane);  // ahead of its use
+    }
+    if (ni <= kLineTemplates) {
+      const int units = barrier ? 4 : groups << sh;
+      for (int u = wave; u < units; u += 4) {
+        const int slot = (u >> sh) * 64 + lane, o0 = min(no, (u & ((1 << sh) - 1)) * per), o1 = min(no, o0 + per);
+        if (u >= 4) en = entry(p, slot);
+        const bool act = slot < nlines;
+        // four lengths: one per length would be 17 pieces of code, each met cold
+        if (ni <= 10) {
+          if (ni <= 6) pass_lines<6>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
+          else pass_lines<10>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
+        } else {
+          if (ni <= 14) pass_lines<14>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
+          else pass_lines<18>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
+        }
+      }
+    } else {
+      // longer lines: an output per thread, straight from LDS
+      for (int e = tid; e < nlines * no; e += 256) {
+        const LineEnt l = P.p[p].tab[e / no];
+        const int o = e % no;
+        y[l.yb + o * sout] = l.off < 0 ? 0.0 : line_dot(mats + l.off + o * ni, x + l.xb, ni, sin);
+      }
+    }
     __syncthreads();
+    cur ^= 1;
+    en = next;
+    groups = ngroups;
+    sh = nsh;
   }
-  const int nfin = dims[0] * dims[1] * dims[2];
-  const double* fin = cur ? buf1 : buf0;
-  if (accumulate) {
-    for (int e0 = 0; e0 < nfin; e0 += UL * 256) {
-      double v[UL];
-#pragma unroll
-      for (int u = 0; u < UL; ++u) {
-        const int e = e0 + u * 256 + (int)threadIdx.x;
-        v[u] = e < nfin ? dst[e] : 0.0;
-      }
-#pragma unroll
-      for (int u = 0; u < UL; ++u) {
-        const int e = e0 + u * 256 + (int)threadIdx.x;
-        if (e < nfin) dst[e] = v[u] + scale * fin[e];
-      }
-    }
-  } else if (post.n > 0) {
-    // the element-wise instructions fed by this pass (scale is 1 here); the other
-    // operands of UL elements per thread are loaded together, as the inputs were
+  const int nfin = P.size_out;
+  const double* const fin = cur ? buf1 : buf0;
+  if (post.n > 0) {
+    // the element-wise instructions fed by this pass; the other operands of UP elements
+    // per thread are loaded together, as the inputs were
+    constexpr int UP = 4;
     double* drow = post.dst + b * post.ds;
-    for (int e0 = 0; e0 < nfin; e0 += UL * 256) {
-      double o[UL][kMaxChain];
+    for (int e0 = 0; e0 < nfin; e0 += UP * 256) {
+      double o[UP][kMaxChain];
 #pragma unroll
-      for (int u = 0; u < UL; ++u) {
-        const int e = e0 + u * 256 + (int)threadIdx.x;
+      for (int u = 0; u < UP; ++u) {
+        const int e = e0 + u * 256 + tid;
         post_load(post, b, e < nfin ? e : 0, o[u]);
       }
 #pragma unroll
-      for (int u = 0; u < UL; ++u) {
-        const int e = e0 + u * 256 + (int)threadIdx.x;
+      for (int u = 0; u < UP; ++u) {
+        const int e = e0 + u * 256 + tid;
         if (e < nfin) drow[e] = post_ops(post, fin[e], o[u]);
       }
     }
   } else {
-    for (int e = threadIdx.x; e < nfin; e += blockDim.x) dst[e] = scale * fin[e];
+    for (int e = tid; e < nfin; e += 256) dst[e] = fin[e];
   }
-}
-
-// LDS bytes of a chain and how it is staged: the matrix pool goes to LDS only if some
-// pass has a line length outside 12..17 (the others read it with scalar loads); one
-// buffer serves when every pass is a line-by-line pass that keeps its line length.
-struct Apply3dShape {
-  size_t lds = 0;
-  int stage_pool = 0, inplace = 0;
-};
-inline Apply3dShape apply3d_shape(int d0, int d1, int d2, const Passes& P) {
-  Apply3dShape s;
-  size_t nl = 0;
-  int dm[3] = {d0, d1, d2}, square = 1;
-  for (int p = 0; p < P.npass; ++p) {
-    nl += (size_t)P.nlines[p];
-    const int nin_ax = dm[P.axis[p]];
-    if (nin_ax < 12 || nin_ax > 17) s.stage_pool = 1;
-    if (P.nout[p] != nin_ax) square = 0;
-    dm[P.axis[p]] = P.nout[p];
-  }
-  s.inplace = (!s.stage_pool && square) ? 1 : 0;
-  s.lds = ((s.inplace ? 1 : 2) * (size_t)P.maxsize + (s.stage_pool ? (size_t)P.pool_size : 0)) * sizeof(double) +
-          nl * sizeof(int);
-  return s;
 }
 
 }  // namespace kad

@@ -142,11 +142,9 @@ struct TrsvExtents {
 
 // Device copy of a chain of 1-D passes (matrix pool + per-line tables).
 struct DevPlan {
-  Passes P;
-  double* pool = nullptr;
-  int* lines = nullptr;
-  int d_in[3] = {0, 0, 0};
-  int d_out[3] = {0, 0, 0};
+  LinePlan P;
+  double* pool = nullptr;  // 1-D transforms: the line's matrix
+  int nin = 0, nout = 0;
 };
 
 struct Ctx {

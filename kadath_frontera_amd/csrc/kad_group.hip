@@ -18,6 +18,7 @@ namespace kad {
 
 namespace {
 typedef const __attribute__((address_space(4))) GroupOp COp;
+typedef const __attribute__((address_space(4))) ClusterStep CStep;
 
 struct Where {
   double* val;
@@ -50,6 +51,73 @@ __device__ __forceinline__ double row_value(const DevRow R, const double* x, boo
   return v;
 }
 
+// An element-wise region of the program: every array it needs from outside is read once
+// (or kept in a temporary), its intermediate values live in LDS temporaries
+// (lds[temporary][element of the thread][thread]), only what other instructions read is
+// stored.  U elements per thread and 8 / U steps have their array operands loaded
+// together: one at a time, a step waited out a memory latency and the decoding of the
+// next one (1900 cycles per step of 256 elements).  Bound by that latency and by the few
+// workgroups that the temporaries' LDS leaves per CU: J^T w at 13x9x8 moves 66 GB at 2.05
+// TB/s.  One instruction at a time it moved more arrays through memory: 34.2 ms, 31.8 now;
+// 5001 fp32 columns at 17x13x12 36.4 and 25.3.
+template <int U>
+__device__ __forceinline__ void cluster_body(const GroupArgs& g, const Where& at, const COp& op, double* lds, int tid) {
+  const int size = op.size, n = op.nsteps;
+  const CStep* const st = (const CStep*)g.steps + op.step0;
+  constexpr int Q = 8 / U > 4 ? 4 : 8 / U;
+  for (int e0 = 0; e0 < size; e0 += 256 * U) {
+    double ga[Q][U], gb[Q][U];
+    auto load = [&](int i0) {
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        if (i0 + i < n) {
+          if (st[i0 + i].a == -2) {
+            const double* const p = at.at(st[i0 + i].ga);
+#pragma unroll
+            for (int u = 0; u < U; ++u) ga[i][u] = p[min(e0 + u * 256 + tid, size - 1)];
+          }
+          if (st[i0 + i].b == -2) {
+            const double* const p = at.at(st[i0 + i].gb);
+#pragma unroll
+            for (int u = 0; u < U; ++u) gb[i][u] = p[min(e0 + u * 256 + tid, size - 1)];
+          }
+        }
+      }
+    };
+    load(0);
+    for (int i0 = 0; i0 < n; i0 += Q) {
+      double ca_[Q][U], cb_[Q][U];
+#pragma unroll
+      for (int i = 0; i < Q; ++i)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          ca_[i][u] = ga[i][u];
+          cb_[i][u] = gb[i][u];
+        }
+      load(i0 + Q);  // the next steps' operands, while these run
+#pragma unroll
+      for (int i = 0; i < Q; ++i) {
+        if (i0 + i >= n) break;
+        const CStep& s = st[i0 + i];
+        const int a = s.a, b = s.b, ca = s.ca, cb = s.cb, d = s.d, kind = s.kind;
+        double* const out = s.gd.slot >= 0 ? at.at(s.gd) : nullptr;
+        const double sc = s.s;
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          double* const l = lds + u * 256 + tid;
+          if (ca >= 0) l[ca * 256 * U] = ca_[i][u];
+          if (cb >= 0) l[cb * 256 * U] = cb_[i][u];
+          const double x = a >= 0 ? l[a * 256 * U] : ca_[i][u];
+          const double y = b >= 0 ? l[b * 256 * U] : cb_[i][u];
+          const double r = ew_op(kind, x, y, sc);
+          if (d >= 0) l[d * 256 * U] = r;
+          if (out && e0 + u * 256 + tid < size) out[e0 + u * 256 + tid] = r;
+        }
+      }
+    }
+  }
+}
+
 template <typename T>
 __device__ __forceinline__ void put_row(void* out, int64_t at, int acc, double v, double c0 = 0.0) {
   T* o = (T*)out + at;
@@ -60,9 +128,14 @@ __device__ __forceinline__ void put_row(void* out, int64_t at, int acc, double v
 __global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
   extern __shared__ double lds[];
   const int bid = blockIdx.x, tid = threadIdx.x;
-  int q = 0;
-  while (q + 1 < g.nent && bid >= g.e[q + 1].blk0) ++q;
-  const int loc = bid - g.e[q].blk0, nbp = g.e[q].nbp;
+  int q = 0, blk = 0;
+#pragma unroll
+  for (int i = 1; i < kGroupEntries; ++i)
+    if (i < g.nent && bid >= g.blk0[i]) {
+      q = i;
+      blk = g.blk0[i];
+    }
+  const int loc = bid - blk, nbp = g.e[q].nbp;
   const int oi = loc / nbp, b = loc - oi * nbp;
   if (oi >= g.e[q].nops || b >= g.e[q].nb) return;  // padding
   const COp& op = *((COp*)g.ops + g.e[q].op0 + oi);
@@ -83,7 +156,7 @@ __global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
       }
     const double* a = at.at(op.a);
     if (kind == GK_LIN) {
-      apply3d_body(a, post.dst, op.d0, op.d1, op.d2, op.P, op.pool, 0, 1.0, op.stage_pool, op.inplace, post, 0, lds);
+      apply3d_body(a, post.dst, op.P, post, 0, lds);
       return;
     }
     const double* y = op.b.slot >= 0 ? at.at(op.b) : nullptr;
@@ -107,6 +180,13 @@ __global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
         if (e < size) post.dst[e] = post_ops(post, ew_op(ew, xv[u], yv[u], s), o[u]);
       }
     }
+    return;
+  }
+  if (kind == GK_CLUSTER) {
+    // few temporaries leave LDS for more elements per thread
+    if (op.per == 4) cluster_body<4>(g, at, op, lds, tid);
+    else if (op.per == 2) cluster_body<2>(g, at, op, lds, tid);
+    else cluster_body<1>(g, at, op, lds, tid);
     return;
   }
   if (kind == GK_SEED) {

@@ -10,7 +10,7 @@ struct DevRow {
   double gw;
 };
 
-enum : int { GK_LIN = 0, GK_EW = 1, GK_EXPORT_IN = 2, GK_EXPORT_BD = 3, GK_EXPORT_GL = 4, GK_SEED = 5 };
+enum : int { GK_LIN = 0, GK_EW = 1, GK_EXPORT_IN = 2, GK_EXPORT_BD = 3, GK_EXPORT_GL = 4, GK_SEED = 5, GK_CLUSTER = 6 };
 
 // An operand: a slot of the value arena (tan = 0) or of the program's region of the
 // tangent arena (tan = 1); slot < 0: none.
@@ -23,18 +23,26 @@ struct GroupStep {
   double s = 0.0;
 };
 
+// One element-wise instruction of a cluster, in execution order.  Operand a / b: a
+// temporary (>= 0), none (-1), or an array (-2: ga / gb), kept in temporary ca / cb when
+// that is >= 0.  The result goes to temporary d (>= 0) and to array gd (slot >= 0).
+constexpr int kClusterTemps = 20;
+struct ClusterStep {
+  int kind = 0, a = -1, b = -1, ca = -1, cb = -1, d = -1;
+  GroupOpnd ga, gb, gd;
+  double s = 0.0;
+};
+
 // One instruction (with the element-wise instructions it absorbed, as PostOp): the
 // workgroup of (instruction, column) does all of it.
 struct GroupOp {
   int kind = 0, nstep = 0;
-  int d0 = 0, d1 = 0, d2 = 0;           // LIN: input dimensions
-  int stage_pool = 0, inplace = 0;      // LIN: Apply3dShape
   int ew = 0, size = 0;                 // EW: kind, elements; SEED: elements
   GroupOpnd dst, a, b;
   double s = 0.0;                       // EW scalar; EXPORT_GL: factor
   GroupStep st[kMaxChain];
-  Passes P;                             // LIN
-  const double* pool = nullptr;
+  int step0 = 0, nsteps = 0, per = 1;   // CLUSTER: its steps in the step table, elements per thread
+  LinePlan P;                           // LIN
   // exports
   const DevRow* rows = nullptr;
   int nrows = 0, row0 = 0, accumulate = 0, bsign = 1;
@@ -52,12 +60,13 @@ struct GroupOp {
 // nbp >= nb columns each), tangent slot s of column b at base + (s nb + b) stride,
 // results in column col0 + b.
 struct GroupEntry {
-  int blk0, nops, op0, nb, nbp, u0;
+  int nops, op0, nb, nbp, u0, pad;
   int64_t base, col0;
 };
 constexpr int kGroupEntries = 32;
 struct GroupArgs {
   const GroupOp* ops = nullptr;
+  const ClusterStep* steps = nullptr;
   double* val = nullptr;
   double* tan = nullptr;
   int64_t stride = 0;
@@ -66,6 +75,7 @@ struct GroupArgs {
   const double* w = nullptr;  // transposed exports: out[column] += w . exported rows
   int dtype = 0;
   int nent = 0;
+  int blk0[kGroupEntries];  // first workgroup of each entry
   GroupEntry e[kGroupEntries];
 };
 

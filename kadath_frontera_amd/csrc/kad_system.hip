@@ -14,6 +14,8 @@
 #include "host/xcts.hpp"
 #include "host/parsed_system.hpp"
 #include "../../include/kadath_amd.h"
+#include <array>
+#include <map>
 #include <vector>
 #include <chrono>
 #include <algorithm>
@@ -400,10 +402,6 @@ __global__ void double_update_kernel(double* __restrict__ v, int size, const dou
   if (e < size) v[e] += scale * X[k];
 }
 
-struct DevPlanX {
-  kad::Passes P;
-  double* pool = nullptr;
-};
 
 struct DevProgram {
   std::vector<Instr> code;       // slots of tangent operands remapped to physical slots
@@ -444,7 +442,7 @@ struct kad_system_impl {
   double* tan_arena = nullptr;  // nphys_max * B * stride
   double* F = nullptr;          // n_rows
   double* scratch = nullptr;    // small
-  std::vector<DevPlanX> plans;
+  std::vector<kad::LinePlan> plans;  // by the tracer's plan ids; npass 0: no instruction uses it
   std::vector<DevRow*> row_tabs;
   std::vector<int*> seed_pos;
   std::vector<double*> seed_val;
@@ -530,6 +528,7 @@ struct kad_system_impl {
   }
   int64_t slot_stride(const Opnd& o) const { return o.space == SP_VAL ? 0 : stride; }
   int setup();
+  int upload_plans();
   // out: fp64 (dtype 0) or fp32 (dtype 1) column-major rows x columns with leading
   // dimension ldo, columns from col0; with w != nullptr the exports are transposed
   // instead (out: fp64 per column, += w . row).  st / tan: the stream and tangent arena
@@ -550,13 +549,14 @@ struct kad_system_impl {
   // grouped execution: the instruction table, the value program, the tangent programs
   // (one per layout entry) and the parameters' programs by dependency level
   kad::GroupOp* gops = nullptr;
+  kad::ClusterStep* gsteps = nullptr;
   GroupProg gval;
   std::vector<GroupProg> gtan, gpar;
   bool gtan_ok = false;         // every tangent program can be grouped
   double* grp_arena = nullptr;  // tangent slots of the columns of one round
   size_t grp_cap = 0;           // doubles
   int group_build(std::vector<Instr> code, int nvirt, bool value, int seed_tab, GroupProg& gp,
-                  std::vector<kad::GroupOp>& ops);
+                  std::vector<kad::GroupOp>& ops, std::vector<kad::ClusterStep>& steps);
   int group_round(const std::vector<GroupItem>& items, void* out, int64_t ldo, int dtype, const double* w);
   int group_columns(std::vector<GroupItem> items, void* out, int64_t ldo, int dtype, const double* w);
   // columns [c0, c1) of J (or, with w, entries of J^T w) into out, whose column 0 is
@@ -627,7 +627,7 @@ static void pull_passes_to_readers(std::vector<Instr>& code, int nvirt) {
   }
 }
 
-static void mark_fusions(std::vector<Instr>& code, int nvirt, const std::vector<DevPlanX>& plans) {
+static void mark_fusions(std::vector<Instr>& code, int nvirt, const std::vector<kad::LinePlan>& plans) {
   pull_passes_to_readers(code, nvirt);
   std::vector<int> reads(nvirt, 0);
   for (Instr& in : code) {
@@ -641,10 +641,7 @@ static void mark_fusions(std::vector<Instr>& code, int nvirt, const std::vector<
     int size = h.size;
     if (h.kind == I_LIN) {
       if (h.plan < 0 || h.plan >= (int)plans.size()) continue;
-      const kad::Passes& P = plans[h.plan].P;
-      int od[3] = {h.din[0], h.din[1], h.din[2]};
-      for (int p = 0; p < P.npass; ++p) od[P.axis[p]] = P.nout[p];
-      size = od[0] * od[1] * od[2];
+      size = plans[h.plan].size_out;
     }
     int m = 0;
     while (m < kad::kMaxChain && t + m + 1 < code.size()) {
@@ -686,7 +683,7 @@ static kad::PostOp chain_of(const std::vector<Instr>& code, size_t t, const std:
 }
 
 // Liveness-based reuse of tangent slots within one program.
-static int allocate_slots(std::vector<Instr>& code, int nvirt, const std::vector<DevPlanX>& plans) {
+static int allocate_slots(std::vector<Instr>& code, int nvirt, const std::vector<kad::LinePlan>& plans) {
   mark_fusions(code, nvirt, plans);
   std::vector<int> last(nvirt, -1);
   auto use = [&](const Opnd& o, int t) {
@@ -737,6 +734,62 @@ static int allocate_slots(std::vector<Instr>& code, int nvirt, const std::vector
   return nphys;
 }
 
+// The line tables and matrices of every plan, for the array its instructions run it on
+// (a plan belongs to one domain and one layout of it).
+int kad_system_impl::upload_plans() {
+  Tracer& tr = sys->tr;
+  std::vector<std::array<int, 3>> din(tr.plans.size(), {0, 0, 0});
+  bool one = true;
+  auto scan = [&](const std::vector<Instr>& code) {
+    for (const Instr& in : code) {
+      if (in.kind != I_LIN) continue;
+      if (in.plan < 0 || in.plan >= (int)tr.plans.size()) {
+        one = false;
+        continue;
+      }
+      const std::array<int, 3> d = {in.din[0], in.din[1], in.din[2]};
+      if (din[in.plan][0] == 0) din[in.plan] = d;
+      one = one && din[in.plan] == d;
+    }
+  };
+  scan(tr.val.code);
+  scan(sys->obs_prog.code);
+  scan(sys->glob_prog.code);
+  for (auto* v : {&sys->tprog, &sys->obs_tprog, &sys->par_prog, &sys->glob_tprog, &sys->glob_par_prog})
+    for (auto& p : *v) scan(p.code);
+  if (!one) return KAD_ERR_ARG;
+  std::vector<double> pools;
+  std::vector<kad::LineEnt> tabs;
+  std::vector<std::array<size_t, kad::MAX_PASSES + 1>> where(tr.plans.size());
+  plans.assign(tr.plans.size(), kad::LinePlan());
+  for (size_t q = 0; q < tr.plans.size(); ++q) {
+    if (din[q][0] == 0) continue;
+    const HostPlan& hp = tr.plans[q];
+    std::vector<kad::PassDesc> pd;
+    for (auto& ps : hp.passes) pd.push_back({ps.axis, ps.nout, ps.line_mat.data()});
+    size_t lines = 0, used = 0;
+    size_t toff[kad::MAX_PASSES];
+    for (size_t p = 0; p < pd.size(); ++p) lines += (size_t)hp.maxsize;
+    std::vector<kad::LineEnt> tab(std::max<size_t>(1, lines));
+    if (!kad::lines_build(din[q][0], din[q][1], din[q][2], pd.data(), (int)pd.size(), (int)hp.pool.size(), plans[q],
+                          tab.data(), tab.size(), &used, toff))
+      return KAD_ERR_ARG;
+    for (int p = 0; p < plans[q].npass; ++p) where[q][p] = tabs.size() + toff[p];
+    where[q][kad::MAX_PASSES] = pools.size();
+    tabs.insert(tabs.end(), tab.begin(), tab.begin() + used);
+    pools.insert(pools.end(), hp.pool.begin(), hp.pool.end());
+  }
+  double* dp;
+  kad::LineEnt* dt;
+  int rc;
+  if ((rc = upload(pools, &dp)) || (rc = upload(tabs, &dt))) return rc;
+  for (size_t q = 0; q < plans.size(); ++q) {
+    plans[q].pool = dp + where[q][kad::MAX_PASSES];
+    for (int p = 0; p < plans[q].npass; ++p) plans[q].p[p].tab = dt + where[q][p];
+  }
+  return KAD_OK;
+}
+
 int kad_system_impl::setup() {
   Tracer& tr = sys->tr;
   // slot stride: the largest domain array (coef layout), rounded to 8 doubles
@@ -749,24 +802,7 @@ int kad_system_impl::setup() {
   for (auto& cs : tr.const_slots)
     KAD_HIP_CHECK(hipMemcpy(val_arena + (int64_t)cs.first * stride, cs.second.data(),
                             cs.second.size() * sizeof(double), hipMemcpyHostToDevice));
-  // plans
-  for (auto& hp : tr.plans) {
-    DevPlanX dp;
-    if ((rc = upload(hp.pool, &dp.pool))) return rc;
-    dp.P.npass = (int)hp.passes.size();
-    dp.P.maxsize = hp.maxsize;
-    dp.P.pool_size = (int)hp.pool.size();
-    if (dp.P.npass > kad::MAX_PASSES) return KAD_ERR_ARG;
-    for (int p = 0; p < dp.P.npass; ++p) {
-      int* lm;
-      if ((rc = upload(hp.passes[p].line_mat, &lm))) return rc;
-      dp.P.axis[p] = hp.passes[p].axis;
-      dp.P.nout[p] = hp.passes[p].nout;
-      dp.P.line_mat[p] = lm;
-      dp.P.nlines[p] = (int)hp.passes[p].line_mat.size();
-    }
-    plans.push_back(dp);
-  }
+  if ((rc = upload_plans())) return rc;
   for (auto& rt : tr.row_tabs) {
     std::vector<DevRow> h(rt.size());
     for (size_t i = 0; i < rt.size(); ++i) h[i] = {rt[i].pos, rt[i].gpos, rt[i].gw};
@@ -849,21 +885,23 @@ int kad_system_impl::setup() {
   }
   // the same programs by dependency level
   std::vector<kad::GroupOp> ops;
-  if ((rc = group_build(tr.val.code, 0, true, -1, gval, ops))) return rc;
+  std::vector<kad::ClusterStep> steps;
+  if ((rc = group_build(tr.val.code, 0, true, -1, gval, ops, steps))) return rc;
   gtan.resize(sys->tprog.size());
   gtan_ok = !gtan.empty();
   for (size_t p = 0; p < sys->tprog.size(); ++p) {
-    if ((rc = group_build(sys->tprog[p].code, sys->tprog[p].nslots, false, tprogs[p].seed_tab, gtan[p], ops))) return rc;
+    if ((rc = group_build(sys->tprog[p].code, sys->tprog[p].nslots, false, tprogs[p].seed_tab, gtan[p], ops, steps)))
+      return rc;
     gtan_ok = gtan_ok && gtan[p].ok;
   }
   gpar.resize(sys->par_prog.size());
   for (int k = 0; k < sys->ndouble; ++k) {
     const int p = sys->dvar_par[k];
-    if ((rc = group_build(sys->par_prog[p].code, sys->par_prog[p].nslots, false, sys->par_tab[p], gpar[p], ops)))
+    if ((rc = group_build(sys->par_prog[p].code, sys->par_prog[p].nslots, false, sys->par_tab[p], gpar[p], ops, steps)))
       return rc;
     gtan_ok = gtan_ok && gpar[p].ok;
   }
-  if ((rc = upload(ops, &gops))) return rc;
+  if ((rc = upload(ops, &gops)) || (rc = upload(steps, &gsteps))) return rc;
   if ((rc = dmalloc((void**)&F, (size_t)sys->n_rows * sizeof(double)))) return rc;
   if ((rc = dmalloc((void**)&scratch, 64 * sizeof(double)))) return rc;
   return KAD_OK;
@@ -883,7 +921,6 @@ int kad_system_impl::run(const std::vector<Instr>& code, int nb, int u0, int see
     const Domain& dm = sys->doms[in.dom];
     switch (in.kind) {
       case I_LIN: {
-        const DevPlanX& p = plans[in.plan];
         const int batch = (in.dst.space == SP_VAL) ? 1 : nb;
         kad::PostOp post;
         if (in.fuse > 0 && fuse_ew) {
@@ -891,8 +928,7 @@ int kad_system_impl::run(const std::vector<Instr>& code, int nb, int u0, int see
           post = chain_of(code, t, slot_ptr, [&](const Opnd& o) { return slot_stride(o); });
           t += in.fuse;
         }
-        int rc = kad::apply3d_launch(slot_ptr(in.a), stride, slot_ptr(in.dst), stride, batch, in.din[0], in.din[1],
-                                     in.din[2], p.P, p.pool, 0, 1.0, s, &post);
+        int rc = kad::apply3d_launch(slot_ptr(in.a), stride, slot_ptr(in.dst), stride, batch, plans[in.plan], s, &post);
         if (rc) return rc;
         break;
       }
@@ -1041,90 +1077,328 @@ bool kad_system_impl::split_values(int ns) {
   return vsplit_ok;
 }
 
+// Instructions that run as one unit of the grouped execution: a pass with the
+// element-wise chain it absorbed (code[t[1..]]), a cluster of element-wise instructions, or
+// one other instruction.
+struct GroupUnit {
+  std::vector<int> t;
+  bool cluster = false;
+  int level = 0;
+};
+
+// Whether the element-wise instructions code[t], t in ts (program order), fit the
+// temporaries of one cluster, and if steps is given, its steps.  An operand from outside
+// that is used again is kept in a temporary while one is free (else it is read again); a
+// value made inside must be kept until its last use inside.  stored(slot): the value is
+// read outside the cluster.  Returns how many of ts fit.
+static size_t cluster_steps(const std::vector<Instr>& code, const std::vector<int>& ts,
+                            const std::function<bool(int)>& stored,
+                            const std::function<kad::GroupOpnd(const Opnd&)>& opnd,
+                            std::vector<kad::ClusterStep>* steps) {
+  typedef std::pair<int, int> Key;  // (space, slot)
+  std::map<Key, std::vector<int>> uses;
+  for (size_t i = 0; i < ts.size(); ++i)
+    for (const Opnd* o : {&code[ts[i]].a, &code[ts[i]].b})
+      if (o->slot >= 0) uses[{o->space, o->slot}].push_back((int)i);
+  auto next_use = [&](const Key& k, int i) {  // the first use after instruction i, or -1
+    auto it = uses.find(k);
+    if (it == uses.end()) return -1;
+    auto u = std::upper_bound(it->second.begin(), it->second.end(), i);
+    return u == it->second.end() ? -1 : *u;
+  };
+  struct Temp {
+    Key key{-1, -1};
+    bool input = false;
+  };
+  std::vector<Temp> tmp(kad::kClusterTemps);
+  auto find = [&](const Key& k) {
+    for (int q = 0; q < (int)tmp.size(); ++q)
+      if (tmp[q].key == k) return q;
+    return -1;
+  };
+  auto release = [&](int i) {  // temporaries whose value is not used after instruction i
+    for (Temp& q : tmp)
+      if (q.key.first >= 0 && next_use(q.key, i) < 0) q = Temp();
+  };
+  for (size_t i = 0; i < ts.size(); ++i) {
+    const Instr& in = code[ts[i]];
+    kad::ClusterStep st;
+    st.kind = in.ew;
+    st.s = in.s;
+    auto operand = [&](const Opnd& o, int& where, int& cache, kad::GroupOpnd& g) {
+      if (o.slot < 0) return;
+      const Key k{o.space, o.slot};
+      const int q = find(k);
+      if (q >= 0) {
+        where = q;
+        return;
+      }
+      where = -2;
+      if (steps) g = opnd(o);
+      if (next_use(k, (int)i) < 0) return;
+      const int f = find({-1, -1});
+      if (f >= 0) {
+        tmp[f].key = k;
+        tmp[f].input = true;
+        cache = f;
+      }
+    };
+    operand(in.a, st.a, st.ca, st.ga);
+    if (in.b.slot >= 0 && in.b.space == in.a.space && in.b.slot == in.a.slot) {
+      st.b = st.a;  // both operands are the same value
+      st.gb = st.ga;
+    } else {
+      operand(in.b, st.b, st.cb, st.gb);
+    }
+    release((int)i);
+    const Key d{in.dst.space, in.dst.slot};
+    const int nu = next_use(d, (int)i);
+    if (nu >= 0) {
+      int f = find({-1, -1});
+      if (f < 0) {  // give up the outside operand that is used last
+        int far = -1;
+        for (int q = 0; q < (int)tmp.size(); ++q)
+          if (tmp[q].input && next_use(tmp[q].key, (int)i) > far) {
+            far = next_use(tmp[q].key, (int)i);
+            f = q;
+          }
+        // (not one that this very step reads from or caches into)
+        if (f < 0) return i;
+        if (f == st.ca || f == st.cb) {
+          if (f == st.ca) st.ca = -1;
+          else st.cb = -1;
+        }
+      }
+      tmp[f].key = d;
+      tmp[f].input = false;
+      st.d = f;
+    }
+    if (steps) {
+      if (stored(in.dst.slot)) st.gd = opnd(in.dst);
+      steps->push_back(st);
+    }
+  }
+  return ts.size();
+}
+
 // The instructions of a program by dependency level: an instruction's level is one past
 // the last of its operands' (ASAP), so the instructions of a level are independent.
-// Tangent programs absorb element-wise chains first (mark_fusions) and their slots are
-// reused between levels: a slot is free again after the last level that reads it.
 // Exports add to rows that earlier exports may have written: in the value program an
 // export follows every earlier one that shares a row, in a tangent program every
-// earlier one (the transposed export adds all of them to one entry).  A program with
-// other instructions, or a slot written twice, stays on the per-instruction path (ok
-// false).
+// earlier one (the transposed export adds all of them to one entry).
+// Tangent programs: the value program's results are all kept, a tangent's are not, so
+// - multiplications and divisions by one drop out (they change no bit);
+// - element-wise instructions between two rounds of passes (the same number of passes on
+//   the longest way to them) run as clusters, split where they are not connected;
+// - a pass whose result only feeds an element-wise instruction that no cluster reads
+//   takes that one (and the chain after it) into its store phase;
+// - slots are reused between levels: free again after the last level that reads them.
+// A program with other instructions, or a slot written twice, stays on the
+// per-instruction path (ok false).
 int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value, int seed_tab, GroupProg& gp,
-                                 std::vector<kad::GroupOp>& ops) {
+                                 std::vector<kad::GroupOp>& ops, std::vector<kad::ClusterStep>& steps) {
   gp = GroupProg();
-  if (!value) mark_fusions(code, nvirt, plans);
   const int space = value ? SP_VAL : SP_TAN;
   const int nslots = std::max(1, value ? sys->tr.nval_slots : nvirt);
-  std::vector<int> wlev(nslots, -1), rlev(nslots, -1);  // level that writes / last reads a slot
-  struct Unit {
-    size_t t;
-    int m, level;
-    double cost;
+  const int N = (int)code.size();
+  auto is_export = [](const Instr& in) {
+    return in.kind == I_EXPORT_IN || in.kind == I_EXPORT_BD || in.kind == I_EXPORT_GL;
   };
-  std::vector<Unit> units;
-  struct Rows {
-    int lo, hi, level;
-  };
-  std::vector<Rows> written;
-  int depth = 0;
-  for (size_t t = 0; t < code.size(); ++t) {
+  // the form that can be grouped
+  std::vector<int> writer(nslots, -1);
+  for (int t = 0; t < N; ++t) {
     const Instr& in = code[t];
-    const int m = (!value && (in.kind == I_LIN || in.kind == I_EW)) ? in.fuse : 0;
-    const bool exp = in.kind == I_EXPORT_IN || in.kind == I_EXPORT_BD || in.kind == I_EXPORT_GL;
-    if (!exp && in.kind != I_LIN && in.kind != I_EW && !(in.kind == I_SEED && !value)) return KAD_OK;
-    int level = 0;
-    std::vector<int> reads;
-    for (int k = 0; k <= m; ++k) {
-      const Instr& e = code[t + k];
-      for (const Opnd* o : {&e.a, &e.b}) {
-        if (o->slot < 0 || (in.kind == I_SEED)) continue;
-        if (o->space != space) {
-          if (value || exp) return KAD_OK;
-          continue;  // the values are there before any tangent
-        }
-        if (k > 0 && o->slot == code[t + k - 1].dst.slot) continue;  // the chain's own value
-        if (o->slot >= nslots) return KAD_OK;
-        level = std::max(level, wlev[o->slot] + 1);
-        reads.push_back(o->slot);
+    if (!is_export(in) && in.kind != I_LIN && in.kind != I_EW && !(in.kind == I_SEED && !value)) return KAD_OK;
+    if (in.kind != I_SEED)
+      for (const Opnd* o : {&in.a, &in.b}) {
+        if (o->slot < 0) continue;
+        if (o->space != space && (value || is_export(in))) return KAD_OK;
+        if (o->space == space && (o->slot >= nslots || (!value && writer[o->slot] < 0))) return KAD_OK;
+      }
+    if (!is_export(in)) {
+      const Opnd& d = in.dst;
+      if (d.space != space || d.slot < 0 || d.slot >= nslots || writer[d.slot] >= 0) return KAD_OK;
+      if (in.kind == I_EW && (in.ew < 0 || in.ew > EW_SDIV || in.a.slot < 0)) return KAD_OK;
+      if (in.kind == I_LIN && (in.plan < 0 || in.plan >= (int)plans.size())) return KAD_OK;
+      writer[d.slot] = t;
+    }
+  }
+  // x * 1 and x / 1: later reads take x
+  std::vector<char> skip(N, 0);
+  if (!value) {
+    std::vector<int> alias(nslots);
+    for (int s = 0; s < nslots; ++s) alias[s] = s;
+    for (int t = 0; t < N; ++t) {
+      Instr& in = code[t];
+      if (in.kind != I_SEED)
+        for (Opnd* o : {&in.a, &in.b})
+          if (o->slot >= 0 && o->space == SP_TAN) o->slot = alias[o->slot];
+      if (in.kind == I_EW && (in.ew == EW_SCAL || in.ew == EW_SDIV) && in.s == 1.0 && in.a.space == SP_TAN) {
+        alias[in.dst.slot] = in.a.slot;
+        skip[t] = 1;
       }
     }
-    if (exp) {
-      const int n = in.kind == I_EXPORT_GL ? 1 : in.nrows;
-      for (const Rows& r : written)
-        if (!value || (in.row0 < r.hi && r.lo < in.row0 + n)) level = std::max(level, r.level + 1);
-      written.push_back({in.row0, in.row0 + n, level});
-    } else {
-      const Opnd& d = code[t + m].dst;
-      if (d.space != space || d.slot < 0 || d.slot >= nslots || wlev[d.slot] >= 0) return KAD_OK;
-      wlev[d.slot] = level;
-    }
-    for (int s : reads) rlev[s] = std::max(rlev[s], level);
-    units.push_back({t, m, level, 0.0});
-    depth = std::max(depth, level + 1);
-    t += m;
   }
-  // slots: reused once no level reads them any more
-  std::vector<int> phys(nslots, -1), freelist;
+  // readers of every slot of this space, in program order
+  std::vector<std::vector<int>> readers(nslots);
+  auto for_reads = [&](int t, const std::function<void(int)>& f) {
+    const Instr& in = code[t];
+    if (in.kind == I_SEED) return;
+    int first = -1;
+    for (const Opnd* o : {&in.a, &in.b})
+      if (o->slot >= 0 && o->space == space && o->slot != first) {
+        f(o->slot);
+        first = o->slot;
+      }
+  };
+  for (int t = 0; t < N; ++t)
+    if (!skip[t]) for_reads(t, [&](int s) { readers[s].push_back(t); });
+  // units
+  std::vector<GroupUnit> units;
+  std::vector<int> unit_of(N, -1);
+  if (value) {
+    for (int t = 0; t < N; ++t) {
+      unit_of[t] = (int)units.size();
+      units.push_back({{t}, false, 0});
+    }
+  } else {
+    std::vector<int> depth(N, 0);  // passes on the longest way to the instruction's result
+    for (int t = 0; t < N; ++t) {
+      if (skip[t]) continue;
+      for_reads(t, [&](int s) { depth[t] = std::max(depth[t], depth[writer[s]]); });
+      if (code[t].kind == I_LIN) ++depth[t];
+    }
+    auto out_size = [&](const Instr& l) { return plans[l.plan].size_out; };
+    // chains absorbed by a pass: each value has one reader, an element-wise instruction
+    // that reads it once, and no element-wise instruction reads the chain's end
+    for (int t = 0; t < N; ++t) {
+      if (skip[t] || code[t].kind != I_LIN) continue;
+      std::vector<int> chain{t};
+      while ((int)chain.size() <= kad::kMaxChain) {
+        const int v = code[chain.back()].dst.slot;
+        if (readers[v].size() != 1) break;
+        const int r = readers[v][0];
+        const Instr& e = code[r];
+        if (e.kind != I_EW || e.size != out_size(code[t])) break;
+        if (e.a.space == SP_TAN && e.a.slot == v && e.b.slot >= 0 && e.b.space == SP_TAN && e.b.slot == v) break;
+        // another tangent operand must be ready before this pass's round
+        const Opnd& o = (e.a.space == SP_TAN && e.a.slot == v) ? e.b : e.a;
+        if (o.slot >= 0 && o.space == SP_TAN && depth[writer[o.slot]] >= depth[t]) break;
+        chain.push_back(r);
+      }
+      while (chain.size() > 1) {  // back to an end that no element-wise instruction reads
+        bool ew = false;
+        for (int r : readers[code[chain.back()].dst.slot]) ew = ew || code[r].kind == I_EW;
+        if (!ew) break;
+        chain.pop_back();
+      }
+      for (int q : chain) unit_of[q] = (int)units.size();
+      units.push_back({chain, false, 0});
+    }
+    // clusters: connected through tangent values, of one depth and array size
+    std::vector<int> root(N);
+    for (int t = 0; t < N; ++t) root[t] = t;
+    std::function<int(int)> top = [&](int x) { return root[x] == x ? x : root[x] = top(root[x]); };
+    auto member = [&](int t) { return !skip[t] && code[t].kind == I_EW && unit_of[t] < 0; };
+    for (int s = 0; s < nslots; ++s) {
+      std::vector<int> m;
+      if (writer[s] >= 0 && member(writer[s])) m.push_back(writer[s]);
+      for (int r : readers[s])
+        if (member(r)) m.push_back(r);
+      for (size_t x = 0; x < m.size(); ++x)
+        for (size_t y = x + 1; y < m.size(); ++y)
+          if (depth[m[x]] == depth[m[y]] && code[m[x]].size == code[m[y]].size) root[top(m[x])] = top(m[y]);
+    }
+    std::map<int, std::vector<int>> clusters;
+    for (int t = 0; t < N; ++t)
+      if (member(t)) clusters[top(t)].push_back(t);
+    for (auto& c : clusters) {
+      std::vector<int> rest = c.second;
+      while (!rest.empty()) {
+        const size_t k = cluster_steps(code, rest, [](int) { return false; }, nullptr, nullptr);
+        if (k == 0) return KAD_OK;  // (one instruction always fits)
+        std::vector<int> part(rest.begin(), rest.begin() + k);
+        for (int t : part) unit_of[t] = (int)units.size();
+        units.push_back({part, true, 0});
+        rest.erase(rest.begin(), rest.begin() + k);
+      }
+    }
+    for (int t = 0; t < N; ++t)
+      if (!skip[t] && unit_of[t] < 0) {
+        unit_of[t] = (int)units.size();
+        units.push_back({{t}, false, 0});
+      }
+  }
+  // levels: longest way over the units' dependencies (an acyclic graph: a cluster's
+  // instructions have the same number of passes before them)
+  std::vector<std::vector<int>> after(units.size());
+  std::vector<int> waits(units.size(), 0);
+  auto edge = [&](int from, int to) {
+    if (from == to) return;
+    after[from].push_back(to);
+    ++waits[to];
+  };
+  std::vector<int> exported;
+  for (int t = 0; t < N; ++t) {
+    if (skip[t]) continue;
+    for_reads(t, [&](int s) {
+      if (writer[s] >= 0) edge(unit_of[writer[s]], unit_of[t]);
+    });
+    if (is_export(code[t])) {
+      const int n = code[t].kind == I_EXPORT_GL ? 1 : code[t].nrows;
+      for (int q : exported) {
+        const int nq = code[q].kind == I_EXPORT_GL ? 1 : code[q].nrows;
+        if (!value || (code[t].row0 < code[q].row0 + nq && code[q].row0 < code[t].row0 + n))
+          edge(unit_of[q], unit_of[t]);
+      }
+      exported.push_back(t);
+    }
+  }
+  std::vector<int> ready;
+  for (size_t u = 0; u < units.size(); ++u)
+    if (waits[u] == 0) ready.push_back((int)u);
+  size_t done = 0;
+  int depth = 0;
+  while (!ready.empty()) {
+    const int u = ready.back();
+    ready.pop_back();
+    ++done;
+    depth = std::max(depth, units[u].level + 1);
+    for (int v : after[u]) {
+      units[v].level = std::max(units[v].level, units[u].level + 1);
+      if (--waits[v] == 0) ready.push_back(v);
+    }
+  }
+  if (done != units.size()) return KAD_OK;
+  // slots: a unit stores what other units read; reused once no level reads them any more
+  std::vector<int> rlev(nslots, -1);
+  std::vector<char> live(nslots, 0);
+  for (int t = 0; t < N; ++t) {
+    if (skip[t]) continue;
+    for_reads(t, [&](int s) {
+      if (writer[s] < 0 || unit_of[writer[s]] == unit_of[t]) return;
+      live[s] = 1;
+      rlev[s] = std::max(rlev[s], units[unit_of[t]].level);
+    });
+  }
   std::vector<std::vector<int>> by_level(depth);
   for (size_t u = 0; u < units.size(); ++u) by_level[units[u].level].push_back((int)u);
+  std::vector<int> phys(nslots, -1), freelist;
   if (!value) {
     std::vector<std::vector<int>> dies(depth);
-    for (int s = 0; s < nslots; ++s)
-      if (wlev[s] >= 0) dies[std::max(wlev[s], rlev[s])].push_back(s);
     for (int l = 0; l < depth; ++l) {
-      for (int u : by_level[l]) {
-        const Instr& e = code[units[u].t + units[u].m];
-        if (e.dst.slot < 0 || e.dst.space != SP_TAN || e.kind == I_EXPORT_IN || e.kind == I_EXPORT_BD ||
-            e.kind == I_EXPORT_GL)
-          continue;
-        if (freelist.empty()) {
-          phys[e.dst.slot] = gp.nphys++;
-        } else {
-          phys[e.dst.slot] = freelist.back();
-          freelist.pop_back();
+      for (int u : by_level[l])
+        for (int t : units[u].t) {
+          if (is_export(code[t]) || !(live[code[t].dst.slot] || (!units[u].cluster && t == units[u].t.back()))) continue;
+          const int s = code[t].dst.slot;
+          if (freelist.empty()) {
+            phys[s] = gp.nphys++;
+          } else {
+            phys[s] = freelist.back();
+            freelist.pop_back();
+          }
+          dies[std::max(l, rlev[s])].push_back(s);
         }
-      }
       for (int s : dies[l]) freelist.push_back(phys[s]);
     }
   }
@@ -1142,42 +1416,53 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
     double bytes = 0.0;
     std::vector<std::pair<double, kad::GroupOp>> lv;  // cost, instruction: the longest start first
     for (int u : by_level[l]) {
-      const size_t t = units[u].t;
-      const int m = units[u].m;
-      const Instr& in = code[t];
+      const std::vector<int>& ts = units[u].t;
+      const Instr& in = code[ts[0]];
       const Domain& dm = sys->doms[in.dom];
       kad::GroupOp op;
       double cost = 0.0;
+      if (units[u].cluster) {
+        op.kind = kad::GK_CLUSTER;
+        op.size = in.size;
+        op.step0 = (int)steps.size();
+        if (cluster_steps(code, ts, [&](int s) { return live[s] != 0; }, opnd, &steps) != ts.size()) return KAD_ERR_ARG;
+        op.nsteps = (int)steps.size() - op.step0;
+        int ntmp = 0;
+        for (int q = op.step0; q < (int)steps.size(); ++q) {
+          const kad::ClusterStep& s = steps[q];
+          ntmp = std::max({ntmp, s.ca + 1, s.cb + 1, s.d + 1});
+          bytes += 8.0 * in.size * ((s.a == -2 && s.ga.tan) + (s.b == -2 && s.gb.tan) + (s.gd.slot >= 0));
+        }
+        // elements per thread: as many as the array has, within 48 KB of temporaries
+        // (three workgroups per CU)
+        op.per = 4;
+        while (op.per > 1 && (ntmp * op.per > 24 || 128 * op.per >= in.size)) op.per /= 2;
+        lds = std::max(lds, (size_t)ntmp * op.per * 256 * sizeof(double));
+        lv.push_back({100.0 * op.nsteps * (double)kad::cdiv(in.size, 256), op});
+        continue;
+      }
       op.a = opnd(in.a);
+      const int m = (int)ts.size() - 1;
       op.nstep = m;
       for (int k = 0; k < m; ++k) {
-        const Instr& e = code[t + k + 1];
-        const int side = (e.a.space == SP_TAN && e.a.slot == code[t + k].dst.slot) ? 0 : 1;
+        const Instr& e = code[ts[k + 1]];
+        const int v = code[ts[k]].dst.slot;
+        const int side = (e.a.space == SP_TAN && e.a.slot == v) ? 0 : 1;
         op.st[k].kind = e.ew;
         op.st[k].side = side;
         op.st[k].o = opnd(side == 0 ? e.b : e.a);
         op.st[k].s = e.s;
       }
-      if (in.kind == I_LIN || in.kind == I_EW || in.kind == I_SEED) op.dst = opnd(code[t + m].dst);
+      if (!is_export(in)) op.dst = opnd(code[ts.back()].dst);
       int nout = in.size;
       switch (in.kind) {
         case I_LIN: {
           op.kind = kad::GK_LIN;
-          op.d0 = in.din[0];
-          op.d1 = in.din[1];
-          op.d2 = in.din[2];
-          op.P = plans[in.plan].P;
-          op.pool = plans[in.plan].pool;
-          const kad::Apply3dShape sh = kad::apply3d_shape(op.d0, op.d1, op.d2, op.P);
-          op.stage_pool = sh.stage_pool;
-          op.inplace = sh.inplace;
-          if (sh.lds > 160 * 1024) return KAD_ERR_ARG;
-          lds = std::max(lds, sh.lds);
-          int od[3] = {op.d0, op.d1, op.d2};
-          for (int p = 0; p < op.P.npass; ++p) od[op.P.axis[p]] = op.P.nout[p];
-          nout = od[0] * od[1] * od[2];
-          bytes += 8.0 * ((double)op.d0 * op.d1 * op.d2 + nout);
-          cost = 1e6 * op.P.npass + nout;
+          op.P = plans[in.plan];
+          lds = std::max(lds, kad::lines_lds(op.P));
+          nout = op.P.size_out;
+          bytes += 8.0 * ((double)op.P.size_in + nout);
+          cost = 2000.0 * op.P.npass + nout;
           break;
         }
         case I_EW:
@@ -1187,7 +1472,7 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
           op.s = in.s;
           op.b = opnd(in.b);
           bytes += 8.0 * in.size * (2.0 + (in.b.slot >= 0 ? 1.0 : 0.0));
-          cost = in.size;
+          cost = 0.1 * in.size;
           break;
         case I_SEED: {
           op.kind = kad::GK_SEED;
@@ -1196,7 +1481,7 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
           op.sval = seed_val[seed_tab];
           op.scnt = seed_cnt[seed_tab];
           op.nu = (int)sys->seeds[seed_tab].cnt.size();
-          cost = in.size;
+          cost = 0.1 * in.size;
           break;
         }
         case I_EXPORT_GL:
@@ -1210,7 +1495,7 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
           op.c0 = in.c0;
           op.accumulate = in.accumulate;
           op.pt = in.pt;
-          cost = 1e7;
+          cost = 1e6;
           break;
         default:
           op.kind = in.kind == I_EXPORT_BD ? kad::GK_EXPORT_BD : kad::GK_EXPORT_IN;
@@ -1244,6 +1529,7 @@ int kad_system_impl::group_round(const std::vector<GroupItem>& items, void* out,
                                  const double* w) {
   kad::GroupArgs g;
   g.ops = gops;
+  g.steps = gsteps;
   g.val = val_arena;
   g.tan = grp_arena;
   g.stride = stride;
@@ -1268,7 +1554,8 @@ int kad_system_impl::group_round(const std::vector<GroupItem>& items, void* out,
       // puts it on the same XCD (and its L2) at every level
       const int nbp = it.nb == 1 ? 1 : (int)kad::cdiv(it.nb, 8) * 8;
       if (nbp > 1) blocks = (int)kad::cdiv(blocks, 8) * 8;
-      g.e[n++] = {blocks, nops, p.op0 + p.lev[l], it.nb, nbp, it.u0, b0, it.col0};
+      g.blk0[n] = blocks;
+      g.e[n++] = {nops, p.op0 + p.lev[l], it.nb, nbp, it.u0, 0, b0, it.col0};
       blocks += nops * nbp;
       lds = std::max(lds, p.lds[l]);
       bytes += p.bytes[l] * it.nb;
@@ -1297,13 +1584,18 @@ int kad_system_impl::group_columns(std::vector<GroupItem> items, void* out, int6
       all += (size_t)p.nphys * stride;
       one = std::max(one, (size_t)p.nphys * stride);
     }
-    // 3 GiB: every column of a 9x7x4 system at once (0.9 GB; 2.64 ms per Jacobian, 4.24
-    // when only 32 MiB of columns run together), several thousand columns of the larger
-    // ones (J^T w at 13x9x8: 42, 37, 34.4, 33.5 ms with 0.5, 1, 3, 12 GiB)
-    const size_t budget = (size_t)3 << 27;  // doubles
-    const size_t cap = std::max(std::min(all, budget), 64 * one);
-    const int rc = dmalloc((void**)&grp_arena, cap * sizeof(double));
-    if (rc) return rc;
+    // 6 GiB: every column of a 9x7x4 system at once, thousands of columns of the larger
+    // ones (5001 columns at 17x13x12: 29.7, 25.7, 25.4 ms with 3, 6, 12 GiB; J^T w at
+    // 13x9x8: 32.7, 32.2, 32.4); less when the card has no room for it
+    const size_t least = 64 * one;
+    size_t cap = std::max(std::min(all, (size_t)6 << 27), least);
+    while (hipMalloc((void**)&grp_arena, cap * sizeof(double)) != hipSuccess) {
+      (void)hipGetLastError();
+      grp_arena = nullptr;
+      if (cap <= least) return KAD_ERR_HIP;
+      cap = std::max(cap / 2, least);
+    }
+    allocs.push_back(grp_arena);
     grp_cap = cap;
   }
   std::vector<GroupItem> round;
@@ -1383,8 +1675,8 @@ int kad_system_impl::jacobian(double* Jd, int64_t ldj) {
 int kad_system_impl::fill_columns(double* Jd, int64_t ldj) {
   // Programs of 2048 columns and more fill the chip with each instruction (8 workgroups
   // per CU); their launches on nfill streams overlap and keep an instruction's arrays
-  // closer together than a whole level's (17x13x12, 2397 columns per program: 0.139 s
-  // against 0.167 grouped; 13x9x8, 819 columns: 34 ms grouped against 62)
+  // closer together than a whole level's (17x13x12, 2397 columns per program: 0.134 s
+  // against 0.146 grouped; 13x9x8, 819 columns: 33 ms grouped against 62)
   const bool wide = (int64_t)sys->n_unknowns >= (int64_t)2048 * (int64_t)tprogs.size();
   if (gtan_ok && fuse_ew && !wide) return columns(0, sys->n_unknowns, 0, Jd, ldj);
   {

@@ -54,36 +54,25 @@ int get_plan(Ctx* c, int dir, int nr, int nt, int np, const int* base_r, const i
     fprintf(stderr, "[kadath_amd] transform plan: %s\n", e.what());
     return KAD_ERR_ARG;
   }
+  // phi, theta, r  (coef.cpp:100-101: d = ndim-1 .. 0) or r, theta, phi (coef_i.cpp:100-101)
+  kad::PassDesc pd[3] = {{2, dir == 0 ? npc : np, lp.data()}, {1, nt, lt.data()}, {0, nr, lr.data()}};
+  if (dir == 1) std::swap(pd[0], pd[2]);
   DevPlan* p = new DevPlan();
-  std::vector<int> lines;
-  lines.insert(lines.end(), lp.begin(), lp.end());
-  lines.insert(lines.end(), lt.begin(), lt.end());
-  lines.insert(lines.end(), lr.begin(), lr.end());
-  int rc = c->upload(pool.data(), pool.size() * sizeof(double), (void**)&p->pool);
-  if (!rc) rc = c->upload(lines.data(), lines.size() * sizeof(int), (void**)&p->lines);
+  std::vector<kad::LineEnt> tab((size_t)3 * nr * nt * npc);
+  size_t used = 0, toff[kad::MAX_PASSES];
+  kad::LineEnt* dt = nullptr;
+  int rc = kad::lines_build(nr, nt, dir == 0 ? np : npc, pd, 3, (int)pool.size(), p->P, tab.data(), tab.size(), &used,
+                            toff)
+               ? KAD_OK
+               : KAD_ERR_ARG;
+  if (!rc) rc = c->upload(pool.data(), pool.size() * sizeof(double), (void**)&p->pool);
+  if (!rc) rc = c->upload(tab.data(), used * sizeof(kad::LineEnt), (void**)&dt);
   if (rc) {
     delete p;
     return rc;
   }
-  const int* dlp = p->lines;
-  const int* dlt = p->lines + 1;
-  const int* dlr = p->lines + 1 + npc;
-  p->P.npass = 3;
-  p->P.maxsize = nr * nt * npc;
-  p->P.pool_size = (int)pool.size();
-  if (dir == 0) {  // phi, theta, r  (coef.cpp:100-101: d = ndim-1 .. 0)
-    p->P.axis[0] = 2; p->P.nout[0] = npc; p->P.line_mat[0] = dlp; p->P.nlines[0] = 1;
-    p->P.axis[1] = 1; p->P.nout[1] = nt;  p->P.line_mat[1] = dlt; p->P.nlines[1] = npc;
-    p->P.axis[2] = 0; p->P.nout[2] = nr;  p->P.line_mat[2] = dlr; p->P.nlines[2] = nt * npc;
-    p->d_in[0] = nr; p->d_in[1] = nt; p->d_in[2] = np;
-    p->d_out[0] = nr; p->d_out[1] = nt; p->d_out[2] = npc;
-  } else {  // r, theta, phi  (coef_i.cpp:100-101: d = 0 .. ndim-1)
-    p->P.axis[0] = 0; p->P.nout[0] = nr; p->P.line_mat[0] = dlr; p->P.nlines[0] = nt * npc;
-    p->P.axis[1] = 1; p->P.nout[1] = nt; p->P.line_mat[1] = dlt; p->P.nlines[1] = npc;
-    p->P.axis[2] = 2; p->P.nout[2] = np; p->P.line_mat[2] = dlp; p->P.nlines[2] = 1;
-    p->d_in[0] = nr; p->d_in[1] = nt; p->d_in[2] = npc;
-    p->d_out[0] = nr; p->d_out[1] = nt; p->d_out[2] = np;
-  }
+  p->P.pool = p->pool;
+  for (int q = 0; q < 3; ++q) p->P.p[q].tab = dt + toff[q];
   c->plans[key.str()] = p;
   *out = p;
   return KAD_OK;
@@ -108,15 +97,15 @@ int get_line_matrix(Ctx* c, int dir, int base, int nconf, const double** dM, int
       delete p;
       return rc;
     }
-    p->d_in[0] = M.nin;
-    p->d_out[0] = M.nout;
+    p->nin = M.nin;
+    p->nout = M.nout;
     c->plans[key.str()] = p;
   } else {
     p = it->second;
   }
   *dM = p->pool;
-  *nin = p->d_in[0];
-  *nout = p->d_out[0];
+  *nin = p->nin;
+  *nout = p->nout;
   return KAD_OK;
 }
 
@@ -136,8 +125,8 @@ int kad_coef_3d(kad_ctx* ctx, int nr, int nt, int np, const int* base_r, const i
   DevPlan* p;
   int rc = get_plan(c, 0, nr, nt, np, base_r, base_t, base_p, &p);
   if (rc) return rc;
-  return kad::apply3d_launch(conf, (int64_t)nr * nt * np, coef, (int64_t)nr * nt * (np + 2), nbatch, nr, nt, np, p->P,
-                             p->pool, 0, 1.0, c->stream);
+  return kad::apply3d_launch(conf, (int64_t)nr * nt * np, coef, (int64_t)nr * nt * (np + 2), nbatch, p->P,
+                             c->stream);
 }
 
 int kad_coef_i_3d(kad_ctx* ctx, int nr, int nt, int np, const int* base_r, const int* base_t, int base_p, int nbatch,
@@ -147,8 +136,8 @@ int kad_coef_i_3d(kad_ctx* ctx, int nr, int nt, int np, const int* base_r, const
   DevPlan* p;
   int rc = get_plan(c, 1, nr, nt, np, base_r, base_t, base_p, &p);
   if (rc) return rc;
-  return kad::apply3d_launch(coef, (int64_t)nr * nt * (np + 2), conf, (int64_t)nr * nt * np, nbatch, nr, nt, np + 2,
-                             p->P, p->pool, 0, 1.0, c->stream);
+  return kad::apply3d_launch(coef, (int64_t)nr * nt * (np + 2), conf, (int64_t)nr * nt * np, nbatch,
+                             p->P, c->stream);
 }
 
 int kad_coef_1d(kad_ctx* ctx, int base, int nconf, int64_t nlines, const double* conf, double* coef) {

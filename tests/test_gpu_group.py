@@ -3,9 +3,10 @@ columns of a group together) against the same programs run one instruction per l
 (set_option(fuse=False)): the operations and their order per element are the same, so F,
 J, its fp32 columns and J^T w must agree bit for bit.
 
-Sizes: smallest grids, odd and even line lengths on both sides of the 12..17 points that
-have line kernels, both unknown orders, a system with a double unknown and integral
-equation, and column ranges that start and end inside a program."""
+Sizes: smallest grids, odd and even line lengths, arrays of few outputs (a thread each)
+and of many (a thread per line), element-wise regions of one and of several elements per
+thread, both unknown orders, a system with a double unknown and integral equation, and
+column ranges that start and end inside a program."""
 import numpy as np
 import pytest
 import torch

@@ -65,3 +65,26 @@ def test_domain_3d(ctx, shape, anti):
     np.testing.assert_allclose(got, cfs, atol=1e-12)
     back = ctx.coef_i_3d(torch.tensor(cfs, device="cuda"), br, bt, bp).cpu().numpy()
     np.testing.assert_allclose(back, vals, atol=1e-12)
+
+
+# both sides of every line of the passes' dispatch: 768 outputs (a thread each), lines of up
+# to 6, 10, 14 and 18 points in registers and longer ones, one to five groups of 64 lines, one
+# LDS buffer (256 lines at most, or passes that keep the line length) and two
+@pytest.mark.parametrize("shape", [(5, 5, 4), (9, 7, 10), (11, 7, 8), (17, 11, 8), (17, 17, 8), (13, 15, 16),
+                                   (15, 13, 14), (7, 17, 12), (19, 5, 4), (9, 19, 12), (5, 9, 20)])
+def test_pass_edges(ctx, shape):
+    nr, nt, npt = shape
+    print(f"pass edges {shape}", flush=True)
+    rng = np.random.default_rng(7 * nr + nt + npt)
+    br, bt, bp = S.std_base(nt, npt, False)
+    nb = 3
+    confs = rng.uniform(-1, 1, (nb, npt, nt, nr))
+    cfs = np.stack([S.coef_3d(confs[b], br, bt, bp) for b in range(nb)])
+    vals = np.stack([S.coef_i_3d(cfs[b], br, bt, bp) for b in range(nb)])
+    # three passes of sums over at most max(shape) + 2 products; every partial result is at most
+    # the sum of |coefficients|
+    atol = 3 * (max(shape) + 2) * 2.0**-52 * max(1.0, np.abs(cfs).sum(axis=(1, 2, 3)).max())
+    got = ctx.coef_3d(torch.tensor(vals, device="cuda"), br, bt, bp).cpu().numpy()
+    np.testing.assert_allclose(got, cfs, rtol=0, atol=atol)
+    back = ctx.coef_i_3d(torch.tensor(cfs, device="cuda"), br, bt, bp).cpu().numpy()
+    np.testing.assert_allclose(back, vals, rtol=0, atol=atol)
