@@ -7,8 +7,13 @@
 // All operands column-major with leading dimensions, as the dense Jacobian is
 // stored (the reference packs J column-major for pdgesv, do_newton.cpp:178-185).
 //
-// Tile: 128x128 per workgroup, 4 waves in a 2x2 grid, each wave 64x64 = 4x4
-// MFMA 16x16 tiles.  K is staged through LDS with register double buffering.
+// Tile (f64, f32): 128x128 per workgroup, 8 waves in a 2x4 grid, each wave 64x32 = 4x2
+// MFMA 16x16 tiles (bf16: 4 waves of 64x64).  K is staged through LDS with register double
+// buffering.  Bound by the matrix cores in the k loop (62.6 TFLOP/s at k = 1024 in f64)
+// and by each tile's first loads and its reading of C around it.  With 4 waves of 64x64 a
+// SIMD held two waves; the four of 8 waves hide more of that: C -= AB with k = 256 took 760
+// us at 8191 x 7935, now 694 (f32 460 and 401), at 12032 x 12032 1460 and 1438 (f32 891,
+// 848).
 // The MFMA is issued with the roles of A and B swapped (D' = B^T A^T = C^T), so
 // lanes 0..15 of an accumulator register hold 16 consecutive ROWS of one column
 // of C: the column-major epilogue is coalesced.
@@ -19,6 +24,7 @@
 namespace kad {
 
 constexpr int GBM = 128, GBN = 128, GNT = 256;
+constexpr int gemm_threads(int bm) { return bm == 64 ? 256 : 512; }  // of gemm_k4_kernel
 constexpr int OP_SUB = 0, OP_SET = 1;
 
 template <int P> struct GemmCfg;
@@ -75,9 +81,9 @@ __device__ inline bool select_tile(const TileSel& sel, int nbm, int nbn, int& tm
   }
   return true;
 }
-template <typename T, int BM = GBM>
+template <typename T, int BM = GBM, int NT = GNT>
 __device__ inline void zero_tile(T* C, int64_t ldc, int m, int n, int row0, int col0, int tid) {
-  for (int e = tid; e < BM * BM; e += GNT) {
+  for (int e = tid; e < BM * BM; e += NT) {
     const int r = row0 + e % BM, c = col0 + e / BM;
     if (r < m && c < n) C[r + (int64_t)c * ldc] = T(0);
   }
@@ -86,11 +92,11 @@ __device__ inline void zero_tile(T* C, int64_t ldc, int m, int n, int row0, int 
 // ---------------------------------------------------------------------------
 // f64 / f32 path: 16x16x4 MFMA, LDS tiles stored k-major: As[k][m], Bs[k][n].
 // ---------------------------------------------------------------------------
-// BM x BM tile per workgroup (BM = 128: the bulk updates; BM = 64: small and narrow
+// BM x BM tile per workgroup (BM = 128, 512 threads: the bulk updates; BM = 64, 256 threads: small and narrow
 // products -- 4x the workgroups, and at most ~100 VGPRs and 35 KB of LDS, so they run
 // beside the bulk update's 128-tiles on the same CUs instead of queueing behind them).
 template <int P, int OP, int BM = GBM>
-__global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
+__global__ __launch_bounds__(gemm_threads(BM), BM == 64 ? 1 : 4) void gemm_k4_kernel(int m, int n, int k,
                                                       const typename GemmCfg<P>::T* __restrict__ A, int64_t lda,
                                                       const typename GemmCfg<P>::T* __restrict__ B, int64_t ldb,
                                                       typename GemmCfg<P>::T* __restrict__ C, int64_t ldc,
@@ -102,9 +108,11 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
   constexpr int BK = GemmCfg<P>::BK;
   constexpr int PADA = (sizeof(T) == 8) ? 4 : 8;
   constexpr int LDA_S = BM + PADA, LDB_S = BM + PADA;
-  constexpr int NA = BM * BK / GNT;  // elements of A per thread per stage
-  constexpr int NB = BM * BK / GNT;
-  constexpr int WT = BM / 2, TI = WT / 16;  // wave tile and its 16x16 MFMA tiles per side
+  constexpr int NT = gemm_threads(BM);
+  constexpr int NA = BM * BK / NT;  // elements of A per thread per stage
+  constexpr int NB = BM * BK / NT;
+  // wave tile (64x32 or 32x32) and its 16x16 MFMA tiles per side
+  constexpr int WM = BM / 2, WN = 32, TI = WM / 16, TJ = WN / 16;
   using acc_t = typename std::conditional<sizeof(T) == 8, d4v, f4v>::type;
   A += (int64_t)blockIdx.z * sel.sa;
   B += (int64_t)blockIdx.z * sel.sb;
@@ -119,17 +127,17 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
   const bool active = select_tile<BM>(sel, nbm, nbn, tm, tn, zero_fill);
   const int row0 = tm * BM, col0 = tn * BM;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  const int wm = (wave & 1) * WT, wn = (wave >> 1) * WT;
+  const int wm = (wave & 1) * WM, wn = (wave >> 1) * WN;
   if (!active) {
-    if (OP == OP_SET && zero_fill) zero_tile<T, BM>(C, ldc, m, n, row0, col0, tid);
+    if (OP == OP_SET && zero_fill) zero_tile<T, BM, NT>(C, ldc, m, n, row0, col0, tid);
     return;
   }
 
-  acc_t acc[TI][TI];
+  acc_t acc[TI][TJ];
 #pragma unroll
   for (int i = 0; i < TI; ++i)
 #pragma unroll
-    for (int j = 0; j < TI; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
+    for (int j = 0; j < TJ; ++j) acc[i][j] = acc_t{0, 0, 0, 0};
 
   // The k loop, with bounds checks on the loads only for tiles at the matrix's edge
   // (EDGE) or a k that is not a whole number of steps.  Inside the matrix the loop is
@@ -142,7 +150,7 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
     auto gload = [&](int k0) {
 #pragma unroll
       for (int e = 0; e < NA; ++e) {
-        const int idx = tid + e * GNT;
+        const int idx = tid + e * NT;
         const int r = idx % BM, kk = idx / BM;
         const int gr = row0 + r, gk = k0 + kk;
         if constexpr (EDGE) {
@@ -157,7 +165,7 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
       }
 #pragma unroll
       for (int e = 0; e < NB; ++e) {
-        const int idx = tid + e * GNT;
+        const int idx = tid + e * NT;
         const int kk = idx % BK, c = idx / BK;
         const int gk = k0 + kk, gc = col0 + c;
         if constexpr (EDGE) {
@@ -165,21 +173,21 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
         } else {
           // scalar base for the element's column group, lane offset kk + (c - c_e) ldb
           const int k0c = min(k0, k - BK);  // the last step's prefetch re-reads the last step
-          const int ce = col0 + e * (GNT / BK);
+          const int ce = col0 + e * (NT / BK);
           const T* base = B + k0c + (int64_t)ce * ldb;
-          rb[e] = base[kk + (c - e * (GNT / BK)) * (int)ldb];
+          rb[e] = base[kk + (c - e * (NT / BK)) * (int)ldb];
         }
       }
     };
     auto sstore = [&](int buf) {
 #pragma unroll
       for (int e = 0; e < NA; ++e) {
-        const int idx = tid + e * GNT;
+        const int idx = tid + e * NT;
         As[buf][(idx / BM) * LDA_S + (idx % BM)] = ra[e];
       }
 #pragma unroll
       for (int e = 0; e < NB; ++e) {
-        const int idx = tid + e * GNT;
+        const int idx = tid + e * NT;
         Bs[buf][(idx % BK) * LDB_S + (idx / BK)] = rb[e];
       }
     };
@@ -197,16 +205,15 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
 #pragma unroll
       for (int kk = 0; kk < BK; kk += 4) {
         const int kr = kk + (lane >> 4);
-        T af[TI], bf[TI];
+        T af[TI], bf[TJ];
 #pragma unroll
-        for (int t = 0; t < TI; ++t) {
-          af[t] = as[kr * LDA_S + wm + t * 16 + (lane & 15)];
-          bf[t] = bs[kr * LDB_S + wn + t * 16 + (lane & 15)];
-        }
+        for (int t = 0; t < TI; ++t) af[t] = as[kr * LDA_S + wm + t * 16 + (lane & 15)];
+#pragma unroll
+        for (int t = 0; t < TJ; ++t) bf[t] = bs[kr * LDB_S + wn + t * 16 + (lane & 15)];
 #pragma unroll
         for (int i = 0; i < TI; ++i)
 #pragma unroll
-          for (int j = 0; j < TI; ++j) {
+          for (int j = 0; j < TJ; ++j) {
             if constexpr (sizeof(T) == 8)
               acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(bf[j], af[i], acc[i][j], 0, 0, 0);
             else
@@ -232,12 +239,12 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
   if (row0 + BM <= m && col0 + BM <= n) {
 #pragma unroll
     for (int h = 0; h < TI; h += TI / 2) {
-      T cv[TI / 2][TI][4];
+      T cv[TI / 2][TJ][4];
       if constexpr (OP == OP_SUB) {
 #pragma unroll
         for (int i = 0; i < TI / 2; ++i)
 #pragma unroll
-          for (int j = 0; j < TI; ++j)
+          for (int j = 0; j < TJ; ++j)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
               const int gr = row0 + wm + (h + i) * 16 + (lane & 15);
@@ -248,7 +255,7 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
 #pragma unroll
       for (int i = 0; i < TI / 2; ++i)
 #pragma unroll
-        for (int j = 0; j < TI; ++j)
+        for (int j = 0; j < TJ; ++j)
 #pragma unroll
           for (int r = 0; r < 4; ++r) {
             const int gr = row0 + wm + (h + i) * 16 + (lane & 15);
@@ -263,7 +270,7 @@ __global__ __launch_bounds__(GNT) void gemm_k4_kernel(int m, int n, int k,
     const int gr = row0 + wm + i * 16 + (lane & 15);
     if (gr >= m) continue;
 #pragma unroll
-    for (int j = 0; j < TI; ++j) {
+    for (int j = 0; j < TJ; ++j) {
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
         const int gc = col0 + wn + j * 16 + (sizeof(T) == 8 ? 4 * r + (lane >> 4) : 4 * (lane >> 4) + r);
@@ -480,7 +487,8 @@ int gemm_launch_sel(int prec, int op, int m, int n, int k, const void* A, int64_
   const int nblocks = (int)(cdiv(m, GBM) * cdiv(n, GBN));
   // fewer 128-tiles than two per CU (and not a compacted tile list): 64-tiles
   const bool small = !sel.cnt && prec != BF16 && (int64_t)nblocks * sel.nbat < 512;
-  dim3 grid(small ? (unsigned)(cdiv(m, 64) * cdiv(n, 64)) : (unsigned)nblocks, 1, (unsigned)sel.nbat), block(GNT);
+  dim3 grid(small ? (unsigned)(cdiv(m, 64) * cdiv(n, 64)) : (unsigned)nblocks, 1, (unsigned)sel.nbat),
+      block(prec == BF16 ? GNT : gemm_threads(small ? 64 : 128));
   GemmTimer* tm = g_gemm_timer;
   bool timed = false;
   if (tm) {
