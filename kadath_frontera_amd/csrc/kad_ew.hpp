@@ -22,6 +22,25 @@ __device__ __forceinline__ double ew_op(int kind, double x, double y, double s) 
   }
 }
 
+// The operation on U elements, decoded once.
+template <int U>
+__device__ __forceinline__ void ew_ops(int kind, double (&x)[U], const double (&y)[U], double s) {
+  auto all = [&](auto f) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) x[u] = f(x[u], y[u]);
+  };
+  switch (kind) {
+    case EWOP_ADD: all([](double p, double q) { return p + q; }); break;
+    case EWOP_SUB: all([](double p, double q) { return p - q; }); break;
+    case EWOP_MUL: all([](double p, double q) { return p * q; }); break;
+    case EWOP_DIV: all([](double p, double q) { return p / q; }); break;
+    case EWOP_SCAL: all([&](double p, double) { return p * s; }); break;
+    case EWOP_SDIV: all([&](double p, double) { return p / s; }); break;
+    case EWOP_ADDS: all([&](double p, double) { return p + s; }); break;
+    default: break;
+  }
+}
+
 // A chain of element-wise instructions applied to a value v as it is stored, each to
 // the previous one's result: step k makes v = op(v, o[b][e]) (side 0) or op(o[b][e], v)
 // (side 1), o its other operand (NULL: none; stride 0: one array for the whole batch).

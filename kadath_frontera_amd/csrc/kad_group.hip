@@ -3,8 +3,8 @@
 // A traced program is a few hundred to a few thousand instructions on small arrays, but
 // its dependency depth is about 32: run one launch per instruction, a residual at 9x7x4
 // is 2004 dependent launches of a single workgroup each.  Here one launch executes every
-// instruction of a dependency level, over all columns of every program in the group,
-// one workgroup per (instruction, column); the instruction is read from a device table
+// instruction of a dependency level, over all columns of every program in the group
+// (element-wise regions by a second one), one workgroup per (instruction, column); the instruction is read from a device table
 // with scalar loads (the workgroup's index is uniform), so all its branches are uniform.
 // Instructions of one level never touch the same memory, and the launch boundary orders
 // the levels.  The operations are those of the per-instruction kernels, in the same
@@ -25,9 +25,11 @@ struct Where {
   double* tan;
   int64_t stride;
   int nb, b;
+  // (32-bit factors: the arrays of an arena are fewer than 2^31, an array has fewer elements)
   template <typename O>
   __device__ __forceinline__ double* at(const O& o) const {
-    return o.tan ? tan + ((int64_t)o.slot * nb + b) * stride : val + (int64_t)o.slot * stride;
+    const unsigned n = o.tan ? (unsigned)o.slot * (unsigned)nb + (unsigned)b : (unsigned)o.slot;
+    return (o.tan ? tan : val) + (uint64_t)n * (unsigned)stride;
   }
 };
 
@@ -51,68 +53,81 @@ __device__ __forceinline__ double row_value(const DevRow R, const double* x, boo
   return v;
 }
 
-// An element-wise region of the program: every array it needs from outside is read once
-// (or kept in a temporary), its intermediate values live in LDS temporaries
-// (lds[temporary][element of the thread][thread]), only what other instructions read is
-// stored.  U elements per thread and 8 / U steps have their array operands loaded
-// together: one at a time, a step waited out a memory latency and the decoding of the
-// next one (1900 cycles per step of 256 elements).  Bound by that latency and by the few
-// workgroups that the temporaries' LDS leaves per CU: J^T w at 13x9x8 moves 66 GB at 2.05
-// TB/s.  One instruction at a time it moved more arrays through memory: 34.2 ms, 31.8 now;
-// 5001 fp32 columns at 17x13x12 36.4 and 25.3.
+// An element-wise region of the program, U elements per lane from element e0: every array
+// it needs from outside is read once (or kept in a temporary), its intermediate values live
+// in registers (temporary d of element u is entry d of t[u], addressed through the register
+// index), only what other instructions read is stored.  The array operands of the next Q
+// steps are loaded while Q steps run.  Bound by instruction issue (about 150 instructions per
+// step and wave, 2/3 of them decoding and register indexing) and, 44% of a wave's time, by
+// the loads; hence four elements per lane, one decoding for them, and no partly filled
+// sweeps.  With one element per lane and the temporaries in LDS J^T w at 13x9x8 took 31.8 ms
+// and 5001 fp32 columns at 17x13x12 25.4, now 26.8 and 21.7 (27.4 and 22.2 with 15
+// temporaries and two waves per SIMD).
 template <int U>
-__device__ __forceinline__ void cluster_body(const GroupArgs& g, const Where& at, const COp& op, double* lds, int tid) {
+__device__ __forceinline__ void cluster_body(const GroupArgs& g, const Where& at, const COp& op, int e0) {
+  typedef double Temps __attribute__((ext_vector_type(kClusterTemps + 1)));
   const int size = op.size, n = op.nsteps;
   const CStep* const st = (const CStep*)g.steps + op.step0;
-  constexpr int Q = 8 / U > 4 ? 4 : 8 / U;
-  for (int e0 = 0; e0 < size; e0 += 256 * U) {
-    double ga[Q][U], gb[Q][U];
-    auto load = [&](int i0) {
+  constexpr int Q = 2;
+  Temps t[U];
 #pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        if (i0 + i < n) {
-          if (st[i0 + i].a == -2) {
-            const double* const p = at.at(st[i0 + i].ga);
+  for (int u = 0; u < U; ++u) t[u] = Temps(0.0);
+  unsigned at_e[U];
 #pragma unroll
-            for (int u = 0; u < U; ++u) ga[i][u] = p[min(e0 + u * 256 + tid, size - 1)];
-          }
-          if (st[i0 + i].b == -2) {
-            const double* const p = at.at(st[i0 + i].gb);
+  for (int u = 0; u < U; ++u) at_e[u] = min(e0 + u * 64, size - 1);
+  double ga[Q][U], gb[Q][U];
+  auto load = [&](int i0) {
 #pragma unroll
-            for (int u = 0; u < U; ++u) gb[i][u] = p[min(e0 + u * 256 + tid, size - 1)];
-          }
+    for (int i = 0; i < Q; ++i) {
+      if (i0 + i < n) {
+        if (st[i0 + i].a == -2) {
+          const double* const p = at.at(st[i0 + i].ga);
+#pragma unroll
+          for (int u = 0; u < U; ++u) ga[i][u] = p[at_e[u]];
+        }
+        if (st[i0 + i].b == -2) {
+          const double* const p = at.at(st[i0 + i].gb);
+#pragma unroll
+          for (int u = 0; u < U; ++u) gb[i][u] = p[at_e[u]];
         }
       }
-    };
-    load(0);
-    for (int i0 = 0; i0 < n; i0 += Q) {
-      double ca_[Q][U], cb_[Q][U];
+    }
+  };
+  load(0);
+  for (int i0 = 0; i0 < n; i0 += Q) {
+    double xa[Q][U], xb[Q][U];
 #pragma unroll
-      for (int i = 0; i < Q; ++i)
+    for (int i = 0; i < Q; ++i)
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          ca_[i][u] = ga[i][u];
-          cb_[i][u] = gb[i][u];
-        }
-      load(i0 + Q);  // the next steps' operands, while these run
+      for (int u = 0; u < U; ++u) {
+        xa[i][u] = ga[i][u];
+        xb[i][u] = gb[i][u];
+      }
+    load(i0 + Q);  // the next steps' operands, while these run
 #pragma unroll
-      for (int i = 0; i < Q; ++i) {
-        if (i0 + i >= n) break;
-        const CStep& s = st[i0 + i];
-        const int a = s.a, b = s.b, ca = s.ca, cb = s.cb, d = s.d, kind = s.kind;
-        double* const out = s.gd.slot >= 0 ? at.at(s.gd) : nullptr;
-        const double sc = s.s;
+    for (int i = 0; i < Q; ++i) {
+      if (i0 + i >= n) break;
+      const CStep& s = st[i0 + i];
+      const int a = s.a, b = s.b;
+      // unconditional register accesses (temporary kClusterTemps takes what nothing reads):
+      // with a branch around each, the compiler selected between copies of all temporaries
+      const int ca = s.ca, cb = s.cb, d = s.d;
+      double x[U], y[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-          double* const l = lds + u * 256 + tid;
-          if (ca >= 0) l[ca * 256 * U] = ca_[i][u];
-          if (cb >= 0) l[cb * 256 * U] = cb_[i][u];
-          const double x = a >= 0 ? l[a * 256 * U] : ca_[i][u];
-          const double y = b >= 0 ? l[b * 256 * U] : cb_[i][u];
-          const double r = ew_op(kind, x, y, sc);
-          if (d >= 0) l[d * 256 * U] = r;
-          if (out && e0 + u * 256 + tid < size) out[e0 + u * 256 + tid] = r;
-        }
+      for (int u = 0; u < U; ++u) {
+        t[u][ca] = xa[i][u];
+        t[u][cb] = xb[i][u];
+        x[u] = a < 0 ? xa[i][u] : t[u][a < 0 ? 0 : a];
+        y[u] = b < 0 ? xb[i][u] : t[u][b < 0 ? 0 : b];
+      }
+      ew_ops<U>(s.kind, x, y, s.s);
+#pragma unroll
+      for (int u = 0; u < U; ++u) t[u][d] = x[u];
+      if (s.gd.slot >= 0) {
+        double* const out = at.at(s.gd);
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+          if (e0 + u * 64 < size) out[at_e[u]] = x[u];
       }
     }
   }
@@ -125,18 +140,40 @@ __device__ __forceinline__ void put_row(void* out, int64_t at, int acc, double v
 }
 }  // namespace
 
-__global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
-  extern __shared__ double lds[];
-  const int bid = blockIdx.x, tid = threadIdx.x;
-  int q = 0, blk = 0;
+// The entry of this workgroup and its place in it.
+__device__ __forceinline__ void group_entry(const GroupArgs& g, int& q, int& oi, int& b) {
+  int blk = 0;
+  q = 0;
 #pragma unroll
   for (int i = 1; i < kGroupEntries; ++i)
-    if (i < g.nent && bid >= g.blk0[i]) {
+    if (i < g.nent && (int)blockIdx.x >= g.blk0[i]) {
       q = i;
       blk = g.blk0[i];
     }
-  const int loc = bid - blk, nbp = g.e[q].nbp;
-  const int oi = loc / nbp, b = loc - oi * nbp;
+  const int loc = blockIdx.x - blk, nbp = g.e[q].nbp;
+  oi = loc / nbp;
+  b = loc - oi * nbp;
+}
+
+// The element-wise regions of a level, in a launch of their own, a wave per
+// kClusterChunk elements of (region, column): their temporaries leave three waves per SIMD,
+// the passes have five.
+__global__ __launch_bounds__(64, 3) void cluster_kernel(GroupArgs g) {
+  int q, oi, b;
+  group_entry(g, q, oi, b);
+  const int nch = g.e[q].nch, op_i = oi / nch, e0 = (oi - op_i * nch) * kClusterChunk;
+  if (op_i >= g.e[q].nops || b >= g.e[q].nb) return;  // padding
+  const COp& op = *((COp*)g.ops + g.e[q].op0 + op_i);
+  if (e0 >= op.size) return;
+  const Where at{g.val, g.tan + g.e[q].base, g.stride, g.e[q].nb, b};
+  cluster_body<kClusterChunk / 64>(g, at, op, e0 + threadIdx.x);
+}
+
+__global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
+  extern __shared__ double lds[];
+  const int tid = threadIdx.x;
+  int q, oi, b;
+  group_entry(g, q, oi, b);
   if (oi >= g.e[q].nops || b >= g.e[q].nb) return;  // padding
   const COp& op = *((COp*)g.ops + g.e[q].op0 + oi);
   const Where at{g.val, g.tan + g.e[q].base, g.stride, g.e[q].nb, b};
@@ -180,13 +217,6 @@ __global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
         if (e < size) post.dst[e] = post_ops(post, ew_op(ew, xv[u], yv[u], s), o[u]);
       }
     }
-    return;
-  }
-  if (kind == GK_CLUSTER) {
-    // few temporaries leave LDS for more elements per thread
-    if (op.per == 4) cluster_body<4>(g, at, op, lds, tid);
-    else if (op.per == 2) cluster_body<2>(g, at, op, lds, tid);
-    else cluster_body<1>(g, at, op, lds, tid);
     return;
   }
   if (kind == GK_SEED) {
@@ -259,10 +289,11 @@ __global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
   }
 }
 
-int group_launch(const GroupArgs& g, int blocks, size_t lds, hipStream_t s) {
+int group_launch(const GroupArgs& g, int blocks, bool clusters, size_t lds, hipStream_t s) {
   if (blocks <= 0) return KAD_OK;
   if (g.nent < 1 || g.nent > kGroupEntries || lds > 160 * 1024) return KAD_ERR_ARG;
-  group_kernel<<<blocks, 256, lds, s>>>(g);
+  if (clusters) cluster_kernel<<<blocks, 64, 0, s>>>(g);
+  else group_kernel<<<blocks, 256, lds, s>>>(g);
   KAD_HIP_CHECK(hipGetLastError());
   return KAD_OK;
 }

@@ -26,7 +26,9 @@ struct GroupStep {
 // One element-wise instruction of a cluster, in execution order.  Operand a / b: a
 // temporary (>= 0), none (-1), or an array (-2: ga / gb), kept in temporary ca / cb when
 // that is >= 0.  The result goes to temporary d (>= 0) and to array gd (slot >= 0).
-constexpr int kClusterTemps = 20;
+// In the device table ca, cb and d are kClusterTemps where there is none.
+constexpr int kClusterTemps = 7;
+constexpr int kClusterChunk = 256;  // elements of a wave
 struct ClusterStep {
   int kind = 0, a = -1, b = -1, ca = -1, cb = -1, d = -1;
   GroupOpnd ga, gb, gd;
@@ -41,7 +43,7 @@ struct GroupOp {
   GroupOpnd dst, a, b;
   double s = 0.0;                       // EW scalar; EXPORT_GL: factor
   GroupStep st[kMaxChain];
-  int step0 = 0, nsteps = 0, per = 1;   // CLUSTER: its steps in the step table, elements per thread
+  int step0 = 0, nsteps = 0;            // CLUSTER: its steps in the step table
   LinePlan P;                           // LIN
   // exports
   const DevRow* rows = nullptr;
@@ -60,7 +62,7 @@ struct GroupOp {
 // nbp >= nb columns each), tangent slot s of column b at base + (s nb + b) stride,
 // results in column col0 + b.
 struct GroupEntry {
-  int nops, op0, nb, nbp, u0, pad;
+  int nops, op0, nb, nbp, u0, nch;
   int64_t base, col0;
 };
 constexpr int kGroupEntries = 32;
@@ -79,6 +81,7 @@ struct GroupArgs {
   GroupEntry e[kGroupEntries];
 };
 
-int group_launch(const GroupArgs& g, int blocks, size_t lds, hipStream_t s);
+// clusters: every instruction of the launch is a CLUSTER, otherwise none is
+int group_launch(const GroupArgs& g, int blocks, bool clusters, size_t lds, hipStream_t s);
 
 }  // namespace kad

@@ -416,6 +416,8 @@ struct GroupProg {
   bool ok = false;             // false: the program runs instruction by instruction
   int op0 = 0, nphys = 0;      // nphys: tangent slots of one column
   std::vector<int> lev;
+  std::vector<int> ncl;        // per level: clusters among them (the last ones)
+  std::vector<int> clsize;     // per level: elements of the largest cluster
   std::vector<size_t> lds;     // per level: the most LDS of an instruction
   std::vector<double> bytes;   // per level: algorithmic HBM bytes of one column (passes and element-wise)
 };
@@ -1427,17 +1429,12 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
         op.step0 = (int)steps.size();
         if (cluster_steps(code, ts, [&](int s) { return live[s] != 0; }, opnd, &steps) != ts.size()) return KAD_ERR_ARG;
         op.nsteps = (int)steps.size() - op.step0;
-        int ntmp = 0;
         for (int q = op.step0; q < (int)steps.size(); ++q) {
-          const kad::ClusterStep& s = steps[q];
-          ntmp = std::max({ntmp, s.ca + 1, s.cb + 1, s.d + 1});
+          kad::ClusterStep& s = steps[q];
+          for (int* w : {&s.ca, &s.cb, &s.d})
+            if (*w < 0) *w = kad::kClusterTemps;
           bytes += 8.0 * in.size * ((s.a == -2 && s.ga.tan) + (s.b == -2 && s.gb.tan) + (s.gd.slot >= 0));
         }
-        // elements per thread: as many as the array has, within 48 KB of temporaries
-        // (three workgroups per CU)
-        op.per = 4;
-        while (op.per > 1 && (ntmp * op.per > 24 || 128 * op.per >= in.size)) op.per /= 2;
-        lds = std::max(lds, (size_t)ntmp * op.per * 256 * sizeof(double));
         lv.push_back({100.0 * op.nsteps * (double)kad::cdiv(in.size, 256), op});
         continue;
       }
@@ -1513,8 +1510,19 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
       for (int k = 0; k < m; ++k) bytes += op.st[k].o.tan ? 8.0 * nout : 0.0;
       lv.push_back({cost, op});
     }
-    std::stable_sort(lv.begin(), lv.end(), [](const auto& x, const auto& y) { return x.first > y.first; });
-    for (auto& x : lv) ops.push_back(x.second);
+    std::stable_sort(lv.begin(), lv.end(), [](const auto& x, const auto& y) {
+      const bool cx = x.second.kind == kad::GK_CLUSTER, cy = y.second.kind == kad::GK_CLUSTER;
+      return cx != cy ? cy : x.first > y.first;  // the clusters last
+    });
+    int ncl = 0, clsize = 0;
+    for (auto& x : lv) {
+      ops.push_back(x.second);
+      if (x.second.kind != kad::GK_CLUSTER) continue;
+      ++ncl;
+      clsize = std::max(clsize, x.second.size);
+    }
+    gp.ncl.push_back(ncl);
+    gp.clsize.push_back(clsize);
     gp.lev.push_back((int)ops.size() - gp.op0);
     gp.lds.push_back(lds);
     gp.bytes.push_back(bytes);
@@ -1540,32 +1548,37 @@ int kad_system_impl::group_round(const std::vector<GroupItem>& items, void* out,
   size_t depth = 0;
   for (const GroupItem& it : items) depth = std::max(depth, it.p->lds.size());
   for (size_t l = 0; l < depth; ++l) {
-    int blocks = 0, n = 0;
-    size_t lds = 0;
-    int64_t base = 0;
     double bytes = 0.0;
-    for (const GroupItem& it : items) {
-      const GroupProg& p = *it.p;
-      const int64_t b0 = base;
-      base += (int64_t)p.nphys * it.nb * stride;
-      if (l >= p.lds.size()) continue;
-      const int nops = p.lev[l + 1] - p.lev[l];
-      // a column's workgroups keep their residue modulo 8, so the round-robin dispatch
-      // puts it on the same XCD (and its L2) at every level
-      const int nbp = it.nb == 1 ? 1 : (int)kad::cdiv(it.nb, 8) * 8;
-      if (nbp > 1) blocks = (int)kad::cdiv(blocks, 8) * 8;
-      g.blk0[n] = blocks;
-      g.e[n++] = {nops, p.op0 + p.lev[l], it.nb, nbp, it.u0, 0, b0, it.col0};
-      blocks += nops * nbp;
-      lds = std::max(lds, p.lds[l]);
-      bytes += p.bytes[l] * it.nb;
-    }
-    g.nent = n;
+    for (const GroupItem& it : items) bytes += l < it.p->lds.size() ? it.p->bytes[l] * it.nb : 0.0;
     kad::GemmTimer* tm = kad::g_apply_timer;
     const int trc = tm && bytes > 0.0 ? tm->begin(ctx->stream, bytes) : 1;
     if (trc < 0) return trc;
-    const int rc = kad::group_launch(g, blocks, lds, ctx->stream);
-    if (rc) return rc;
+    for (const bool clusters : {false, true}) {
+      int blocks = 0, n = 0;
+      size_t lds = 0;
+      int64_t base = 0;
+      for (const GroupItem& it : items) {
+        const GroupProg& p = *it.p;
+        const int64_t b0 = base;
+        base += (int64_t)p.nphys * it.nb * stride;
+        if (l >= p.lds.size()) continue;
+        const int first = clusters ? p.lev[l + 1] - p.ncl[l] : p.lev[l];
+        const int nops = (clusters ? p.lev[l + 1] : p.lev[l + 1] - p.ncl[l]) - first;
+        if (nops == 0) continue;
+        // a column's workgroups keep their residue modulo 8, so the round-robin dispatch
+        // puts it on the same XCD (and its L2) at every level
+        const int nbp = it.nb == 1 ? 1 : (int)kad::cdiv(it.nb, 8) * 8;
+        if (nbp > 1) blocks = (int)kad::cdiv(blocks, 8) * 8;
+        g.blk0[n] = blocks;
+        const int nch = clusters ? (int)kad::cdiv(p.clsize[l], kad::kClusterChunk) : 1;
+        g.e[n++] = {nops, p.op0 + first, it.nb, nbp, it.u0, nch, b0, it.col0};
+        blocks += nops * nch * nbp;
+        lds = std::max(lds, p.lds[l]);
+      }
+      g.nent = n;
+      const int rc = kad::group_launch(g, blocks, clusters, lds, ctx->stream);
+      if (rc) return rc;
+    }
     if (trc == 0 && tm->end(ctx->stream)) return KAD_ERR_HIP;
   }
   return KAD_OK;
@@ -1585,8 +1598,9 @@ int kad_system_impl::group_columns(std::vector<GroupItem> items, void* out, int6
       one = std::max(one, (size_t)p.nphys * stride);
     }
     // 6 GiB: every column of a 9x7x4 system at once, thousands of columns of the larger
-    // ones (5001 columns at 17x13x12: 29.7, 25.7, 25.4 ms with 3, 6, 12 GiB; J^T w at
-    // 13x9x8: 32.7, 32.2, 32.4); less when the card has no room for it
+    // ones (with the regions' temporaries in LDS, 5001 columns at 17x13x12 took 29.7, 25.7,
+    // 25.4 ms with 3, 6, 12 GiB, J^T w at 13x9x8 32.7, 32.2, 32.4); less when the card has
+    // no room for it
     const size_t least = 64 * one;
     size_t cap = std::max(std::min(all, (size_t)6 << 27), least);
     while (hipMalloc((void**)&grp_arena, cap * sizeof(double)) != hipSuccess) {
@@ -1675,8 +1689,8 @@ int kad_system_impl::jacobian(double* Jd, int64_t ldj) {
 int kad_system_impl::fill_columns(double* Jd, int64_t ldj) {
   // Programs of 2048 columns and more fill the chip with each instruction (8 workgroups
   // per CU); their launches on nfill streams overlap and keep an instruction's arrays
-  // closer together than a whole level's (17x13x12, 2397 columns per program: 0.134 s
-  // against 0.146 grouped; 13x9x8, 819 columns: 33 ms grouped against 62)
+  // closer together than a whole level's (17x13x12, 2397 columns per program: 0.131 s
+  // against 0.137 grouped; 13x9x8, 819 columns: 27 ms grouped against 62)
   const bool wide = (int64_t)sys->n_unknowns >= (int64_t)2048 * (int64_t)tprogs.size();
   if (gtan_ok && fuse_ew && !wide) return columns(0, sys->n_unknowns, 0, Jd, ldj);
   {
