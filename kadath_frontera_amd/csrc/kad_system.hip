@@ -1317,7 +1317,9 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
     for (auto& c : clusters) {
       std::vector<int> rest = c.second;
       while (!rest.empty()) {
-        const size_t k = cluster_steps(code, rest, [](int) { return false; }, nullptr, nullptr);
+        // (the first 64 instructions decide: the temporaries end a region long before)
+        const std::vector<int> head(rest.begin(), rest.begin() + std::min<size_t>(rest.size(), 64));
+        const size_t k = cluster_steps(code, head, [](int) { return false; }, nullptr, nullptr);
         if (k == 0) return KAD_OK;  // (one instruction always fits)
         std::vector<int> part(rest.begin(), rest.begin() + k);
         for (int t : part) unit_of[t] = (int)units.size();
