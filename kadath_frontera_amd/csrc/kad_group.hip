@@ -61,8 +61,8 @@ __device__ __forceinline__ double row_value(const DevRow R, const double* x, boo
 // step and wave, 2/3 of them decoding and register indexing) and, 44% of a wave's time, by
 // the loads; hence four elements per lane, one decoding for them, and no partly filled
 // sweeps.  With one element per lane and the temporaries in LDS J^T w at 13x9x8 took 31.8 ms
-// and 5001 fp32 columns at 17x13x12 25.4, now 26.8 and 21.7 (27.4 and 22.2 with 15
-// temporaries and two waves per SIMD).
+// and 5001 fp32 columns at 17x13x12 25.4, now 26.2 and 20.9 (15 temporaries and two waves
+// per SIMD were 2% slower than 7 and three).
 template <int U>
 __device__ __forceinline__ void cluster_body(const GroupArgs& g, const Where& at, const COp& op, int e0) {
   typedef double Temps __attribute__((ext_vector_type(kClusterTemps + 1)));
