@@ -45,6 +45,13 @@ inline int arg_error(const char* why) {
   return KAD_ERR_ARG;
 }
 
+// |a| as the pivot search compares it, as idamax does: a NaN is passed over (it takes the
+// least value, and no row comes before row j), except in row j itself, where the search
+// starts and no later entry exceeds it.
+__device__ __forceinline__ double pivot_abs(double a, bool row_j) {
+  return a == a ? fabs(a) : (row_j ? (double)INFINITY : 0.0);
+}
+
 // Block-wide (max |a|, first index) reduction.
 template <typename T>
 __device__ void block_argmax(double v, int idx, double* sv, int* si, double& bv, int& bi) {
@@ -557,7 +564,7 @@ __global__ __launch_bounds__(256) void ff_first_kernel(const T* __restrict__ A, 
   int id = -1;
   if (i < n) {
     map_out[i] = i;
-    v = fabs((double)A[i + (int64_t)c0 * lda]);
+    v = pivot_abs((double)A[i + (int64_t)c0 * lda], i == c0);
     id = i;
   }
   double bv;
@@ -624,7 +631,7 @@ __global__ __launch_bounds__(256) void ff_step_kernel(T* __restrict__ A, int64_t
       x -= l * urow[c];
       ai[(int64_t)(j + c) * lda] = x;
       if (c == 1) {
-        v = fabs((double)x);
+        v = pivot_abs((double)x, i == j + 1);
         id = i;
       }
     }
@@ -705,14 +712,15 @@ __device__ __forceinline__ unsigned long long slot_load(const unsigned long long
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// |v| as an unsigned key that orders as the value does (high and low words; FP32: one).
-__device__ __forceinline__ void abs_key(double v, unsigned& hi, unsigned& lo) {
+// |v| as an unsigned key that orders as the value does (high and low words; FP32: one);
+// a NaN's key as pivot_abs: the least, or in row j the largest.
+__device__ __forceinline__ void abs_key(double v, bool row_j, unsigned& hi, unsigned& lo) {
   const unsigned long long b = (unsigned long long)__double_as_longlong(v);
-  hi = (unsigned)(b >> 32) & 0x7fffffffu;
-  lo = (unsigned)b;
+  hi = v == v ? (unsigned)(b >> 32) & 0x7fffffffu : (row_j ? ~0u : 0u);
+  lo = v == v ? (unsigned)b : 0u;
 }
-__device__ __forceinline__ void abs_key(float v, unsigned& hi, unsigned& lo) {
-  hi = __builtin_bit_cast(unsigned, v) & 0x7fffffffu;
+__device__ __forceinline__ void abs_key(float v, bool row_j, unsigned& hi, unsigned& lo) {
+  hi = v == v ? __builtin_bit_cast(unsigned, v) & 0x7fffffffu : (row_j ? ~0u : 0u);
   lo = 0;
 }
 
@@ -795,7 +803,7 @@ __global__ __launch_bounds__(TH) void ffp_kernel(T* __restrict__ A, int64_t lda,
       const int j = c0 + jj, par = s & 1;
       // 1. the wave's candidate among its rows at positions >= j, then the workgroup's
       unsigned hi, lo;
-      abs_key(row[s], hi, lo);
+      abs_key(row[s], pos == j, hi, lo);
       const int best = wave_best(hi, lo, pos >= j ? pos : -1);
       if (lane == (best < 0 ? 0 : best)) {
         wk[par][wave][0] = hi;
@@ -872,7 +880,7 @@ __global__ __launch_bounds__(TH) void ffp_kernel(T* __restrict__ A, int64_t lda,
         int cpos = -1;
         if (lane < G) {
           cpos = (int)xim[lane * rec];
-          abs_key(reinterpret_cast<const T*>(xim + lane * rec + VW)[0], chi, clo);
+          abs_key(reinterpret_cast<const T*>(xim + lane * rec + VW)[0], cpos == j, chi, clo);
         }
         const int bg = wave_best(chi, clo, cpos);
         p = bg < 0 ? -1 : __builtin_amdgcn_readlane(cpos, bg);

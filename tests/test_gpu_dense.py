@@ -184,6 +184,61 @@ def test_persistent_panel_ties_match_per_column(ctx, prec, monkeypatch):
     assert torch.equal(d1, d2)
 
 
+def _pivots(A, k):
+    """The first k interchanges and info of LU with idamax's choice: the first entry no later
+    one exceeds, so a NaN is taken in row j only (right-looking, in A's own precision)."""
+    A, piv, info = A.copy(), [], 0
+    with np.errstate(invalid="ignore", divide="ignore", over="ignore"):
+        for j in range(k):
+            best = abs(A[j, j])
+            p = j
+            for i in range(j + 1, len(A)):
+                if abs(A[i, j]) > best:
+                    best, p = abs(A[i, j]), i
+            piv.append(p)
+            A[[j, p]] = A[[p, j]]
+            if A[j, j] == 0:
+                info = info or j + 1
+            else:
+                A[j + 1:, j] /= A[j, j]
+            A[j + 1:, j + 1:] -= np.outer(A[j + 1:, j], A[j, j + 1:])
+    return piv, info
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [37, 700, 1100])
+@pytest.mark.parametrize("where", ["late", "early", "first", "zeros", "infinite"])
+def test_pivot_search_passes_over_nan(ctx, prec, n, where, monkeypatch):
+    """The pivot search on columns with NaN and infinities, in the persistent panel (one
+    workgroup, several) and in the per-column kernels: idamax's choice.  The first 36 pivots
+    are compared (one base panel and the start of the next), where no two candidates are
+    within rounding."""
+    print(f"pivot search nan {prec} n={n} {where}", flush=True)
+    dt = np.float64 if prec == "f64" else np.float32
+    A = np.random.default_rng(n).standard_normal((n, n)).astype(dt)
+    if where == "late":
+        A[n - 1, 2] = np.nan       # passed over until only its row is left
+    elif where == "early":
+        A[20, 0] = np.nan          # passed over until it lies in row j
+    elif where == "first":
+        A[0, 0] = np.nan           # row j itself
+    elif where == "zeros":
+        A[:, 0] = 0                # the first zero, not the NaN
+        A[n - 2, 0] = np.nan
+    else:
+        A[n // 2, 1] = np.inf      # larger than every number, and then NaN in its row
+        A[n - 1, 1] = np.nan
+    want, winfo = _pivots(A, 36)
+    tdt = torch.float64 if prec == "f64" else torch.float32
+    d1, d2 = colmajor(A, tdt), colmajor(A, tdt)
+    ipiv1, _, info1 = ctx.lu_factor(prec, d1)
+    ctx.sync()
+    ipiv2, info2 = _per_column_factor(monkeypatch, prec, d2)
+    assert ipiv1.cpu().numpy()[:36].tolist() == want
+    assert ipiv2.cpu().numpy()[:36].tolist() == want
+    assert info1 == info2 and (info1 == winfo or winfo == 0)
+
+
 @pytest.mark.parametrize("prec", ["f64", "f32"])
 def test_persistent_panel_large_grid_matches_per_column(ctx, prec, monkeypatch):
     """Dense n = 40000: the first panels are taller than the persistent panel takes
