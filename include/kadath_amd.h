@@ -81,7 +81,9 @@ int kad_lu_factor(kad_ctx* ctx, int prec, int n, void* A, int64_t lda, int* ipiv
  * panel chain is one matrix's: the diagonal domain blocks of the domain-decomposed
  * solve below, which replaces the single pdgesv_ factorisation
  * (src_par/do_newton.cpp:317-320) by independent per-domain ones.  The matrices are
- * taken as dense; each pivot search is LAPACK's within its matrix. */
+ * taken as dense; each pivot search is LAPACK's within its matrix.  The panel's workgroups
+ * (n / 256 per matrix) must fit the CUs together, and at most 64 of them a matrix when
+ * nbat > 1: KAD_ERR_ARG otherwise. */
 int kad_lu_factor_batched(kad_ctx* ctx, int prec, int n, int nbat, void* A, int64_t lda, int64_t strideA, int* ipiv,
                           int* perm, int* info);
 

@@ -1024,8 +1024,10 @@ inline bool ffp_shape(int m, int nbat, int ncu, FfpShape& s) {
   if (m < 1) return false;
   // one workgroup of 1024 rows against several of 256: n = 600 2.05 ms against 2.39, 1215
   // 4.07 against 4.74; beyond that 256 rows per workgroup (n = 5000 20.4 ms, 20.9 with
-  // 512), 512 where 256 would need too many workgroups
+  // 512), 512 where 256 would need too many workgroups (one matrix: a batch of orders
+  // above 64 x 256 is refused)
   for (int th : {1024, 256, 512}) {
+    if (th == 512 && nbat > 1) break;
     s.th = th;
     s.grid = (int)cdiv(m, th);
     if (s.grid <= (th == 1024 ? 1 : FFP_MAX_GRID) && s.grid * nbat <= ncu) break;

@@ -263,6 +263,20 @@ def test_persistent_panel_large_grid_matches_per_column(ctx, prec, monkeypatch):
     torch.cuda.empty_cache()
 
 
+def test_batch_above_the_panel_s_workgroups_is_refused(ctx):
+    """A batch needs every panel in at most 64 workgroups of 256 rows per matrix: the
+    largest order is 16384, whatever the number of CUs, and A stays as it was."""
+    from kadath_frontera_amd._lib import KadError
+    print("batch of order 16640", flush=True)
+    A = torch.ones((2, 16640, 16640), dtype=torch.float64, device="cuda").transpose(1, 2)
+    with pytest.raises(KadError):
+        ctx.lu_factor_batched("f64", A)
+    ctx.sync()
+    assert bool((A == 1).all())
+    del A
+    torch.cuda.empty_cache()
+
+
 def test_persistent_panel_abandoned_barrier_reports_error(ctx, monkeypatch):
     """The persistent panel's waits are bounded: with a spin limit of 0 (set from the
     host, KAD_LU_SPIN) its waits for the other workgroups' candidates are abandoned at
