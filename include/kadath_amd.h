@@ -245,7 +245,11 @@ typedef struct kad_system kad_system;
  * and row order (system_of_eqs.cpp:597-612, kerr.cpp:84-99); order 1: domain-major
  * (unknowns by domain then field, rows by the equation's domain with matching
  * d|d+1 rows in d+1), which makes J block-tridiagonal by domain -- same system,
- * rows and columns permuted.  batch: Jacobian columns per tangent launch chain. */
+ * rows and columns permuted.  batch: the most columns of one (field, domain)'s tangent
+ * program that run together.  The set-up takes the device memory of `batch` columns of the
+ * largest program, run instruction by instruction; the first Jacobian, jvp_fill or vjp may
+ * raise that once to what `batch` columns of every program take by dependency level, to
+ * 6 GiB or to half of the card's free memory, whichever is least. */
 int kad_xcts_create(kad_ctx* ctx, int nr, int nt, int np, const double* bounds, int nbounds, int dmin, int dmax,
                     double n0, double a, double ome, int order, int batch, kad_system** out);
 int kad_xcts_destroy(kad_system* s);
@@ -393,7 +397,7 @@ int kad_sysdef_coloc(kad_sysdef* def, int d, double* r, double* theta, double* p
  * destroyed. */
 int kad_sysdef_host_trace(kad_sysdef* def, int order, int* info, int* row_layout, int cap);
 /* Trace and upload (order 0: reference unknown / row order, 1: domain-major; batch:
- * Jacobian columns per tangent launch chain).  Consumes def (freed, also on error). */
+ * as in kad_xcts_create).  Consumes def (freed, also on error). */
 int kad_system_build(kad_ctx* ctx, kad_sysdef* def, int order, int batch, kad_system** out);
 
 /* ---- entry points of every system (XCTS or built from strings) ---------- */
@@ -431,7 +435,9 @@ int kad_system_get_double(kad_system* s, int k, double* value);
  * which 2 = forget the factorisations kept for reuse (solvers 5 and 7 too): the next
  * step factors its own J.  which 3 = streams of the Jacobian fill (1-4, default 3): the
  * tangent programs are dealt to that many streams, each with its own tangent arena
- * (nphys x batch x slot doubles more per extra stream); J is the same bit for bit.
+ * (nphys x batch x slot doubles more per extra stream); J is the same bit for bit.  Used
+ * where the programs do not run by dependency level (which 5 off, or a whole J whose
+ * programs have 2048 columns and more on average).
  * which 4 = static pivoting in solvers 6-7 (1, the default; 0: partial pivoting at
  * every factorisation): after a factorisation with partial pivoting, later steps of
  * the solve factor their J with its pivot orders (kad_dd_factor_static), falling
@@ -443,7 +449,8 @@ int kad_system_get_double(kad_system* s, int k, double* value);
  * refinement then needs more than 6 inner steps.  which 5 = an
  * element-wise instruction whose operand is made by the spectral pass just before it,
  * and used nowhere else, is applied in that pass's store phase (1, the default; 0:
- * launched on its own); J is the same bit for bit. */
+ * launched on its own, one launch per instruction instead of one per dependency level);
+ * J is the same bit for bit. */
 int kad_system_set_option(kad_system* s, int which, double value);
 /* as kad_xcts_do_newton / kad_xcts_last_solve */
 int kad_system_do_newton(kad_system* s, double precision, double* error, int solver, double* times);

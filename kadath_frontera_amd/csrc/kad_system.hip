@@ -4,7 +4,7 @@
 //
 // Replaces System_of_eqs::do_newton (src_par/do_newton.cpp:65-430):
 //   sec_member / check_equations   -> value program + |F|_inf
-//   do_col_J over all columns      -> tangent programs, B columns per launch chain
+//   do_col_J over all columns      -> tangent programs, at most B columns of each at a time
 //   pdgesv_                        -> kad LU (fp64) or low-precision LU + fp64 refinement
 //   xx_to_vars + old - var         -> CSR update kernel on the coefficient arrays
 #include "kad_common.hpp"
@@ -441,7 +441,8 @@ struct kad_system_impl {
   int B = 256;
   int64_t stride = 0;          // doubles per slot per batch element
   double* val_arena = nullptr;  // nval_slots * stride
-  double* tan_arena = nullptr;  // nphys_max * B * stride
+  double* tan_arena = nullptr;  // nphys_max * B * stride (levels_ready may give it more)
+  size_t tan_cap = 0;           // doubles
   double* F = nullptr;          // n_rows
   double* scratch = nullptr;    // small
   std::vector<kad::LinePlan> plans;  // by the tracer's plan ids; npass 0: no instruction uses it
@@ -511,6 +512,7 @@ struct kad_system_impl {
       if (fev[i]) (void)hipEventDestroy(fev[i]);
     }
     for (void* p : allocs) (void)hipFree(p);
+    if (tan_arena) (void)hipFree(tan_arena);
     delete sys;
   }
   int dmalloc(void** p, size_t bytes) {
@@ -555,8 +557,8 @@ struct kad_system_impl {
   GroupProg gval;
   std::vector<GroupProg> gtan, gpar;
   bool gtan_ok = false;         // every tangent program can be grouped
-  double* grp_arena = nullptr;  // tangent slots of the columns of one round
-  size_t grp_cap = 0;           // doubles
+  bool tan_sized = false;       // the arena has its size for the levels
+  bool levels_ready();
   int group_build(std::vector<Instr> code, int nvirt, bool value, int seed_tab, GroupProg& gp,
                   std::vector<kad::GroupOp>& ops, std::vector<kad::ClusterStep>& steps);
   int group_round(const std::vector<GroupItem>& items, void* out, int64_t ldo, int dtype, const double* w);
@@ -564,10 +566,6 @@ struct kad_system_impl {
   // columns [c0, c1) of J (or, with w, entries of J^T w) into out, whose column 0 is
   // column col_base of J: the double unknowns' programs, then the tangent programs'
   int columns(int c0, int c1, int64_t col_base, void* out, int64_t ldo, int dtype = 0, const double* w = nullptr);
-  int ensure_tan_arena() {
-    if (tan_arena) return KAD_OK;
-    return dmalloc((void**)&tan_arena, (size_t)std::max(1, nphys_max) * B * stride * sizeof(double));
-  }
   bool vals_current = false;  // the value arena holds the value pass of the current fields
   int ensure_values() { return vals_current ? KAD_OK : value_pass(); }
   int value_pass();
@@ -885,6 +883,8 @@ int kad_system_impl::setup() {
     nphys_max = std::max(nphys_max, dp.nphys);
     glob_par_progs.push_back(std::move(dp));
   }
+  tan_cap = (size_t)std::max(1, nphys_max) * B * stride;
+  KAD_HIP_CHECK(hipMalloc((void**)&tan_arena, tan_cap * sizeof(double)));
   // the same programs by dependency level
   std::vector<kad::GroupOp> ops;
   std::vector<kad::ClusterStep> steps;
@@ -912,11 +912,7 @@ int kad_system_impl::setup() {
 int kad_system_impl::run(const std::vector<Instr>& code, int nb, int u0, int seed_tab, void* out, int64_t col0,
                          int64_t ldo, int dtype, const double* w, hipStream_t st, double* tan) {
   hipStream_t s = st ? st : ctx->stream;
-  if (!tan) {
-    const int rc = ensure_tan_arena();
-    if (rc) return rc;
-    tan = tan_arena;
-  }
+  if (!tan) tan = tan_arena;
   auto slot_ptr = [&](const Opnd& o) { return this->slot_ptr(o, tan); };
   for (size_t t = 0; t < code.size(); ++t) {
     const Instr& in = code[t];
@@ -1541,7 +1537,7 @@ int kad_system_impl::group_round(const std::vector<GroupItem>& items, void* out,
   g.ops = gops;
   g.steps = gsteps;
   g.val = val_arena;
-  g.tan = grp_arena;
+  g.tan = tan_arena;
   g.stride = stride;
   g.out = out;
   g.ldo = ldo;
@@ -1586,34 +1582,42 @@ int kad_system_impl::group_round(const std::vector<GroupItem>& items, void* out,
   return KAD_OK;
 }
 
+// Whether the tangent programs run by levels, with the arena for it.  At most B columns of
+// a program run at a time, and the arena has room for those of every program together: a
+// region's arrays stay for a whole level, so a column takes about three times the slots it
+// takes instruction by instruction.  At most 6 GiB (with the regions' temporaries in LDS,
+// 5001 columns at 17x13x12 took 29.7, 25.7, 25.4 ms with 3, 6, 12 GiB, J^T w at 13x9x8 32.7,
+// 32.2, 32.4), and at most half of the card's free memory, which leaves the other half to
+// the caller.  Where that is less than the arena of the set-up, the columns go through that
+// one in more rounds, and instruction by instruction if it does not hold one column.
+bool kad_system_impl::levels_ready() {
+  if (!gtan_ok || !fuse_ew) return false;
+  size_t all = 0, one = 0;
+  auto add = [&](const GroupProg& p, int cnt) {
+    all += (size_t)p.nphys * std::min(cnt, B) * stride;
+    one = std::max(one, (size_t)p.nphys * stride);
+  };
+  for (size_t p = 0; p < gtan.size(); ++p) add(gtan[p], tprogs[p].cnt);
+  for (auto& p : gpar) add(p, 1);
+  if (!tan_sized) {
+    tan_sized = true;
+    size_t want = std::min(all, (size_t)6 << 27), free = 0, total = 0;
+    if (want > tan_cap && hipMemGetInfo(&free, &total) == hipSuccess) {
+      want = std::min(want, free / 2 / sizeof(double));
+      double* more = nullptr;
+      if (want > tan_cap && hipMalloc((void**)&more, want * sizeof(double)) == hipSuccess) {
+        (void)hipFree(tan_arena);
+        tan_arena = more;
+        tan_cap = want;
+      }
+    }
+    (void)hipGetLastError();
+  }
+  return tan_cap >= one;
+}
+
 // The items in rounds that fit the arena.
 int kad_system_impl::group_columns(std::vector<GroupItem> items, void* out, int64_t ldo, int dtype, const double* w) {
-  if (items.empty()) return KAD_OK;
-  if (!grp_arena) {
-    size_t all = 0, one = 0;
-    for (size_t p = 0; p < gtan.size(); ++p) {
-      all += (size_t)gtan[p].nphys * tprogs[p].cnt * stride;
-      one = std::max(one, (size_t)gtan[p].nphys * stride);
-    }
-    for (auto& p : gpar) {
-      all += (size_t)p.nphys * stride;
-      one = std::max(one, (size_t)p.nphys * stride);
-    }
-    // 6 GiB: every column of a 9x7x4 system at once, thousands of columns of the larger
-    // ones (with the regions' temporaries in LDS, 5001 columns at 17x13x12 took 29.7, 25.7,
-    // 25.4 ms with 3, 6, 12 GiB, J^T w at 13x9x8 32.7, 32.2, 32.4); less when the card has
-    // no room for it
-    const size_t least = 64 * one;
-    size_t cap = std::max(std::min(all, (size_t)6 << 27), least);
-    while (hipMalloc((void**)&grp_arena, cap * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      grp_arena = nullptr;
-      if (cap <= least) return KAD_ERR_HIP;
-      cap = std::max(cap / 2, least);
-    }
-    allocs.push_back(grp_arena);
-    grp_cap = cap;
-  }
   std::vector<GroupItem> round;
   size_t used = 0;
   auto flush = [&]() -> int {
@@ -1626,14 +1630,15 @@ int kad_system_impl::group_columns(std::vector<GroupItem> items, void* out, int6
   for (GroupItem it : items) {
     const size_t per = std::max<size_t>(1, (size_t)it.p->nphys * stride);
     while (it.nb > 0) {
-      const int64_t room = (int64_t)((grp_cap - used) / per);
-      if ((int)round.size() >= kad::kGroupEntries || room < std::min(it.nb, 64)) {
+      const int64_t room = (int64_t)((tan_cap - used) / per);
+      if ((int)round.size() >= kad::kGroupEntries || (room < std::min({it.nb, B, 64}) && !round.empty())) {
         const int rc = flush();
         if (rc) return rc;
         continue;
       }
       GroupItem q = it;
-      q.nb = (int)std::min<int64_t>(it.nb, room);
+      q.nb = (int)std::min<int64_t>(std::min(it.nb, B), room);
+      if (q.nb < 1) return KAD_ERR_ALLOC;  // (levels_ready: one column fits)
       round.push_back(q);
       used += per * q.nb;
       it.u0 += q.nb;
@@ -1668,7 +1673,7 @@ int kad_system_impl::value_pass() {
     KAD_HIP_CHECK(hipEventRecord(fev[0], s0));
     for (int i = 1; i < ns; ++i) KAD_HIP_CHECK(hipStreamWaitEvent(fstream[i], fev[0], 0));
     for (int i = 0; i < ns && rc == KAD_OK; ++i)
-      rc = run(vparts[i], 1, 0, -1, F, 0, 0, 0, nullptr, i ? fstream[i] : s0, val_arena);
+      rc = run(vparts[i], 1, 0, -1, F, 0, 0, 0, nullptr, i ? fstream[i] : s0, tan_arena);
     for (int i = 1; i < ns; ++i) {
       KAD_HIP_CHECK(hipEventRecord(fev[i], fstream[i]));
       KAD_HIP_CHECK(hipStreamWaitEvent(s0, fev[i], 0));
@@ -1694,10 +1699,9 @@ int kad_system_impl::fill_columns(double* Jd, int64_t ldj) {
   // closer together than a whole level's (17x13x12, 2397 columns per program: 0.131 s
   // against 0.137 grouped; 13x9x8, 819 columns: 27 ms grouped against 62)
   const bool wide = (int64_t)sys->n_unknowns >= (int64_t)2048 * (int64_t)tprogs.size();
-  if (gtan_ok && fuse_ew && !wide) return columns(0, sys->n_unknowns, 0, Jd, ldj);
+  if (!wide && levels_ready()) return columns(0, sys->n_unknowns, 0, Jd, ldj);
   {
-    int rc = double_columns(Jd, ldj, 0, sys->ndouble, 0);
-    if (!rc) rc = ensure_tan_arena();
+    const int rc = double_columns(Jd, ldj, 0, sys->ndouble, 0);
     if (rc) return rc;
   }
   hipStream_t s0 = ctx->stream;
@@ -3191,7 +3195,7 @@ int kad_jvp_fill(kad_system* s, int col_begin, int col_count, void* J_tile, int6
   const size_t es = dtype == 0 ? sizeof(double) : sizeof(float);
   KAD_HIP_CHECK(hipMemset2DAsync(J_tile, (size_t)ld * es, 0, (size_t)m * es, (size_t)col_count, st));
   const int c1 = col_begin + col_count;
-  if (S->gtan_ok && S->fuse_ew) {
+  if (S->levels_ready()) {
     if ((rc = S->columns(col_begin, c1, col_begin, J_tile, ld, dtype))) return rc;
     KAD_HIP_CHECK(hipStreamSynchronize(st));
     return KAD_OK;
@@ -3218,7 +3222,7 @@ int kad_vjp(kad_system* s, const double* w, double* out) {
   int rc = S->ensure_values();
   if (rc) return rc;
   KAD_HIP_CHECK(hipMemsetAsync(out, 0, (size_t)S->sys->n_unknowns * sizeof(double), st));
-  if (S->gtan_ok && S->fuse_ew) {
+  if (S->levels_ready()) {
     if ((rc = S->columns(0, S->sys->n_unknowns, 0, out, 0, 0, w))) return rc;
     KAD_HIP_CHECK(hipStreamSynchronize(st));
     return KAD_OK;

@@ -62,3 +62,66 @@ def test_traced_system_levels(ctx):
         got[fuse] = (s.residual(), s.jacobian())
     assert torch.equal(got[False][0], got[True][0]) and torch.equal(got[False][1], got[True][1])
     s.close()
+
+
+@pytest.mark.parametrize("nd,batch,spin", [(7, 3, None), (2, 16, None), (2, 1, None), (2, 7, 0.1)])
+def test_columns_in_several_rounds(ctx, nd, batch, spin):
+    """Few columns of a program at a time: programs split over many rounds that the arena's
+    room ends (2 domains, 10 programs) or the 32 programs of a launch (7 domains, 35),
+    column ranges that start and end inside a program and a split."""
+    bounds = [2.0 ** q for q in range(nd)]
+    got = {}
+    for b in (512, batch):  # the reference: one instruction per launch, whole programs
+        s = _flat(programs.kerr(ctx, (5, 5, 4), bounds, n0=0.5, a=1.0, ome=0.05, spin=spin), 1, b)
+        s.set_option(fuse=b == batch)
+        w = torch.tensor(np.random.default_rng(2).standard_normal(s.m), device="cuda")
+        lo, cnt = s.n // 5 + 1, s.n // 2 + 1
+        got[b] = [s.jvp_fill(0, s.n), s.jvp_fill(lo, cnt, dtype=torch.float32), s.vjp(w)]
+        s.close()
+    for a, b in zip(got[512], got[batch]):
+        assert torch.equal(a, b)
+    assert torch.equal(got[batch][0][:, lo:lo + cnt].float(), got[batch][1])
+
+
+def _taken(f):
+    torch.cuda.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    f()
+    torch.cuda.synchronize()
+    return before - torch.cuda.mem_get_info()[0]
+
+
+def test_batch_bounds_the_arena(ctx):
+    """J^T w forms no matrix: what it takes is the tangent arena, `batch` columns of every
+    program at most."""
+    taken = {}
+    for batch in (4096, 8):  # (the first call also loads the kernels)
+        s = _flat(programs.kerr(ctx, (9, 7, 4), BOUNDS[:3], n0=0.5, a=1.0, ome=0.05), 1, batch)
+        w = torch.ones(s.m, dtype=torch.float64, device="cuda")
+        s.residual()
+        taken[batch] = _taken(lambda: s.vjp(w))
+        s.close()
+    print(f"arena {taken}", flush=True)
+    assert 0 < taken[8] < taken[4096] / 8  # programs of 130 to 230 columns: 16 times and more
+
+
+def test_arena_leaves_room_on_the_card(ctx):
+    """With some 2 GiB left on the card the arena takes at most half of them (all columns at
+    once would take 6), and the columns go through it in more rounds with the same results."""
+    s = _flat(programs.kerr(ctx, (13, 9, 8), BOUNDS, n0=0.5, a=1.0, ome=0.05), 1, 256)
+    w = torch.tensor(np.random.default_rng(3).standard_normal(s.m), device="cuda")
+    s.set_option(fuse=False)
+    ref = s.vjp(w).clone()
+    s.set_option(fuse=True)
+    torch.cuda.empty_cache()
+    hold = torch.empty(torch.cuda.mem_get_info()[0] - (2 << 30), dtype=torch.uint8, device="cuda")
+    try:
+        free = torch.cuda.mem_get_info()[0]
+        taken = _taken(lambda: s.vjp(w))
+        print(f"free {free} taken {taken}", flush=True)
+        assert 0 < taken <= free // 2
+        assert torch.equal(s.vjp(w), ref)
+    finally:
+        del hold
+        s.close()
+        torch.cuda.empty_cache()
