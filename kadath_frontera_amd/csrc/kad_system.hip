@@ -767,9 +767,14 @@ int kad_system_impl::upload_plans() {
     const HostPlan& hp = tr.plans[q];
     std::vector<kad::PassDesc> pd;
     for (auto& ps : hp.passes) pd.push_back({ps.axis, ps.nout, ps.line_mat.data()});
-    size_t lines = 0, used = 0;
+    size_t lines = 0, used = 0, size = (size_t)din[q][0] * din[q][1] * din[q][2];
+    int nin[3] = {din[q][0], din[q][1], din[q][2]};
     size_t toff[kad::MAX_PASSES];
-    for (size_t p = 0; p < pd.size(); ++p) lines += (size_t)hp.maxsize;
+    for (const kad::PassDesc& ps : pd) {
+      lines += size / nin[ps.axis];
+      size = size / nin[ps.axis] * ps.nout;
+      nin[ps.axis] = ps.nout;
+    }
     std::vector<kad::LineEnt> tab(std::max<size_t>(1, lines));
     if (!kad::lines_build(din[q][0], din[q][1], din[q][2], pd.data(), (int)pd.size(), (int)hp.pool.size(), plans[q],
                           tab.data(), tab.size(), &used, toff))
@@ -885,9 +890,14 @@ int kad_system_impl::setup() {
   }
   tan_cap = (size_t)std::max(1, nphys_max) * B * stride;
   KAD_HIP_CHECK(hipMalloc((void**)&tan_arena, tan_cap * sizeof(double)));
-  // the same programs by dependency level
+  // the same programs by dependency level (adds 0.6 ms to a set-up of 26.3 ms at 9x7x4, 0.7 to
+  // 44.5 at 13x9x8, 1.3 to 88 at 17x13x12, systems given by strings)
   std::vector<kad::GroupOp> ops;
   std::vector<kad::ClusterStep> steps;
+  size_t most = tr.val.code.size();  // (an entry is some 500 bytes: no copies as the table grows)
+  for (auto& p : sys->tprog) most += p.code.size();
+  for (auto& p : sys->par_prog) most += p.code.size();
+  ops.reserve(most);
   if ((rc = group_build(tr.val.code, 0, true, -1, gval, ops, steps))) return rc;
   gtan.resize(sys->tprog.size());
   gtan_ok = !gtan.empty();
@@ -1084,91 +1094,93 @@ struct GroupUnit {
   int level = 0;
 };
 
-// Whether the element-wise instructions code[t], t in ts (program order), fit the
-// temporaries of one cluster, and if steps is given, its steps.  An operand from outside
-// that is used again is kept in a temporary while one is free (else it is read again); a
-// value made inside must be kept until its last use inside.  stored(slot): the value is
-// read outside the cluster.  Returns how many of ts fit.
-static size_t cluster_steps(const std::vector<Instr>& code, const std::vector<int>& ts,
-                            const std::function<bool(int)>& stored,
-                            const std::function<kad::GroupOpnd(const Opnd&)>& opnd,
-                            std::vector<kad::ClusterStep>* steps) {
-  typedef std::pair<int, int> Key;  // (space, slot)
-  std::map<Key, std::vector<int>> uses;
-  for (size_t i = 0; i < ts.size(); ++i)
-    for (const Opnd* o : {&code[ts[i]].a, &code[ts[i]].b})
-      if (o->slot >= 0) uses[{o->space, o->slot}].push_back((int)i);
-  auto next_use = [&](const Key& k, int i) {  // the first use after instruction i, or -1
-    auto it = uses.find(k);
-    if (it == uses.end()) return -1;
-    auto u = std::upper_bound(it->second.begin(), it->second.end(), i);
-    return u == it->second.end() ? -1 : *u;
-  };
+// The next readers in a list of instructions: next[3 i] and next[3 i + 1] are the places in
+// the list of the next instruction after ts[i] that reads its operand a or b, next[3 i + 2]
+// that of its result (kNever: none).  seen: every slot of the two spaces at kNever, as on
+// return.
+constexpr int kNever = 1 << 30;
+static void next_readers(const std::vector<Instr>& code, const std::vector<int>& ts, std::vector<int> (&seen)[2],
+                         std::vector<int>& next) {
+  next.assign(3 * ts.size(), kNever);
+  for (int i = (int)ts.size() - 1; i >= 0; --i) {
+    const Instr& in = code[ts[i]];
+    next[3 * i + 2] = seen[in.dst.space][in.dst.slot];
+    if (in.a.slot >= 0) next[3 * i] = seen[in.a.space][in.a.slot];
+    if (in.b.slot >= 0) next[3 * i + 1] = seen[in.b.space][in.b.slot];
+    for (const Opnd* o : {&in.a, &in.b})
+      if (o->slot >= 0) seen[o->space][o->slot] = i;
+  }
+  for (int t : ts)
+    for (const Opnd* o : {&code[t].a, &code[t].b})
+      if (o->slot >= 0) seen[o->space][o->slot] = kNever;
+}
+
+// How many of the element-wise instructions code[ts[i]], i from begin to end (program order),
+// fit the temporaries of one cluster, and if steps is given, its steps.  An operand from
+// outside that is used again is kept in a temporary while one is free (else it is read
+// again); a value made inside must be kept until its last use inside.  next: next_readers of
+// ts.  stored(slot): the value is read outside the cluster.
+static int cluster_steps(const std::vector<Instr>& code, const std::vector<int>& ts, const std::vector<int>& next,
+                         int begin, int end, const std::function<bool(int)>& stored,
+                         const std::function<kad::GroupOpnd(const Opnd&)>& opnd,
+                         std::vector<kad::ClusterStep>* steps) {
   struct Temp {
-    Key key{-1, -1};
+    int space = -1, slot = -1;  // -1: free
+    int next = kNever;          // the place of its next reader
     bool input = false;
   };
-  std::vector<Temp> tmp(kad::kClusterTemps);
-  auto find = [&](const Key& k) {
-    for (int q = 0; q < (int)tmp.size(); ++q)
-      if (tmp[q].key == k) return q;
+  Temp tmp[kad::kClusterTemps];
+  auto find = [&](int space, int slot) {
+    for (int q = 0; q < kad::kClusterTemps; ++q)
+      if (tmp[q].space == space && tmp[q].slot == slot) return q;
     return -1;
   };
-  auto release = [&](int i) {  // temporaries whose value is not used after instruction i
-    for (Temp& q : tmp)
-      if (q.key.first >= 0 && next_use(q.key, i) < 0) q = Temp();
-  };
-  for (size_t i = 0; i < ts.size(); ++i) {
+  for (int i = begin; i < end; ++i) {
     const Instr& in = code[ts[i]];
     kad::ClusterStep st;
     st.kind = in.ew;
     st.s = in.s;
-    auto operand = [&](const Opnd& o, int& where, int& cache, kad::GroupOpnd& g) {
+    auto operand = [&](const Opnd& o, int nx, int& where, int& cache, kad::GroupOpnd& g) {
       if (o.slot < 0) return;
-      const Key k{o.space, o.slot};
-      const int q = find(k);
+      const int q = find(o.space, o.slot);
       if (q >= 0) {
         where = q;
+        tmp[q].next = nx;
         return;
       }
       where = -2;
       if (steps) g = opnd(o);
-      if (next_use(k, (int)i) < 0) return;
-      const int f = find({-1, -1});
+      if (nx >= end) return;
+      const int f = find(-1, -1);
       if (f >= 0) {
-        tmp[f].key = k;
-        tmp[f].input = true;
+        tmp[f] = {o.space, o.slot, nx, true};
         cache = f;
       }
     };
-    operand(in.a, st.a, st.ca, st.ga);
+    operand(in.a, next[3 * i], st.a, st.ca, st.ga);
     if (in.b.slot >= 0 && in.b.space == in.a.space && in.b.slot == in.a.slot) {
       st.b = st.a;  // both operands are the same value
       st.gb = st.ga;
     } else {
-      operand(in.b, st.b, st.cb, st.gb);
+      operand(in.b, next[3 * i + 1], st.b, st.cb, st.gb);
     }
-    release((int)i);
-    const Key d{in.dst.space, in.dst.slot};
-    const int nu = next_use(d, (int)i);
-    if (nu >= 0) {
-      int f = find({-1, -1});
+    for (Temp& q : tmp)  // free those whose value is not read after this instruction
+      if (q.next >= end) q = Temp();
+    if (next[3 * i + 2] < end) {
+      int f = find(-1, -1);
       if (f < 0) {  // give up the outside operand that is used last
         int far = -1;
-        for (int q = 0; q < (int)tmp.size(); ++q)
-          if (tmp[q].input && next_use(tmp[q].key, (int)i) > far) {
-            far = next_use(tmp[q].key, (int)i);
+        for (int q = 0; q < kad::kClusterTemps; ++q)
+          if (tmp[q].input && tmp[q].next > far) {
+            far = tmp[q].next;
             f = q;
           }
-        // (not one that this very step reads from or caches into)
-        if (f < 0) return i;
-        if (f == st.ca || f == st.cb) {
-          if (f == st.ca) st.ca = -1;
-          else st.cb = -1;
-        }
+        if (f < 0) return i - begin;
+        // (this very step may have put it there: then it is read from its array again)
+        if (f == st.ca) st.ca = -1;
+        if (f == st.cb) st.cb = -1;
       }
-      tmp[f].key = d;
-      tmp[f].input = false;
+      tmp[f] = {in.dst.space, in.dst.slot, next[3 * i + 2], false};
       st.d = f;
     }
     if (steps) {
@@ -1176,7 +1188,7 @@ static size_t cluster_steps(const std::vector<Instr>& code, const std::vector<in
       steps->push_back(st);
     }
   }
-  return ts.size();
+  return end - begin;
 }
 
 // The instructions of a program by dependency level: an instruction's level is one past
@@ -1254,6 +1266,9 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
   // units
   std::vector<GroupUnit> units;
   std::vector<int> unit_of(N, -1);
+  std::vector<int> seen[2], next;  // next_readers
+  seen[SP_VAL].assign(std::max(1, sys->tr.nval_slots), kNever);
+  seen[SP_TAN].assign(nslots, kNever);
   if (value) {
     for (int t = 0; t < N; ++t) {
       unit_of[t] = (int)units.size();
@@ -1305,22 +1320,26 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
         if (member(r)) m.push_back(r);
       for (size_t x = 0; x < m.size(); ++x)
         for (size_t y = x + 1; y < m.size(); ++y)
-          if (depth[m[x]] == depth[m[y]] && code[m[x]].size == code[m[y]].size) root[top(m[x])] = top(m[y]);
+          if (depth[m[x]] == depth[m[y]] && code[m[x]].size == code[m[y]].size) {
+            root[top(m[x])] = top(m[y]);  // the later ones follow from m[y]
+            break;
+          }
     }
     std::map<int, std::vector<int>> clusters;
     for (int t = 0; t < N; ++t)
       if (member(t)) clusters[top(t)].push_back(t);
     for (auto& c : clusters) {
-      std::vector<int> rest = c.second;
-      while (!rest.empty()) {
+      const std::vector<int>& all = c.second;
+      next_readers(code, all, seen, next);
+      for (int done = 0; done < (int)all.size();) {
         // (the first 64 instructions decide: the temporaries end a region long before)
-        const std::vector<int> head(rest.begin(), rest.begin() + std::min<size_t>(rest.size(), 64));
-        const size_t k = cluster_steps(code, head, [](int) { return false; }, nullptr, nullptr);
+        const int k = cluster_steps(code, all, next, done, std::min((int)all.size(), done + 64),
+                                    [](int) { return false; }, nullptr, nullptr);
         if (k == 0) return KAD_OK;  // (one instruction always fits)
-        std::vector<int> part(rest.begin(), rest.begin() + k);
+        const std::vector<int> part(all.begin() + done, all.begin() + done + k);
         for (int t : part) unit_of[t] = (int)units.size();
         units.push_back({part, true, 0});
-        rest.erase(rest.begin(), rest.begin() + k);
+        done += k;
       }
     }
     for (int t = 0; t < N; ++t)
@@ -1414,7 +1433,9 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
   for (int l = 0; l < depth; ++l) {
     size_t lds = 0;
     double bytes = 0.0;
-    std::vector<std::pair<double, kad::GroupOp>> lv;  // cost, instruction: the longest start first
+    std::vector<kad::GroupOp> lv;
+    std::vector<std::pair<double, int>> order;  // cost, instruction: the longest start first
+    lv.reserve(by_level[l].size());
     for (int u : by_level[l]) {
       const std::vector<int>& ts = units[u].t;
       const Instr& in = code[ts[0]];
@@ -1425,7 +1446,10 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
         op.kind = kad::GK_CLUSTER;
         op.size = in.size;
         op.step0 = (int)steps.size();
-        if (cluster_steps(code, ts, [&](int s) { return live[s] != 0; }, opnd, &steps) != ts.size()) return KAD_ERR_ARG;
+        next_readers(code, ts, seen, next);
+        if (cluster_steps(code, ts, next, 0, (int)ts.size(), [&](int s) { return live[s] != 0; }, opnd, &steps) !=
+            (int)ts.size())
+          return KAD_ERR_ARG;
         op.nsteps = (int)steps.size() - op.step0;
         for (int q = op.step0; q < (int)steps.size(); ++q) {
           kad::ClusterStep& s = steps[q];
@@ -1433,7 +1457,8 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
             if (*w < 0) *w = kad::kClusterTemps;
           bytes += 8.0 * in.size * ((s.a == -2 && s.ga.tan) + (s.b == -2 && s.gb.tan) + (s.gd.slot >= 0));
         }
-        lv.push_back({100.0 * op.nsteps * (double)kad::cdiv(in.size, 256), op});
+        order.push_back({100.0 * op.nsteps * (double)kad::cdiv(in.size, 256), (int)lv.size()});
+        lv.push_back(op);
         continue;
       }
       op.a = opnd(in.a);
@@ -1506,18 +1531,20 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
           break;
       }
       for (int k = 0; k < m; ++k) bytes += op.st[k].o.tan ? 8.0 * nout : 0.0;
-      lv.push_back({cost, op});
+      order.push_back({cost, (int)lv.size()});
+      lv.push_back(op);
     }
-    std::stable_sort(lv.begin(), lv.end(), [](const auto& x, const auto& y) {
-      const bool cx = x.second.kind == kad::GK_CLUSTER, cy = y.second.kind == kad::GK_CLUSTER;
+    std::stable_sort(order.begin(), order.end(), [&](const auto& x, const auto& y) {
+      const bool cx = lv[x.second].kind == kad::GK_CLUSTER, cy = lv[y.second].kind == kad::GK_CLUSTER;
       return cx != cy ? cy : x.first > y.first;  // the clusters last
     });
     int ncl = 0, clsize = 0;
-    for (auto& x : lv) {
-      ops.push_back(x.second);
-      if (x.second.kind != kad::GK_CLUSTER) continue;
+    for (auto& x : order) {
+      const kad::GroupOp& op = lv[x.second];
+      ops.push_back(op);
+      if (op.kind != kad::GK_CLUSTER) continue;
       ++ncl;
-      clsize = std::max(clsize, x.second.size);
+      clsize = std::max(clsize, op.size);
     }
     gp.ncl.push_back(ncl);
     gp.clsize.push_back(clsize);
