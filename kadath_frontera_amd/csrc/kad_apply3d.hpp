@@ -203,21 +203,37 @@ __device__ __forceinline__ void apply3d_body(const double* __restrict__ src, dou
         const int slot = (u >> sh) * 64 + lane, o0 = min(no, (u & ((1 << sh) - 1)) * per), o1 = min(no, o0 + per);
         if (u >= 4) en = entry(p, slot);
         const bool act = slot < nlines;
-        // four lengths: one per length would be 17 pieces of code, each met cold
+        // five lengths: one per length would be 17 pieces of code, each met cold (without
+        // the one of 16, 2349 transforms to coefficients at 17x17x16 took 293 us, now 273,
+        // and 4096 there and back at 15x13x12 206, now 201)
         if (ni <= 10) {
           if (ni <= 6) pass_lines<6>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
           else pass_lines<10>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
         } else {
           if (ni <= 14) pass_lines<14>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
+          else if (ni <= 16) pass_lines<16>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
           else pass_lines<18>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
         }
       }
     } else {
-      // longer lines: an output per thread, straight from LDS
-      for (int e = tid; e < nlines * no; e += 256) {
-        const LineEnt l = P.p[p].tab[e / no];
-        const int o = e % no;
+      // longer lines: an output per thread, straight from LDS; the next one's place is
+      // loaded ahead (without, 3315 transforms there and back at 21x13x12 took 403 us, now 392)
+      const int n = nlines * no;
+      auto place = [&](int e, LineEnt& l, int& o) {
+        const int q = e / no;
+        o = e - q * no;
+        if (e < n) l = P.p[p].tab[q];
+      };
+      LineEnt l{0, 0, -1, 0};
+      int o = 0;
+      place(tid, l, o);
+      for (int e = tid; e < n; e += 256) {
+        LineEnt ln{0, 0, -1, 0};
+        int on = 0;
+        place(e + 256, ln, on);
         y[l.yb + o * sout] = l.off < 0 ? 0.0 : line_dot(mats + l.off + o * ni, x + l.xb, ni, sin);
+        l = ln;
+        o = on;
       }
     }
     __syncthreads();
