@@ -1723,8 +1723,11 @@ int kad_system_impl::jacobian(double* Jd, int64_t ldj) {
 int kad_system_impl::fill_columns(double* Jd, int64_t ldj) {
   // Programs of 2048 columns and more fill the chip with each instruction (8 workgroups
   // per CU); their launches on nfill streams overlap and keep an instruction's arrays
-  // closer together than a whole level's (17x13x12, 2397 columns per program: 0.131 s
-  // against 0.137 grouped; 13x9x8, 819 columns: 27 ms grouped against 62)
+  // closer together than a whole level's.  ms by levels and on streams, columns per program:
+  // 675 13.5, 14.6; 798 18.2, 18.4; 1006 26.4, 25.7 (2 domains 13.0, 13.7); 1214 36.0, 34.3;
+  // 1719 47.1, 45.5; 2079 64.2, 62.2; 2356 79.2, 79.7 (5 domains 137.7, 135.5).  From 1000
+  // the streams lead by up to 5% where a whole program runs at once; with a smaller batch
+  // they trail (798, batch 512, 18.3, 24.8; 1214, batch 1024, 36.0, 39.9).
   const bool wide = (int64_t)sys->n_unknowns >= (int64_t)2048 * (int64_t)tprogs.size();
   if (!wide && levels_ready()) return columns(0, sys->n_unknowns, 0, Jd, ldj);
   {
