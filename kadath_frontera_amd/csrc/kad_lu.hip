@@ -209,7 +209,8 @@ struct ZeroRhs {
 //   tiles, k = 32), whose operands were loaded before the substitution.
 // Bound by latency, not by arithmetic: it replaces 8 launches of a 32-row leaf (a lane
 // per column, 15-20 us each) and 7 products between them (10-13 us) per 256 rows, which
-// were on the panel's critical path.  TRSM_FIGURES
+// were on the panel's critical path.  One launch takes 13 us inside the panels of n = 1215;
+// with it that LU went from 9.3 to 7.7 ms, n = 8191 from 67 to 57.
 constexpr int TRB = 32;          // rows per step
 constexpr int TRSM_ROWS = 256;   // most rows of one launch
 constexpr int TRSM_COLS = 16;    // columns per workgroup
@@ -233,21 +234,6 @@ struct Mfma16<float> {
   static __device__ __forceinline__ int row(int lane, int r) { return 4 * (lane >> 4) + r; }
 };
 
-// The value of lane N of every 16-lane row, to all its lanes (DPP row_newbcast).
-template <int N>
-__device__ __forceinline__ float row_bcast(float v) {
-  const int w = __builtin_bit_cast(int, v);
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(w, w, 0x150 + N, 0xF, 0xF, false));
-}
-template <int N>
-__device__ __forceinline__ double row_bcast(double v) {
-  const long long b = __double_as_longlong(v);
-  const int hi = (int)(b >> 32), lo = (int)b;
-  const int ohi = __builtin_amdgcn_update_dpp(hi, hi, 0x150 + N, 0xF, 0xF, false);
-  const int olo = __builtin_amdgcn_update_dpp(lo, lo, 0x150 + N, 0xF, 0xF, false);
-  return __longlong_as_double(((long long)ohi << 32) | (unsigned)olo);
-}
-
 // Steps K .. 31 of the substitution: lane g of a row holds rows 2g and 2g + 1 (y0, y1).
 template <typename T, bool UP, int K>
 __device__ __forceinline__ void trsm_steps(T& y0, T& y1, const T* __restrict__ Ls, const T* __restrict__ ds, int g) {
@@ -257,7 +243,7 @@ __device__ __forceinline__ void trsm_steps(T& y0, T& y1, const T* __restrict__ L
     q = q / ds[K];
     if (g == K / 2) ((K & 1) ? y1 : y0) = q;
   }
-  const T x = row_bcast<K / 2>(q);
+  const T x = lane16<K / 2>(q);
   y0 = 2 * g > K ? y0 - l0 * x : y0;
   y1 = 2 * g + 1 > K ? y1 - l1 * x : y1;
   if constexpr (K + 1 < TRB) trsm_steps<T, UP, K + 1>(y0, y1, Ls, ds, g);
@@ -670,11 +656,12 @@ __global__ void ff_scatter_kernel(T* __restrict__ A, int64_t lda, int n, int c0,
 //      among ties); after one barrier every wave knows the workgroup's best, and the
 //      wave that owns it stages that row in LDS;
 //   2. with several workgroups, each publishes its candidate's position and the columns
-//      >= j of its row, reads all candidates in one round trip, each word flagged with
-//      its column (no grid barrier: a word is current when its flag is), and reduces them
-//      itself -- LAPACK's choice, the first index of max |a|;
+//      >= j of its row, reads all candidates (four slots per thread and round trip: in
+//      FP64 1 to 5 round trips for up to 64 workgroups of 256 rows), each word flagged with its column
+//      (no grid barrier: a word is current when its flag is), and reduces them itself --
+//      LAPACK's choice, the first index of max |a|;
 //   3. positions, multipliers and the rank-1 update, with the per-column kernel's
-//      operations; the next column's candidates come out of the update.
+//      operations.
 // At the end the interchanges are applied to the panel's other columns [k0, c0) and
 // [c1, k1) (exact: those columns are not read in between).
 // Bound by latency: the chain of its columns is the factorisation's critical path.

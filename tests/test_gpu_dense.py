@@ -240,11 +240,35 @@ def test_pivot_search_passes_over_nan(ctx, prec, n, where, monkeypatch):
 
 
 @pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [100, 1024, 1025, 3000])
+def test_pivot_search_ties_and_zero_columns(ctx, prec, n, monkeypatch):
+    """A first column of +-1 (its first row is the pivot), a column of zeros (row j, and the
+    first exactly zero pivot is reported), a column whose last row alone is not zero, in one
+    workgroup and several and in the per-column kernels."""
+    print(f"pivot search ties {prec} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n)).astype(np.float64 if prec == "f64" else np.float32)
+    A[:, 0] = rng.choice([-1.0, 1.0], n)
+    A[:, 5] = 0
+    A[:-1, 7] = 0
+    want, winfo = _pivots(A, 36)
+    assert want[0] == 0 and want[5] == 5 and winfo == 6
+    tdt = torch.float64 if prec == "f64" else torch.float32
+    d1, d2 = colmajor(A, tdt), colmajor(A, tdt)
+    ipiv1, _, info1 = ctx.lu_factor(prec, d1)
+    ctx.sync()
+    ipiv2, info2 = _per_column_factor(monkeypatch, prec, d2)
+    assert info1 == info2 == winfo
+    assert ipiv1.cpu().numpy()[:36].tolist() == ipiv2.cpu().numpy()[:36].tolist() == want
+
+
+@pytest.mark.parametrize("prec", ["f64", "f32"])
 def test_persistent_panel_large_grid_matches_per_column(ctx, prec, monkeypatch):
     """Dense n = 40000: the first panels are taller than the persistent panel takes
-    (64 workgroups of 256 rows) and run on the per-column kernels; from 16384 rows down
-    the persistent panel runs with up to 64 workgroups exchanging candidates.  Bitwise
-    agreement with the per-column kernels throughout."""
+    (64 workgroups of 512 rows) and run on the per-column kernels; from 32768 rows down
+    the persistent panel runs with up to 64 workgroups exchanging candidates, of 512 rows
+    and from 16384 rows down of 256.  Bitwise agreement with the per-column kernels
+    throughout."""
     print(f"persistent panel n=40000 {prec}", flush=True)
     n = 40000
     dt = torch.float64 if prec == "f64" else torch.float32

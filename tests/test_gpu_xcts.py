@@ -63,9 +63,11 @@ def test_jacobian_matches_oracle(oracle_sys, gpu_sys):
 
 
 def test_jacobian_fill_streams_give_the_same_J(oracle_sys, gpu_sys):
-    # the tangent programs dealt to 1-4 streams (batch 128: several column tiles per
-    # program, run one after another on their stream's arena) fill J bit for bit alike,
-    # and the value program split by domain over the same streams gives the same F
+    # by dependency level (a system of this size) the number of streams changes nothing;
+    # one launch per instruction, the tangent programs dealt to 1-4 streams (batch 128:
+    # several column tiles per program, run one after another on their stream's arena) fill
+    # the same J bit for bit, and the value program split by domain over the same streams
+    # gives the same F
     _, X0 = oracle_sys
     gpu_sys.set_guess(X0)
     try:
@@ -78,13 +80,47 @@ def test_jacobian_fill_streams_give_the_same_J(oracle_sys, gpu_sys):
             assert torch.equal(gpu_sys.jacobian(), J1), k
         with pytest.raises(RuntimeError):
             gpu_sys.set_option(fill_streams=5)
+        for k in (1, 2, 3, 4):
+            gpu_sys.set_option(fill_streams=k, fuse=False)
+            assert torch.equal(gpu_sys.residual(), F1), k
+            assert torch.equal(gpu_sys.jacobian(), J1), k
     finally:
-        gpu_sys.set_option(fill_streams=3)
+        gpu_sys.set_option(fill_streams=3, fuse=True)
+
+
+def test_wide_programs_on_streams_give_the_levels_J(ctx):
+    # programs of more than 2048 columns fill a whole J on the streams, fused or one launch
+    # per instruction; kad_jvp_fill of the same system runs by dependency level.  All alike bit
+    # for bit (batch 1000: three column tiles per program and arena).
+    import ctypes
+    from kadath_frontera_amd._lib import lib
+    from kadath_frontera_amd.xcts import XctsSystem
+    s = XctsSystem(ctx, (17, 13, 12), [1.0, 2.0], n0=0.5, a=1.0, ome=0.05, batch=1000, order=1)
+    assert s.n >= 2048 * len(s.layout)
+    s.set_guess(s.perturbation(4))
+    s.residual()
+    T = torch.empty((s.n, s.m), dtype=torch.float64, device="cuda")
+    for lo in range(0, s.n, 7000):  # tiles that begin and end inside a program
+        cnt = min(7000, s.n - lo)
+        assert lib.kad_jvp_fill(s.h, lo, cnt, ctypes.c_void_p(T[lo:].data_ptr()), s.m, 0) == 0
+    ctx.sync()
+    try:
+        for fuse, streams in ((True, 1), (True, 2), (True, 3), (True, 4), (False, 3)):
+            s.set_option(fuse=fuse, fill_streams=streams)
+            print(f"wide fill fuse {fuse} streams {streams}", flush=True)
+            J = s.jacobian()
+            assert torch.equal(J.T, T), (fuse, streams)
+            del J
+    finally:
+        s.close()
+        del T
+        torch.cuda.empty_cache()
 
 
 def test_fused_element_wise_instructions_give_the_same_J(oracle_sys, gpu_sys):
-    # the element-wise instructions applied in the spectral pass that feeds them, or
-    # launched on their own: the same J bit for bit
+    # by dependency level, or one launch per instruction: the same J bit for bit (the
+    # instructions with element-wise ones applied in the pass that feeds them:
+    # test_wide_programs_on_streams_give_the_levels_J)
     _, X0 = oracle_sys
     gpu_sys.set_guess(X0)
     try:
