@@ -203,15 +203,18 @@ __device__ __forceinline__ void apply3d_body(const double* __restrict__ src, dou
         const int slot = (u >> sh) * 64 + lane, o0 = min(no, (u & ((1 << sh) - 1)) * per), o1 = min(no, o0 + per);
         if (u >= 4) en = entry(p, slot);
         const bool act = slot < nlines;
-        // five lengths: one per length would be 17 pieces of code, each met cold (without
-        // the one of 16, 2349 transforms to coefficients at 17x17x16 took 293 us, now 273,
-        // and 4096 there and back at 15x13x12 206, now 201)
+        // five lengths: one per length would be 17 pieces of code, each met cold.  Without the
+        // one of 16, 2349 transforms to coefficients at 17x17x16 took 293 us, now 273, and 4096
+        // there and back at 15x13x12 206, now 201; it is laid out of the others' way (553 us per
+        // residual at 17x13x12, which does not meet it, with it among them, 543 so, 549
+        // without it).
         if (ni <= 10) {
           if (ni <= 6) pass_lines<6>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
           else pass_lines<10>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
         } else {
           if (ni <= 14) pass_lines<14>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
-          else if (ni <= 16) pass_lines<16>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
+          else if (__builtin_expect(ni == 15 || ni == 16, 0))
+            pass_lines<16>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
           else pass_lines<18>(x, y, mats, en, act, ni, sin, sout, o0, o1, barrier);
         }
       }
