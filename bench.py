@@ -44,29 +44,30 @@ SEED = 20261202
 PEAK = {"f64": 78.6, "f32": 157.3, "bf16": 2500.0}  # MI355X dense matrix TFLOP/s (vendor figures)
 # HBM bytes per launch, from two rocprofv3 --pmc passes (FETCH_SIZE, then WRITE_SIZE),
 # FETCH_SIZE scaled by 2.0 and WRITE_SIZE by 1.0: the factors at which the same
-# counters read a 256 MiB device-to-device copy (131093.6 KiB fetched, 262144.0 KiB
+# counters read a 256 MiB device-to-device copy (131092.8 KiB fetched, 262144.0 KiB
 # written).
-#   apply3d: over the residual and Jacobian fill of this workload (--fill-only, 6566
-#     launches, 3.736e11 algorithmic bytes with the element-wise instructions applied in
-#     their store phase), traffic / algorithmic bytes = 1.0050; the bench reports that
-#     ratio times its live algorithmic bytes per launch.
-APPLY3D_TRAFFIC_RATIO = (2.0 * 99981830.5625 + 166654442.78125) * 1024.0 / 373567286352.0
+#   apply3d: over the residual and Jacobian fill of this workload (--fill-only, 2974
+#     launches, 3.831e11 algorithmic bytes with the element-wise instructions applied in
+#     their store phase, 0.1% of them the value program's 62 level launches, whose traffic
+#     is not counted), traffic / algorithmic bytes = 1.005; the bench reports that ratio
+#     times its live algorithmic bytes per launch.
+APPLY3D_TRAFFIC_RATIO = (2.0 * 104647884.3125 + 166558747.34375) * 1024.0 / 383111671696.0
 # gemm_k4: the launches of one iteration span many shapes (64- and 128-tiles, the domain
 # blocks' updates, the triangular solves' and the Woodbury products), and counter passes
 # over the whole LU are not taken (the one tried ended in a segfault of the profiler's host
 # counter path, with the persistent panel kernel spinning beside the GEMM), so the line's
 # traffic stays null. The kernel is measured on its own at one domain block's trailing
 # update instead (--gemm-only: C 12032 x 12032 -= A 12032 x 256 B, same calibration):
-# 2 x 981412.0 KiB fetched + 1131008 KiB written = 3.168 GB per launch, 1.339 x the
-# algorithmic 2.366 GB (C read and written once, the A and B panels re-fetched about 17
-# times over eight L2s), at 23.4 flop/B, above the FP64 ridge: compute-bound.
+# 2 x 992280.5 KiB fetched + 1131008 KiB written = 3.190 GB per launch, 1.349 x the
+# algorithmic 2.366 GB (C read and written once, the A and B panels re-fetched about 18
+# times over eight L2s), at 23.2 flop/B, above the FP64 ridge: compute-bound.
 # traffic_model_bytes is the operand traffic per launch of the executed tiles (each 128 x
 # 128 C tile reads its 128 x k A and k x 128 B panels, reads and writes C), an upper bound
 # on HBM bytes when nothing is reused through L2.
 GEMM_TRAFFIC_NOTE = ("traffic is not measured over the LU's mixed GEMM launches; measured alone at a domain "
-                     "block's trailing update (12032 x 12032 x 256, --gemm-only) gemm_k4 moves 3.168 GB per "
-                     "launch = 1.339 x its algorithmic bytes (C once, A/B panels re-fetched), compute-bound at "
-                     "23.4 flop/B; traffic_model_bytes = operand bytes per launch of the executed tiles with no "
+                     "block's trailing update (12032 x 12032 x 256, --gemm-only) gemm_k4 moves 3.190 GB per "
+                     "launch = 1.349 x its algorithmic bytes (C once, A/B panels re-fetched), compute-bound at "
+                     "23.2 flop/B; traffic_model_bytes = operand bytes per launch of the executed tiles with no "
                      "L2 reuse")
 
 
