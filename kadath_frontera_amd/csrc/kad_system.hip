@@ -1629,16 +1629,19 @@ bool kad_system_impl::levels_ready() {
   if (!tan_sized) {
     tan_sized = true;
     size_t want = std::min(all, (size_t)6 << 27), free = 0, total = 0;
-    if (want > tan_cap && hipMemGetInfo(&free, &total) == hipSuccess) {
+    double* more = nullptr;
+    if (want > tan_cap) {
+      // (work on the present arena ends on the context's stream)
+      bool ok = hipStreamSynchronize(ctx->stream) == hipSuccess && hipMemGetInfo(&free, &total) == hipSuccess;
       want = std::min(want, free / 2 / sizeof(double));
-      double* more = nullptr;
-      if (want > tan_cap && hipMalloc((void**)&more, want * sizeof(double)) == hipSuccess) {
+      if (ok && want > tan_cap) ok = hipMalloc((void**)&more, want * sizeof(double)) == hipSuccess;
+      if (!ok) (void)hipGetLastError();  // no room: the present arena serves
+      if (ok && more) {
         (void)hipFree(tan_arena);
         tan_arena = more;
         tan_cap = want;
       }
     }
-    (void)hipGetLastError();
   }
   return tan_cap >= one;
 }
