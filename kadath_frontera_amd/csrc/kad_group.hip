@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256) void group_kernel(GroupArgs g) {
 
 int group_launch(const GroupArgs& g, int blocks, bool clusters, size_t lds, hipStream_t s) {
   if (blocks <= 0) return KAD_OK;
-  if (g.nent < 1 || g.nent > kGroupEntries || lds > 160 * 1024) return KAD_ERR_ARG;
+  if (g.nent < 1 || g.nent > kGroupEntries || lds > kMaxLds) return KAD_ERR_ARG;
   if (clusters) cluster_kernel<<<blocks, 64, 0, s>>>(g);
   else group_kernel<<<blocks, 256, lds, s>>>(g);
   KAD_HIP_CHECK(hipGetLastError());

@@ -100,7 +100,7 @@ bool lines_build(int d0, int d1, int d2, const PassDesc* passes, int npass, int 
   if (P.small) P.single = 0;  // outputs by other threads than read the line: two buffers
   P.size_out = dm[0] * dm[1] * dm[2];
   *used = n;
-  return lines_lds(P) <= 160 * 1024;
+  return true;
 }
 
 int apply3d_launch(const double* in, int64_t in_stride, double* out, int64_t out_stride, int nbatch, const LinePlan& P,
@@ -109,7 +109,7 @@ int apply3d_launch(const double* in, int64_t in_stride, double* out, int64_t out
   if (post && post->n > 0 && (post->n > kMaxChain || !post->dst)) return KAD_ERR_ARG;
   const PostOp pop = post ? *post : PostOp();
   const size_t lds = lines_lds(P);
-  if (lds > 160 * 1024) return KAD_ERR_ARG;
+  if (lds > kMaxLds || P.npass < 1) return KAD_ERR_ARG;
   GemmTimer* tm = g_apply_timer;
   bool timed = false;
   if (tm) {

@@ -43,6 +43,8 @@ struct LinePlan {
   Pass p[MAX_PASSES];
 };
 
+constexpr size_t kMaxLds = 160 * 1024;  // of a workgroup
+
 // LDS bytes of a chain (kad_apply3d.hpp).
 inline size_t lines_lds(const LinePlan& P) {
   return ((P.single ? 1 : 2) * (size_t)P.maxsize + (size_t)P.pool_size) * sizeof(double);
@@ -50,7 +52,8 @@ inline size_t lines_lds(const LinePlan& P) {
 
 // The line tables of a chain over a d0 x d1 x d2 array, one after another in tab (HOST); the
 // caller uploads them and sets every pass's tab to its part (toff) and the pool.  False:
-// more passes than MAX_PASSES or more LDS than a workgroup has.
+// no pass or more than MAX_PASSES, or more than cap lines.  (A chain that needs more LDS than
+// a workgroup has is laid out; its launches are refused.)
 bool lines_build(int d0, int d1, int d2, const PassDesc* passes, int npass, int pool_size, LinePlan& P,
                  LineEnt* tab, size_t cap, size_t* used, size_t* toff);
 

@@ -1229,7 +1229,9 @@ int kad_system_impl::group_build(std::vector<Instr> code, int nvirt, bool value,
       const Opnd& d = in.dst;
       if (d.space != space || d.slot < 0 || d.slot >= nslots || writer[d.slot] >= 0) return KAD_OK;
       if (in.kind == I_EW && (in.ew < 0 || in.ew > EW_SDIV || in.a.slot < 0)) return KAD_OK;
-      if (in.kind == I_LIN && (in.plan < 0 || in.plan >= (int)plans.size())) return KAD_OK;
+      if (in.kind == I_LIN && (in.plan < 0 || in.plan >= (int)plans.size() ||
+                               kad::lines_lds(plans[in.plan]) > kad::kMaxLds))
+        return KAD_OK;
       writer[d.slot] = t;
     }
   }

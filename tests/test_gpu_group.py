@@ -125,3 +125,18 @@ def test_arena_leaves_room_on_the_card(ctx):
         del hold
         s.close()
         torch.cuda.empty_cache()
+
+
+def test_arrays_beyond_lds_build_and_refuse_to_run(ctx):
+    """Domain arrays whose transforms need more LDS than a workgroup has: the system is built
+    (its layout and coefficients are there), what would run a transform is refused."""
+    s = XctsSystem(ctx, (33, 17, 16), BOUNDS[:2], n0=0.5, a=1.0, ome=0.05, batch=4, order=1)
+    assert s.n == s.m and sum(q[3] for q in s.layout) == s.n
+    cf = s.coef(0, 1)
+    cf[0, 0, 0] = 1.25
+    s.set_coef(0, 1, cf)
+    assert s.coef(0, 1)[0, 0, 0] == 1.25
+    for f in (s.residual, lambda: s.do_newton(1e-10, "f64-dd")):
+        with pytest.raises(RuntimeError):
+            f()
+    s.close()
