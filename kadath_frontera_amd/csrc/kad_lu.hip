@@ -131,7 +131,8 @@ __global__ __launch_bounds__(1024) void row_tile_mask_kernel(const T* __restrict
   if (threadIdx.x == 0) mask[blockIdx.x] = any;
 }
 // Last nonzero row of each 128-column tile: out[tile] = max over the 256-row chunks
-// (workgroup (tile, chunk); out starts at -1).  A chunk is read from its end, 32 rows at
+// (workgroup (tile, chunk)); -1 where there is none, with several chunks only if out starts
+// there.  A chunk is read from its end, 32 rows at
 // a time, until a nonzero is met, so a dense matrix costs one step of it (a full scan
 // took 180 us at n = 1215, 470 at 8191).
 template <typename T>
@@ -140,6 +141,10 @@ __global__ __launch_bounds__(256) void col_extent_kernel(const T* __restrict__ A
   const int c0 = blockIdx.x * 128, r0 = blockIdx.y * 256;
   const int ce = min(c0 + 128, n), re = min(r0 + 256, n);
   const int tr = threadIdx.x & 31, tc = threadIdx.x >> 5;  // row within a step, one of 8 column groups
+  if (gridDim.y == 1) {
+    if (threadIdx.x == 0) out[blockIdx.x] = -1;
+    __syncthreads();
+  }
   for (int rb = r0 + (re - r0 - 1) / 32 * 32; rb >= r0; rb -= 32) {
     const int r = rb + tr;
     int any = 0;
@@ -1359,7 +1364,7 @@ int getrf(T* A, int64_t lda, int n, int* ipiv, int nb, int gemm_prec, LuWork& w,
   const int ntc = (int)cdiv(n, 128), nrc = (int)cdiv(n, 256);
   std::vector<int> ext(ntc, bat ? n - 1 : -1);
   if (!bat) {
-    KAD_HIP_CHECK(hipMemsetAsync(w.ext, 0xff, ntc * sizeof(int), w.stream));  // -1
+    if (nrc > 1) KAD_HIP_CHECK(hipMemsetAsync(w.ext, 0xff, ntc * sizeof(int), w.stream));  // -1
     col_extent_kernel<T><<<dim3(ntc, nrc), 256, 0, w.stream>>>(A, lda, n, w.ext);
     KAD_HIP_CHECK(hipGetLastError());
     KAD_HIP_CHECK(hipMemcpyAsync(ext.data(), w.ext, ntc * sizeof(int), hipMemcpyDeviceToHost, w.stream));

@@ -43,7 +43,8 @@ __device__ __forceinline__ double tri_at(const T* F, int64_t lda, int r, int c) 
 // Each row's residual X T - I is at rounding level, as the column-by-column inversion's
 // was (joining inverted quarters by products would square the conditioning of
 // ill-conditioned blocks into it).  The block is held as a lower triangle (an upper one
-// with both index orders reversed).
+// with both index orders reversed).  Of a partial last block only the columns that hold it
+// run (an order of 8 was solved in 193 us with all of them, 101 so).
 constexpr int DIB = 32;  // columns per step
 
 template <typename T>
@@ -58,8 +59,11 @@ __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__
   const int r0 = blk * TBS;
   const int nb = min(TBS, n - r0);
   const int t = threadIdx.x;
-  // M(i, c), i >= c: the triangle (reversed for uplo 1), the identity past nb
-  for (int e0 = 0; e0 < TBS * TBS; e0 += 256 * 8) {
+  // M(i, c), i >= c: the triangle (reversed for uplo 1), the identity past nb; steps that
+  // hold rows of the block: the first ns (the last ones for uplo 1)
+  const int ns = (nb + DIB - 1) / DIB, Jlo = uplo == 0 ? 0 : TBS / DIB - ns, Jhi = Jlo + ns - 1;
+  const int c0 = uplo == 0 ? 0 : TBS - nb;  // the block's first row and column here
+  for (int e0 = 0; e0 < TBS * DIB * ns; e0 += 256 * 8) {
     double v[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -80,13 +84,13 @@ __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__
   __syncthreads();
   const int r = t & (TBS - 1), half = t >> 7, rb = r / DIB;
 #pragma unroll 1
-  for (int J = TBS / DIB - 1; J >= 0; --J) {
+  for (int J = Jhi; J >= Jlo; --J) {
     const int j0 = J * DIB, jh = j0 + half * (DIB / 2);
     // p(j) = I(r, j) - sum over the later column blocks of X(r, k) T(k, j)
     double p[DIB / 2];
 #pragma unroll
     for (int j = 0; j < DIB / 2; ++j) p[j] = jh + j == r ? 1.0 : 0.0;
-    for (int k = j0 + DIB; k < (rb + 1) * DIB; ++k) {
+    for (int k = j0 + DIB; k < (min(rb, Jhi) + 1) * DIB; ++k) {
       const double xk = M[r][k];
 #pragma unroll
       for (int j = 0; j < DIB / 2; ++j) p[j] -= xk * M[k][jh + j];
@@ -95,7 +99,7 @@ __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__
 #pragma unroll
       for (int j = 0; j < DIB / 2; ++j) pbuf[r][j] = p[j];
     __syncthreads();
-    const bool mine = !half && rb >= J;
+    const bool mine = !half && rb >= J && rb <= Jhi;
     double x[DIB];
     if (mine) {
 #pragma unroll
@@ -105,6 +109,7 @@ __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__
       }
 #pragma unroll
       for (int j = DIB - 1; j >= 0; --j) {
+        if (j0 + j < c0 || j0 + j >= c0 + nb) continue;  // uniform: a column of the identity
 #pragma unroll
         for (int k = j + 1; k < DIB; ++k) x[j] -= x[k] * M[j0 + k][j0 + j];
         if (uplo == 1) x[j] /= M[j0 + j][j0 + j];

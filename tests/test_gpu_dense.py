@@ -184,6 +184,29 @@ def test_persistent_panel_ties_match_per_column(ctx, prec, monkeypatch):
     assert torch.equal(d1, d2)
 
 
+@pytest.mark.parametrize("prec", ["f64", "f32"])
+@pytest.mark.parametrize("n", [1, 2, 31, 32, 33, 64, 65, 96, 97, 127, 128, 129, 161, 255])
+def test_solve_partial_blocks(ctx, prec, n):
+    """Solves whose last 128-row block is partial, by columns and by 32-column steps of the
+    diagonal blocks' inverses, both transposes.  A is diagonally dominant, so its factors'
+    triangles are well conditioned and every 128-row step's error is a few n u of the
+    solution."""
+    print(f"solve partial blocks {prec} n={n}", flush=True)
+    rng = np.random.default_rng(n)
+    A = rng.standard_normal((n, n)) / n + 2 * np.eye(n)
+    b = rng.standard_normal(n)
+    dt = torch.float64 if prec == "f64" else torch.float32
+    dA = colmajor(A, dt)
+    A = dA.double().cpu().numpy().copy()
+    _, perm, info = ctx.lu_factor(prec, dA)
+    assert info == 0
+    u = 2.0 ** (-53 if prec == "f64" else -24)
+    for trans in (0, 1):
+        x = ctx.lu_solve(prec, dA, perm, torch.tensor(b, device="cuda"), trans).cpu().numpy()
+        ref = np.linalg.solve(A.T if trans else A, b)
+        assert np.abs(x - ref).max() <= 8 * n * u * np.abs(ref).max(), (trans, np.abs(x - ref).max())
+
+
 def _pivots(A, k):
     """The first k interchanges and info of LU with idamax's choice: the first entry no later
     one exceeds, so a NaN is taken in row j only (right-looking, in A's own precision)."""
