@@ -47,21 +47,17 @@ __device__ __forceinline__ double tri_at(const T* F, int64_t lda, int r, int c) 
 // run (an order of 8 was solved in 193 us with all of them, 101 so).
 constexpr int DIB = 32;  // columns per step
 
-template <typename T>
-__global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__ F, int64_t lda, int n, int uplo,
-                                                           int tr_out, double* __restrict__ W, int64_t sF = 0,
-                                                           int64_t sW = 0) {
-  F += (int64_t)blockIdx.y * sF;  // factors blockIdx.y of a batch
-  W += (int64_t)blockIdx.y * sW;
-  __shared__ double M[TBS][TBS + 1];
-  __shared__ double pbuf[TBS][DIB / 2 + 1];
-  const int blk = blockIdx.x;
-  const int r0 = blk * TBS;
-  const int nb = min(TBS, n - r0);
+// FULL: nb = TBS (code of its own: with the partial block's bounds on every column a solve of
+// order 1215 took 9 us more).
+template <typename T, bool FULL>
+__device__ __forceinline__ void diag_inverse_body(const T* __restrict__ F, int64_t lda, int r0, int nb_, int uplo,
+                                                  int tr_out, double* __restrict__ out, double (*M)[TBS + 1],
+                                                  double (*pbuf)[DIB / 2 + 1]) {
+  const int nb = FULL ? TBS : nb_;
   const int t = threadIdx.x;
   // M(i, c), i >= c: the triangle (reversed for uplo 1), the identity past nb; steps that
   // hold rows of the block: the first ns (the last ones for uplo 1)
-  const int ns = (nb + DIB - 1) / DIB, Jlo = uplo == 0 ? 0 : TBS / DIB - ns, Jhi = Jlo + ns - 1;
+  const int ns = (nb + DIB - 1) / DIB, Jlo = FULL || uplo == 0 ? 0 : TBS / DIB - ns, Jhi = Jlo + ns - 1;
   const int c0 = uplo == 0 ? 0 : TBS - nb;  // the block's first row and column here
   for (int e0 = 0; e0 < TBS * DIB * ns; e0 += 256 * 8) {
     double v[8];
@@ -109,7 +105,7 @@ __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__
       }
 #pragma unroll
       for (int j = DIB - 1; j >= 0; --j) {
-        if (j0 + j < c0 || j0 + j >= c0 + nb) continue;  // uniform: a column of the identity
+        if (!FULL && (j0 + j < c0 || j0 + j >= c0 + nb)) continue;  // uniform: a column of the identity
 #pragma unroll
         for (int k = j + 1; k < DIB; ++k) x[j] -= x[k] * M[j0 + k][j0 + j];
         if (uplo == 1) x[j] /= M[j0 + j][j0 + j];
@@ -123,12 +119,25 @@ __global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__
     }
     __syncthreads();
   }
-  double* out = W + (int64_t)blk * TBS * WCOLS;
   for (int e = t; e < TBS * TBS; e += 256) {
     const int i = tr_out ? e / TBS : e % TBS, c = tr_out ? e % TBS : e / TBS;
     const bool tri = i < nb && c < nb && (uplo == 0 ? i >= c : i <= c);
     out[e] = !tri ? 0.0 : uplo == 0 ? M[i][c] : M[TBS - 1 - i][TBS - 1 - c];
   }
+}
+
+template <typename T>
+__global__ __launch_bounds__(256) void diag_inverse_kernel(const T* __restrict__ F, int64_t lda, int n, int uplo,
+                                                           int tr_out, double* __restrict__ W, int64_t sF = 0,
+                                                           int64_t sW = 0) {
+  F += (int64_t)blockIdx.y * sF;  // factors blockIdx.y of a batch
+  W += (int64_t)blockIdx.y * sW;
+  __shared__ double M[TBS][TBS + 1];
+  __shared__ double pbuf[TBS][DIB / 2 + 1];
+  const int r0 = blockIdx.x * TBS, nb = min(TBS, n - r0);
+  double* out = W + (int64_t)blockIdx.x * TBS * WCOLS;
+  if (nb == TBS) diag_inverse_body<T, true>(F, lda, r0, nb, uplo, tr_out, out, M, pbuf);
+  else diag_inverse_body<T, false>(F, lda, r0, nb, uplo, tr_out, out, M, pbuf);
 }
 
 // Coupling half of W_k: -inv(T_kk) T_kp, with T accessed through tri_at and
