@@ -247,9 +247,9 @@ typedef struct kad_system kad_system;
  * d|d+1 rows in d+1), which makes J block-tridiagonal by domain -- same system,
  * rows and columns permuted.  batch: the most columns of one (field, domain)'s tangent
  * program that run together.  The set-up takes the device memory of `batch` columns of the
- * largest program, run instruction by instruction; the first Jacobian, jvp_fill or vjp may
- * raise that once to what `batch` columns of every program take by dependency level, to
- * 6 GiB or to half of the card's free memory, whichever is least. */
+ * largest program, run instruction by instruction; the first Jacobian, jvp_fill or vjp whose
+ * columns do not fit it raises it once to what `batch` columns of every program take by
+ * dependency level, to 6 GiB or to half of the card's free memory, whichever is least. */
 int kad_xcts_create(kad_ctx* ctx, int nr, int nt, int np, const double* bounds, int nbounds, int dmin, int dmax,
                     double n0, double a, double ome, int order, int batch, kad_system** out);
 int kad_xcts_destroy(kad_system* s);

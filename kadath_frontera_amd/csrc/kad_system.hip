@@ -441,7 +441,7 @@ struct kad_system_impl {
   int B = 256;
   int64_t stride = 0;          // doubles per slot per batch element
   double* val_arena = nullptr;  // nval_slots * stride
-  double* tan_arena = nullptr;  // nphys_max * B * stride (levels_ready may give it more)
+  double* tan_arena = nullptr;  // nphys_max * B * stride (grow_arena may give it more)
   size_t tan_cap = 0;           // doubles
   double* F = nullptr;          // n_rows
   double* scratch = nullptr;    // small
@@ -559,6 +559,7 @@ struct kad_system_impl {
   bool gtan_ok = false;         // every tangent program can be grouped
   bool tan_sized = false;       // the arena has its size for the levels
   bool levels_ready();
+  void grow_arena();
   int group_build(std::vector<Instr> code, int nvirt, bool value, int seed_tab, GroupProg& gp,
                   std::vector<kad::GroupOp>& ops, std::vector<kad::ClusterStep>& steps);
   int group_round(const std::vector<GroupItem>& items, void* out, int64_t ldo, int dtype, const double* w);
@@ -1611,45 +1612,50 @@ int kad_system_impl::group_round(const std::vector<GroupItem>& items, void* out,
   return KAD_OK;
 }
 
-// Whether the tangent programs run by levels, with the arena for it.  At most B columns of
-// a program run at a time, and the arena has room for those of every program together: a
-// region's arrays stay for a whole level, so a column takes about three times the slots it
-// takes instruction by instruction.  At most 6 GiB (with the regions' temporaries in LDS,
-// 5001 columns at 17x13x12 took 29.7, 25.7, 25.4 ms with 3, 6, 12 GiB, J^T w at 13x9x8 32.7,
-// 32.2, 32.4), and at most half of the card's free memory, which leaves the other half to
-// the caller.  Where that is less than the arena of the set-up, the columns go through that
-// one in more rounds, and instruction by instruction if it does not hold one column.
+// The tangent arena with room for what the levels take, once: at most B columns of a program
+// run at a time, and those of every program together have room (a region's arrays stay for a
+// whole level, so a column takes about three times the slots it takes instruction by
+// instruction).  At most 6 GiB (with the regions' temporaries in LDS, 5001 columns at
+// 17x13x12 took 29.7, 25.7, 25.4 ms with 3, 6, 12 GiB, J^T w at 13x9x8 32.7, 32.2, 32.4), and
+// at most half of the card's free memory, which leaves the other half to the caller.  Where
+// that is less than the arena of the set-up, that one serves, in more rounds.
+void kad_system_impl::grow_arena() {
+  if (tan_sized) return;
+  tan_sized = true;
+  size_t want = 0, free = 0, total = 0;
+  for (size_t p = 0; p < gtan.size(); ++p) want += (size_t)gtan[p].nphys * std::min(tprogs[p].cnt, B) * stride;
+  for (auto& p : gpar) want += (size_t)p.nphys * stride;
+  want = std::min(want, (size_t)6 << 27);
+  if (want <= tan_cap) return;
+  // (work on the present arena ends on the context's stream)
+  bool ok = hipStreamSynchronize(ctx->stream) == hipSuccess && hipMemGetInfo(&free, &total) == hipSuccess;
+  want = std::min(want, free / 2 / sizeof(double));
+  double* more = nullptr;
+  if (ok && want > tan_cap) ok = hipMalloc((void**)&more, want * sizeof(double)) == hipSuccess;
+  if (!ok) (void)hipGetLastError();  // no room: the present arena serves
+  if (ok && more) {
+    (void)hipFree(tan_arena);
+    tan_arena = more;
+    tan_cap = want;
+  }
+}
+
+// Whether the tangent programs run by levels: the arena holds one column of any of them
+// (otherwise they run instruction by instruction).
 bool kad_system_impl::levels_ready() {
   if (!gtan_ok || !fuse_ew) return false;
-  size_t all = 0, one = 0;
-  auto add = [&](const GroupProg& p, int cnt) {
-    all += (size_t)p.nphys * std::min(cnt, B) * stride;
-    one = std::max(one, (size_t)p.nphys * stride);
-  };
-  for (size_t p = 0; p < gtan.size(); ++p) add(gtan[p], tprogs[p].cnt);
-  for (auto& p : gpar) add(p, 1);
-  if (!tan_sized) {
-    tan_sized = true;
-    size_t want = std::min(all, (size_t)6 << 27), free = 0, total = 0;
-    double* more = nullptr;
-    if (want > tan_cap) {
-      // (work on the present arena ends on the context's stream)
-      bool ok = hipStreamSynchronize(ctx->stream) == hipSuccess && hipMemGetInfo(&free, &total) == hipSuccess;
-      want = std::min(want, free / 2 / sizeof(double));
-      if (ok && want > tan_cap) ok = hipMalloc((void**)&more, want * sizeof(double)) == hipSuccess;
-      if (!ok) (void)hipGetLastError();  // no room: the present arena serves
-      if (ok && more) {
-        (void)hipFree(tan_arena);
-        tan_arena = more;
-        tan_cap = want;
-      }
-    }
-  }
+  size_t one = 0;
+  for (auto* v : {&gtan, &gpar})
+    for (auto& p : *v) one = std::max(one, (size_t)p.nphys * stride);
+  if (one > tan_cap) grow_arena();
   return tan_cap >= one;
 }
 
 // The items in rounds that fit the arena.
 int kad_system_impl::group_columns(std::vector<GroupItem> items, void* out, int64_t ldo, int dtype, const double* w) {
+  size_t need = 0;
+  for (const GroupItem& it : items) need += (size_t)it.p->nphys * it.nb * stride;
+  if (need > tan_cap) grow_arena();
   std::vector<GroupItem> round;
   size_t used = 0;
   auto flush = [&]() -> int {

@@ -99,6 +99,11 @@ def test_batch_bounds_the_arena(ctx):
         s = _flat(programs.kerr(ctx, (9, 7, 4), BOUNDS[:3], n0=0.5, a=1.0, ome=0.05), 1, batch)
         w = torch.ones(s.m, dtype=torch.float64, device="cuda")
         s.residual()
+        if batch == 4096:  # a few columns fit the set-up's arena
+            s.set_option(fuse=False)
+            s.jvp_fill(3, 5)
+            s.set_option(fuse=True)
+            assert _taken(lambda: s.jvp_fill(3, 5)) == 0
         taken[batch] = _taken(lambda: s.vjp(w))
         s.close()
     print(f"arena {taken}", flush=True)
